@@ -120,8 +120,8 @@ int pade_op_apply_axpby(pade_op_t op, int oper, int axis, double alpha, const do
  * graph capture, tight serving or time-stepping loops, harnesses that forbid
  * hipMalloc).  Same arguments, result and error codes as
  * pade_op_apply_axpby.  The intermediates some applies need (the
- * one-lane-per-pencil path's accumulate temporary, used for n not a
- * multiple of 16 or above 1024; the bounded cd06 second derivative with an
+ * one-lane-per-pencil path's accumulate temporary, reserved for every n not
+ * a multiple of 16 or above 1024; the bounded cd06 second derivative with an
  * epilogue) come from one static device array of
  * PADE_NOALLOC_SCRATCH_BYTES per device instead of the stream-ordered
  * allocator; an apply that would need more returns 400 before launching
@@ -214,11 +214,13 @@ int pade_op_dense_info(pade_op_t op, int oper, int prec, int axis, int f_dtype, 
  * over na x nb pencils runs on an operator created with (kind, n, dx,
  * periodic, bc1, bcn) -- the codes that build it: init-time for cd06 and
  * cd06stagg, else the apply-time ones -- for dtype PADE_F64 / PADE_F32 and
- * adjoint 0 / 1.  info[8] = {M, PW, P, generic, mode, launches, 0, 0}: M
+ * adjoint 0 / 1.  info[8] = {M, PW, P, generic, mode, launches, uneven, 0}: M
  * the partition length, PW the partitions per wave, P the partitions per
  * pencil, generic = 1 for the one-lane-per-pencil path (M = n, P = 1), mode
  * 0 strided rows (y, z), 1 x pencils through LDS transposes, 2 the
- * staggered system form, and launches the kernel launches of one apply.  The
+ * staggered system form, launches the kernel launches of one apply, and
+ * uneven = 1 when M does not divide the rows and the partitions hold at most
+ * M of them.  The
  * strided-row kernels address the field with 32-bit per-lane byte offsets (a
  * lane's pencil relative to its workgroup's first pencil plus (PW - 1) * M
  * points along the pencil); variants whose offsets would reach 2^32, or
@@ -258,6 +260,18 @@ int pade_permute3(const void *src, void *dst, int elem_size, int n1, int n2, int
  * on CPU. */
 int pade_plan_export(int kind, int oper, int n, double dx, int periodic, int bc1, int bcn,
                      int adjoint, int M, double *tab, long long tab_len, int *meta);
+
+/* The same for a pencil length that M (16, 32 or 64) does not divide: the
+ * table of its uneven partitions (a staggered operator with an edge array:
+ * its system form).  meta[64]: as pade_plan_export in [0, 32), [32] = W, the
+ * partitions of a reduced-system row, [33 + p] = first row of partition p.
+ * Every partition occupies M slots: its rows, then padding slots with y_t =
+ * y_{t-2} and a zero right-hand side; the last partition has M rows.  The
+ * reduced-system rows hold, for every partition, 4 rows of 4 W values: entry
+ * j for partition p - kq + j (cyclic when periodic), or partition j when W =
+ * P.  Returns 21 when the length has no such split.  Used by tests. */
+int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, int bc1, int bcn,
+                            int adjoint, int M, double *tab, long long tab_len, int *meta);
 
 /* Pointwise stages of the compressible solver's Runge-Kutta substep
  * (src/compressible/cgrid.F90, one ideal-gas species), each one streaming

@@ -27,6 +27,7 @@ EXPORTS = [
     "pade_op_apply_host", "pade_gradient", "pade_divergence", "pade_curl", "pade_filter3d",
     "pade_op_filter3_complex", "pade_op_filter3_complex_host",
     "pade_op_dense_apply", "pade_op_dense_info", "pade_plan_variant", "pade_pencil_copy", "pade_permute3", "pade_plan_export",
+    "pade_plan_export_uneven",
     "pade_last_error", "pade_version",
     "pade_cg_conserved", "pade_cg_primitive", "pade_cg_strain", "pade_cg_lad_mu", "pade_cg_lad_bulk",
     "pade_cg_lad_kap", "pade_cg_fluxes", "pade_cg_rk_stage",
@@ -93,6 +94,7 @@ def load():
     lib.pade_permute3.argtypes = [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]
     lib.pade_plan_export.argtypes = [c_int, c_int, c_int, c_double, c_int, c_int, c_int, c_int, c_int, dp,
                                      c_ll, ip]
+    lib.pade_plan_export_uneven.argtypes = lib.pade_plan_export.argtypes
     v, d = c_void_p, c_double
     lib.pade_cg_conserved.argtypes = [c_ll, v, v, v, v, v, v, v, v]   # bad_index: device uint64
     lib.pade_cg_primitive.argtypes = [c_ll, v, d, d, v, v, v, v, v, v, v, v]
@@ -139,10 +141,10 @@ def plan_variant(kind, oper, n, dx, periodic, axis, na, nb, bc1=0, bcn=0, dtype=
     """Kernel an apply would run (host-only, pade_plan_variant): a dict with
     the partition length M, partitions per wave PW, partitions P, ``generic``
     (one lane per pencil), ``mode`` (0 strided rows, 1 x pencils, 2 staggered
-    system form) and ``launches`` per apply.  bc1 / bcn: the codes that build
+    system form), ``launches`` per apply and ``uneven`` (M does not divide the rows).  bc1 / bcn: the codes that build
     the operator (init-time for cd06 / cd06stagg, else apply-time)."""
     info = (ctypes.c_int * 8)()
     check(load().pade_plan_variant(int(kind), int(oper), int(n), float(dx), int(bool(periodic)), int(bc1), int(bcn),
                                    int(bool(adjoint)), int(axis), int(na), int(nb), int(dtype), info))
     return {"M": info[0], "PW": info[1], "P": info[2], "generic": bool(info[3]), "mode": info[4],
-            "launches": info[5]}
+            "launches": info[5], "uneven": bool(info[6])}

@@ -46,6 +46,8 @@ struct Variant {
     int coef_len = 0, ncls = 0, kq = 0;
     int cls[pade::kMaxPartitions] = {0};
     int len = 0;
+    bool uneven = false;   // partitions of `parts`
+    pade::UnevenParts parts;
 };
 
 struct PlanKey {
@@ -57,17 +59,24 @@ struct PlanKey {
 };
 
 struct Plan {
-    std::vector<Variant> spike;  // register-path variants (M in {16,32,64}), ascending M
+    std::vector<Variant> spike;  // register-path variants (M in {16,32,64}), ascending M; the
+                                 // uneven ones only where no M divides the rows
     Variant generic;             // whole pencil as one partition
     bool has_generic = false;
     pade::OpMatrices mats;       // for the dense form
 };
 
 // Assemble the table of one variant; returns 0 or an error code.
-int build_variant(const pade::OpMatrices &m, int M, std::vector<double> &tab, Variant &v)
+// parts: the uneven partitions to use, or null for an even split into M rows.
+int build_variant(const pade::OpMatrices &m, int M, std::vector<double> &tab, Variant &v,
+                  const pade::UnevenParts *parts = nullptr)
 {
     pade::SpikeFactors sf;
-    if (int rc = pade::spike_factor(m, M, sf)) return rc;
+    if (int rc = parts ? pade::spike_factor_uneven(m, *parts, sf) : pade::spike_factor(m, M, sf)) return rc;
+    if (parts) {
+        v.uneven = true;
+        v.parts = *parts;
+    }
     const int P = sf.P;
     const bool periodic = m.periodic;
     const int m4 = 4 * P;
@@ -97,10 +106,8 @@ int build_variant(const pade::OpMatrices &m, int M, std::vector<double> &tab, Va
         if (c < 0) { c = (int)reps.size(); reps.push_back(p); }
         if (p < pade::kMaxPartitions) v.cls[p] = c;
     }
-    if (periodic && reps.size() != 1) return 3;  // periodic blocks are identical by construction
+    if (periodic && !parts && reps.size() != 1) return 3;  // even periodic blocks are identical by construction
     v.ncls = (int)reps.size();
-    v.coef_len = v.ncls * 10 * M + (periodic ? 4 * m4 : P * 4 * m4);
-    v.len = (pade::kOffCoef + v.coef_len + 15) & ~15;
     // reduced-system window: farthest partition whose weight is not negligible
     double qmax = 0.0;
     for (double x : sf.Q) qmax = std::max(qmax, std::fabs(x));
@@ -114,6 +121,9 @@ int build_variant(const pade::OpMatrices &m, int M, std::vector<double> &tab, Va
                 if (periodic) d = std::min(d, P - d);
                 v.kq = std::max(v.kq, d);
             }
+    const int window = std::min(2 * v.kq + 1, P);
+    v.coef_len = v.ncls * 10 * M + (parts ? P * 16 * window : (periodic ? 4 * m4 : P * 4 * m4));
+    v.len = (pade::kOffCoef + v.coef_len + 15) & ~15;
     v.off = (long long)tab.size();
     tab.resize(tab.size() + v.len, 0.0);
     double *t = &tab[v.off];
@@ -135,6 +145,18 @@ int build_variant(const pade::OpMatrices &m, int M, std::vector<double> &tab, Va
         }
     }
     double *qa = ca + (size_t)v.ncls * 10 * M;
+    if (parts) {
+        for (int p = 0; p < P; p++)
+            for (int c = 0; c < 4; c++)
+                for (int j = 0; j < window; j++) {
+                    int q = window == P ? j : p - v.kq + j;
+                    if (periodic) q = (q + P) % P;
+                    if (q < 0 || q >= P) continue;
+                    for (int k = 0; k < 4; k++)
+                        qa[((size_t)p * 4 + c) * 4 * window + 4 * j + k] = sf.Q[((size_t)p * 4 + c) * m4 + 4 * q + k];
+                }
+        return 0;
+    }
     const int nq = periodic ? 1 : P;
     for (int p = 0; p < nq; p++)
         for (int c = 0; c < 4; c++)
@@ -195,6 +217,26 @@ int plan_key_bc(const pade_op_s *op, int bc)
 // caller's codes, then SolveZPenta_CMPLX with penta_nn).
 constexpr int kFilterRhsBc = 100 + pade::FILTER;
 
+// Partition sizes of the register path that serve this operator: those that
+// divide its rows, or else the uneven splits.
+void add_spike_variants(const pade::OpMatrices &m, std::vector<double> &tab, Plan &pl)
+{
+    for (int M : {16, 32, 64}) {
+        if (m.n % M || m.n / M > pade::kMaxPartitions) continue;
+        Variant v;
+        if (build_variant(m, M, tab, v) == 0) pl.spike.push_back(v);
+    }
+    if (!pl.spike.empty()) return;
+    for (int M : {16, 32, 64}) {
+        pade::UnevenParts parts;
+        Variant v;
+        // (those that pick_variant never prefers are not built: 64 rows up to
+        // n = 256, 32 on longer bounded pencils)
+        if (m.n <= 256 ? M == 64 : (M == 32 && !m.periodic)) continue;
+        if (pade::uneven_parts(m.n, M, parts) && build_variant(m, M, tab, v, &parts) == 0) pl.spike.push_back(v);
+    }
+}
+
 // One plan: the operator's matrices and the factor tables of every partition
 // size that divides its rows (appended to `tab`), plus the
 // one-lane-per-pencil form.  bc1 / bcn are the codes that build the
@@ -215,11 +257,7 @@ int build_plan(int kind, int oper, int n, double dx, bool periodic, int bc1, int
         if (int rc = pade::build_stagg_system(oper, n, dx, bc1, bcn, sys)) return fail(rc, "operator construction failed");
     }
     const pade::OpMatrices &pm = sys_form ? sys : pl.mats;
-    for (int M : {16, 32, 64}) {
-        if (pm.n % M || pm.n / M > pade::kMaxPartitions) continue;
-        Variant v;
-        if (build_variant(pm, M, tab, v) == 0) pl.spike.push_back(v);
-    }
+    add_spike_variants(pm, tab, pl);
     if (m >= 4 && build_variant(pl.mats, m, tab, pl.generic) == 0) pl.has_generic = true;
     return 0;
 }
@@ -265,11 +303,7 @@ int build_all_plans(pade_op_s *op)
             if (int rc = operator_matrices(op->kind, pade::FILTER, op->n, op->dx, false, b1, bn, false, pl.mats))
                 return fail(rc, "operator construction failed");
             pl.mats.band = nn.band;      // (bc1, bcn) right-hand side, (0, 0) left-hand side
-            for (int M : {16, 32, 64}) {
-                if (op->n % M || op->n / M > pade::kMaxPartitions) continue;
-                Variant v;
-                if (build_variant(pl.mats, M, tab, v) == 0) pl.spike.push_back(v);
-            }
+            add_spike_variants(pl.mats, tab, pl);
             if (op->n >= 4 && build_variant(pl.mats, op->n, tab, pl.generic) == 0) pl.has_generic = true;
             op->plans[{kFilterRhsBc, b1, bn, 0}] = std::move(pl);
         }
@@ -339,6 +373,11 @@ bool offsets_fit(const pade::ApplyArgs<T> &a, int mode, int M, int PW)
     return lmax + part < (1LL << 32);
 }
 
+// Fewest pencils that uneven partitions serve.  Below it (one workgroup's
+// worth or two of the whole chip) the one-lane-per-pencil kernel runs, as
+// pade_plan_variant reports for 100 x pencils of 100 points.
+constexpr long long kUnevenPencils = 128;
+
 template <typename T>
 const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mode, int *pw_out)
 {
@@ -374,6 +413,8 @@ const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mod
     const bool prefer_whole = mode == 1 && pl.mats.periodic;
     // eligible (variant, partitions per wave) pairs and their wave counts
     auto waves_of = [&](const Variant &v, int pw) -> long long {
+        // uneven kernels take two partitions per wave
+        if (v.uneven && (pw != 2 || npencils < kUnevenPencils)) return -1;
         if ((v.P + pw - 1) / pw > 8) return -1;
         if (pw == 8 && (mode != 1 || v.P > 8 || (v.M != 32 && v.M != 64))) return -1;
         // four partitions per wave: strided rows only, by request (tuning)
@@ -510,6 +551,9 @@ int plan_launch(const Plan &pl, bool periodic, int axis, const T *f, T *df, int 
     a.ncls = v->ncls;
     a.kq = v->kq;
     for (int k = 0; k < pade::kMaxPartitions; k++) a.cls[k] = v->cls[k];
+    a.ubase = v->parts.base;
+    a.uextra = v->parts.extra;
+    a.uunit = v->parts.unit;
     a.axpby = 0;
     a.alpha = T(1);
     a.beta = T(0);
@@ -544,7 +588,18 @@ int apply_one(pade_op_t op, const Plan &pl, int axis, const T *f, T *df, int na,
             a.alpha = epi.alpha;
             a.beta = epi.beta;
         }
-        e = pade::launch_spike<T>(a, v->M, pw, pw == 8 ? whole_pencil_waves() : 1, kadj, mode, s);
+        if (v->uneven) {
+            // The allocation-free entry point refuses accumulating applies
+            // whose one-lane form would not fit its array; lengths that take
+            // uneven partitions keep that documented limit.
+            if (ws.on && epi.on) {
+                T *unused = nullptr;
+                if (int rc = scratch_get<T>(ws, (size_t)a.npencils * n, s, &unused, "accumulate temporary")) return rc;
+            }
+            e = pade::launch_uneven<T>(a, v->M, kadj, mode, s);
+        } else {
+            e = pade::launch_spike<T>(a, v->M, pw, pw == 8 ? whole_pencil_waves() : 1, kadj, mode, s);
+        }
         if (e != hipSuccess) return hip_fail(e, "spike_apply launch");
         return 0;
     }
@@ -957,15 +1012,15 @@ int pade_plan_variant(int kind, int oper, int n, double dx, int periodic, int bc
     if (int rc = build_plan(kind, oper, n, filter_kind ? 1.0 : dx, periodic != 0, bc1, bcn, adjoint != 0, tab, pl))
         return rc;
     int rc;
-    int M = 0, pw = 1, P = 0, generic = 0, mode = 0;
+    int M = 0, pw = 1, P = 0, generic = 0, mode = 0, uneven = 0;
     if (dtype == PADE_F64) {
         LaunchPlan<double> L;
         rc = plan_launch<double>(pl, periodic != 0, axis, nullptr, nullptr, na, nb, L);
-        if (!rc) { M = L.v->M; pw = L.pw; P = L.v->P; generic = L.generic; mode = L.mode; }
+        if (!rc) { M = L.v->M; pw = L.pw; P = L.v->P; generic = L.generic; mode = L.mode; uneven = L.v->uneven; }
     } else {
         LaunchPlan<float> L;
         rc = plan_launch<float>(pl, periodic != 0, axis, nullptr, nullptr, na, nb, L);
-        if (!rc) { M = L.v->M; pw = L.pw; P = L.v->P; generic = L.generic; mode = L.mode; }
+        if (!rc) { M = L.v->M; pw = L.pw; P = L.v->P; generic = L.generic; mode = L.mode; uneven = L.v->uneven; }
     }
     if (rc) return rc;
     info[0] = M;
@@ -973,6 +1028,7 @@ int pade_plan_variant(int kind, int oper, int n, double dx, int periodic, int bc
     info[2] = P;
     info[3] = generic;
     info[4] = mode;
+    info[6] = uneven;
     return 0;
 }
 
@@ -1049,6 +1105,39 @@ int pade_plan_export(int kind, int oper, int n, double dx, int periodic, int bc1
     int vals[32] = {rows, v.M, v.P, periodic ? 1 : 0, v.nbl, v.nbr, pade::kOffBl, pade::kOffBr,
                     pade::kOffCoef, v.coef_len, v.ncls, v.kq, v.len, cols, m.rect ? 1 : 0, m.tail ? 1 : 0};
     for (int k = 0; k < pade::kMaxPartitions; k++) vals[16 + k] = v.cls[k];
+    std::memcpy(meta, vals, sizeof(vals));
+    if (tab) {
+        if (tab_len < v.len) return fail(400, "table buffer too small");
+        std::copy(t.begin(), t.end(), tab);
+    }
+    return 0;
+}
+
+int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, int bc1, int bcn, int adjoint, int M,
+                            double *tab, long long tab_len, int *meta)
+{
+    if (!meta) return fail(400, "null meta");
+    if (kind < pade::CD06 || kind > pade::GAUSSIAN) return fail(400, "unknown operator kind");
+    if (!oper_valid(kind, oper)) return fail(21, "operation not provided for this operator kind");
+    if (int ierr = pade::init_error(kind, n, periodic != 0)) return fail(ierr, "grid too small");
+    pade::OpMatrices m;
+    const bool filter_kind = kind == pade::CF90 || kind == pade::GAUSSIAN;
+    if (int rc = operator_matrices(kind, oper, n, filter_kind ? 1.0 : dx, periodic != 0, bc1, bcn, adjoint != 0, m))
+        return fail(rc, "operator construction failed");
+    if (kind == pade::CD06STAGG && !periodic && (pade::stagg_edge_in(oper) || pade::stagg_edge_out(oper)))
+        if (int rc = pade::build_stagg_system(oper, n, dx, bc1, bcn, m)) return fail(rc, "operator construction failed");
+    pade::UnevenParts parts;
+    if ((M != 16 && M != 32 && M != 64) || !pade::uneven_parts(m.n, M, parts))
+        return fail(21, "no uneven split of this length");
+    std::vector<double> t;
+    Variant v;
+    if (int rc = build_variant(m, M, t, v, &parts)) return fail(rc == 1 ? 400 : rc, "factorisation failed");
+    const int cols = m.n_in ? m.n_in : m.n;
+    int vals[64] = {m.n, v.M, v.P, periodic ? 1 : 0, v.nbl, v.nbr, pade::kOffBl, pade::kOffBr,
+                    pade::kOffCoef, v.coef_len, v.ncls, v.kq, v.len, cols, m.rect ? 1 : 0, m.tail ? 1 : 0};
+    for (int k = 0; k < pade::kMaxPartitions; k++) vals[16 + k] = v.cls[k];
+    vals[32] = std::min(2 * v.kq + 1, v.P);
+    for (int p = 0; p < v.P; p++) vals[33 + p] = parts.start(p);
     std::memcpy(meta, vals, sizeof(vals));
     if (tab) {
         if (tab_len < v.len) return fail(400, "table buffer too small");

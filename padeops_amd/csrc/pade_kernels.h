@@ -20,7 +20,10 @@ constexpr int kBColsDev = 16;
 //       then the reduced-system rows: periodic -> the 4 rows (4P each) of
 //       partition 0 (partition p uses them rotated by p); bounded -> the 4
 //       rows of every partition ([P][4][4P]).
-// Partition p uses block cls[p].
+// Partition p uses block cls[p].  Uneven partitions store of every
+// partition's reduced-system rows the entries of its window only
+// ([P][4][4W], W = min(2 kq + 1, P); entry j belongs to partition p - kq + j,
+// cyclic when periodic, or to partition j when W = P).
 constexpr int kOffBl = 16;
 constexpr int kOffBr = 144;
 constexpr int kOffCoef = 272;
@@ -44,6 +47,9 @@ struct ApplyArgs {
     int ncls;              // number of coefficient blocks
     int kq;                // reduced-system window: partitions p-kq..p+kq (2kq+1 >= P: all)
     int cls[kMaxPartitions];
+    // uneven partitions: partition p < P - 1 has ubase + (p < uextra ? uunit : 0)
+    // rows and starts at row p * ubase + min(p, uextra) * uunit, the last has M
+    int ubase, uextra, uunit;
     int axpby;             // 0: out = op(f); 1: out = alpha * op(f) + beta * out
     int remap;             // workgroup order: 0 launch order; C > 0 each of the 8 XCDs
                            // (workgroup i runs on XCD i % 8) takes runs of C
@@ -51,13 +57,16 @@ struct ApplyArgs {
     T alpha, beta;
 };
 
-size_t spike_lds_bytes(size_t tsize, int M, int P, int PW, bool adj, int mode, int coef_len, bool bnd, int gw);
-
 // mode 0: strided rows (y, z); 1: x pencils through LDS transposes; 2:
 // strided rows of a bounded staggered operator in system form (forward only).
 // GW: whole-pencil x waves (PW = 8) per workgroup (other variants: 1).
 template <typename T>
 hipError_t launch_spike(const ApplyArgs<T> &a, int M, int PW, int GW, bool adj, int mode, hipStream_t s);
+
+// The same solve over uneven partitions (a pencil length that is no multiple
+// of M), two partitions per wave; modes as above.
+template <typename T>
+hipError_t launch_uneven(const ApplyArgs<T> &a, int M, bool adj, int mode, hipStream_t s);
 
 template <typename T>
 hipError_t launch_generic(const ApplyArgs<T> &a, bool adj, T *work, hipStream_t s);

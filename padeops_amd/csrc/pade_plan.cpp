@@ -622,20 +622,19 @@ void transpose_operator(const OpMatrices &f, OpMatrices &t)
 
 namespace {
 
-// Band LU (no pivoting) of rows [r0, r0+M) restricted to that block.
+// Band LU (no pivoting) of rows [r0, r0+rows) restricted to that block, in
+// M >= rows slots (the slots beyond the rows hold y_t = y_{t-2}).
 // lu[t*5 + {0..4}] = l1, l2, 1/pivot, u1/pivot, u2/pivot.
-int band_lu_block(const OpMatrices &op, int r0, int M, double *lu)
+int band_lu_block(const OpMatrices &op, int r0, int rows, int M, double *lu)
 {
-    const int n = op.n;
     std::vector<double> U((size_t)M * 3, 0.0);  // U rows: offsets 0..2
     for (int t = 0; t < M; t++) {
         const int i = r0 + t;
-        double row[5];
-        for (int o = -2; o <= 2; o++) {
+        double row[5] = {-1.0, 0.0, 1.0, 0.0, 0.0};
+        for (int o = -2; o <= 2 && t < rows; o++) {
             const int tt = t + o;
-            row[o + 2] = (tt >= 0 && tt < M) ? op.band[(size_t)i * 5 + o + 2] : 0.0;
+            row[o + 2] = (tt >= 0 && tt < rows) ? op.band[(size_t)i * 5 + o + 2] : 0.0;
         }
-        (void)n;
         double l1 = 0.0, l2 = 0.0;
         if (t >= 2) {
             const double *u = &U[(size_t)(t - 2) * 3];
@@ -682,10 +681,13 @@ void band_lu_solve(const double *lu, int M, double *x)
     }
 }
 
-// In-place Gauss-Jordan inverse with partial pivoting (small dense matrices).
+// In-place Gauss-Jordan inverse with partial pivoting (small matrices, most
+// entries zero: the reduced systems couple neighbouring partitions only, so a
+// pivot row updates the columns where it has entries).
 int invert(std::vector<double> &a, int m)
 {
     std::vector<double> inv((size_t)m * m, 0.0);
+    std::vector<int> ca, ci;
     for (int i = 0; i < m; i++) inv[(size_t)i * m + i] = 1.0;
     for (int c = 0; c < m; c++) {
         int piv = c;
@@ -698,18 +700,20 @@ int invert(std::vector<double> &a, int m)
                 std::swap(inv[(size_t)piv * m + k], inv[(size_t)c * m + k]);
             }
         const double d = 1.0 / a[(size_t)c * m + c];
+        ca.clear();
+        ci.clear();
         for (int k = 0; k < m; k++) {
             a[(size_t)c * m + k] *= d;
             inv[(size_t)c * m + k] *= d;
+            if (a[(size_t)c * m + k] != 0.0) ca.push_back(k);
+            if (inv[(size_t)c * m + k] != 0.0) ci.push_back(k);
         }
         for (int r = 0; r < m; r++) {
             if (r == c) continue;
             const double f = a[(size_t)r * m + c];
             if (f == 0.0) continue;
-            for (int k = 0; k < m; k++) {
-                a[(size_t)r * m + k] -= f * a[(size_t)c * m + k];
-                inv[(size_t)r * m + k] -= f * inv[(size_t)c * m + k];
-            }
+            for (int k : ca) a[(size_t)r * m + k] -= f * a[(size_t)c * m + k];
+            for (int k : ci) inv[(size_t)r * m + k] -= f * inv[(size_t)c * m + k];
         }
     }
     a.swap(inv);
@@ -718,15 +722,14 @@ int invert(std::vector<double> &a, int m)
 
 }  // namespace
 
-int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
+namespace {
+
+// The factors of P partitions of M slots: partition p holds rows start(p) ..
+// start(p) + rows(p) - 1 in its first slots.
+template <typename Start, typename Rows>
+int factor_parts(const OpMatrices &op, int M, int P, Start start, Rows rows, SpikeFactors &out)
 {
     const int n = op.n;
-    // partitions of at least 8 rows; a bounded pencil solved whole (one
-    // partition, no reduced system) may be as short as 4 (the staggered
-    // operators on n = 5..7 cells)
-    const bool whole_bounded = !op.periodic && M == n && n >= 4;
-    if ((M < 8 && !whole_bounded) || n % M != 0) return 1;
-    const int P = n / M;
     out = SpikeFactors();
     out.n = n;
     out.M = M;
@@ -738,21 +741,22 @@ int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
     std::vector<double> col(M);
     for (int p = 0; p < P; p++) {
         double *lu = &out.lu[(size_t)p * M * 5];
-        if (int rc = band_lu_block(op, p * M, M, lu)) return rc;
+        const int mp = rows(p);
+        if (int rc = band_lu_block(op, start(p), mp, M, lu)) return rc;
         // coupling columns: rows of this block that reference columns outside it
         for (int c = 0; c < 4; c++) {
             std::fill(col.begin(), col.end(), 0.0);
             bool any = false;
-            for (int t = 0; t < M; t++) {
-                const int i = p * M + t;
+            for (int t = 0; t < mp; t++) {
+                const int i = start(p) + t;
                 for (int o = -2; o <= 2; o++) {
                     const int tt = t + o;
-                    if (tt >= 0 && tt < M) continue;
+                    if (tt >= 0 && tt < mp) continue;
                     const double v = op.band[(size_t)i * 5 + o + 2];
                     if (v == 0.0) continue;
                     // tt = -2,-1 -> tail of left neighbour (c = 0,1);
-                    // tt = M, M+1 -> head of right neighbour (c = 2,3)
-                    const int cc = tt < 0 ? tt + 2 : 2 + (tt - M);
+                    // tt = rows, rows+1 -> head of right neighbour (c = 2,3)
+                    const int cc = tt < 0 ? tt + 2 : 2 + (tt - mp);
                     if (cc == c) { col[t] += v; any = true; }
                 }
             }
@@ -761,15 +765,16 @@ int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
         }
     }
     if (!op.periodic && P == 1) return 0;
-    // reduced system over the tips: unknown 4q + k, k = 0,1 head rows (0,1),
-    // k = 2,3 tail rows (M-2, M-1)
+    // reduced system over the tips: unknown 4q + k, k = 0,1 head slots (0,1),
+    // k = 2,3 tail slots (M-2, M-1), which hold the last two rows, exchanged
+    // when the partition has an odd number of padding slots
     const int m = 4 * P;
     std::vector<double> R((size_t)m * m, 0.0);
     auto nbr_index = [&](int p, int c) -> int {
         if (c < 2) {
             int q = p - 1;
             if (q < 0) { if (!op.periodic) return -1; q += P; }
-            return 4 * q + 2 + c;
+            return 4 * q + 2 + ((M - rows(q)) % 2 ? 1 - c : c);
         }
         int q = p + 1;
         if (q >= P) { if (!op.periodic) return -1; q -= P; }
@@ -794,6 +799,43 @@ int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
                 out.Q[((size_t)p * 4 + c) * m + k] = j < 0 ? 0.0 : R[(size_t)j * m + k];
         }
     return 0;
+}
+
+}  // namespace
+
+int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
+{
+    // partitions of at least 8 rows; a bounded pencil solved whole (one
+    // partition, no reduced system) may be as short as 4 (the staggered
+    // operators on n = 5..7 cells)
+    const bool whole_bounded = !op.periodic && M == op.n && op.n >= 4;
+    if ((M < 8 && !whole_bounded) || op.n % M != 0) return 1;
+    return factor_parts(op, M, op.n / M, [&](int p) { return p * M; }, [&](int) { return M; }, out);
+}
+
+bool uneven_parts(int n, int M, UnevenParts &out)
+{
+    if (n <= M || n % M == 0) return false;
+    // Short partitions lose accuracy where A is nearly singular (cf90: the
+    // bounded adjoint's error against 128-bit arithmetic grows from 2e-13
+    // with 20 or more rows to 1e-12 with 8 to 12), so 16-row partitions
+    // serve only lengths that two of them hold.
+    if (M == 16 && n > 32) return false;
+    out = UnevenParts();
+    out.n = n;
+    out.M = M;
+    out.P = (n + M - 1) / M;
+    out.unit = n % 16 == 0 && M == 64 ? 16 : (n % 4 == 0 ? 4 : (n % 2 == 0 ? 2 : 1));
+    const int units = (n - M) / out.unit;             // the unit divides n and M
+    out.base = units / (out.P - 1) * out.unit;
+    out.extra = units % (out.P - 1);
+    return out.P <= 16 && out.base >= 8;
+}
+
+int spike_factor_uneven(const OpMatrices &op, const UnevenParts &u, SpikeFactors &out)
+{
+    if (op.n != u.n || u.P < 2) return 1;
+    return factor_parts(op, u.M, u.P, [&](int p) { return u.start(p); }, [&](int p) { return u.rows(p); }, out);
 }
 
 int dense_operator(const OpMatrices &op, std::vector<double> &D)

@@ -64,6 +64,26 @@ struct OpMatrices {
     double tail_dn = 0.0, tail_idg = 0.0;
 };
 
+// Split of n rows into P partitions of M register slots each when M does not
+// divide n.  Partition p < P - 1 holds `base` (+ `unit` for p < extra) rows
+// and its remaining slots are padding; the last holds M rows, so that the
+// special rows of a bounded pencil keep their slots at both ends.  `unit` is
+// the largest of 4, 2, 1 that divides n (16-byte starts for x pencils), or 16
+// for M = 64 and n a multiple of 16 (whole-line starts of FP64 x pencils).  A
+// padding slot t carries the equation y_t = y_{t-2}, which stays inside the
+// band: the last two slots of every partition then repeat its last two rows
+// (exchanged when the number of padding slots is odd), and the kernels' tip
+// slots are those of an even split.
+struct UnevenParts {
+    int n = 0, M = 0, P = 0, base = 0, extra = 0, unit = 1;
+    int rows(int p) const { return p == P - 1 ? M : base + (p < extra ? unit : 0); }
+    int start(int p) const { return p * base + (p < extra ? p : extra) * unit; }
+};
+// The split of n rows for M slots: false when there is none (M divides n,
+// more than 16 partitions, partitions of fewer than 8 rows, or more than two
+// of 16 slots).
+bool uneven_parts(int n, int M, UnevenParts &out);
+
 // Partitioned solve factors (all FP64 on the host).
 struct SpikeFactors {
     int n = 0, M = 0, P = 0;
@@ -92,6 +112,8 @@ void transpose_operator(const OpMatrices &fwd, OpMatrices &adj);
 
 // Factor A for a partitioned solve with partition size M (n % M == 0).
 int spike_factor(const OpMatrices &op, int M, SpikeFactors &out);
+// The same over uneven partitions; lu, S and Q are per slot (P * M of them).
+int spike_factor_uneven(const OpMatrices &op, const UnevenParts &parts, SpikeFactors &out);
 
 // Error code init() returns for this size (0 ok, 2/3/7 as the reference).
 int init_error(int kind, int n, bool periodic);

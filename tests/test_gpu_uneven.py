@@ -1,0 +1,107 @@
+"""Uneven partitions on the GPU (pencil lengths that no partition size
+divides): forward, accumulating and adjoint applies along every axis against
+the dense oracle, at the edges of the splits (shortest partitions, odd and
+even padding, one and two partitions in the last wave) with pencil counts
+that leave the last workgroup partly empty.  FP64 to 1e-12, FP32 to the
+suite's banded tolerance."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import pade_dense as pd
+import padeops_amd as po
+from padeops_amd import _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+KIND = {"cd06": po.cd06, "cd10": po.cd10, "cf90": po.cf90, "gaussian": po.gaussian}
+OPER = {"d1": _lib.PADE_D1, "d2": _lib.PADE_D2, "filter": _lib.PADE_FILTER}
+
+
+def setup(kind, n, periodic, axis, seed, dtype=torch.float64, pencils=(67, 5)):
+    op = KIND[kind]()
+    assert (op.init(n, periodic) if kind in ("cf90", "gaussian") else op.init(n, 0.05, periodic, 0, 0)) == 0
+    shape = list(pencils)
+    shape.insert(axis - 1, n)
+    f = np.random.default_rng(seed).standard_normal(shape)
+    ft = po.as_fortran(torch.tensor(f, device=DEV, dtype=dtype))
+    return op, ft, ft.cpu().double().numpy()
+
+
+def rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+CASES = [("cd10", "d1", True, (0, 0)), ("cd10", "d2", True, (0, 0)), ("cf90", "filter", True, (0, 0)),
+         ("cd06", "d1", True, (0, 0)), ("cd10", "d1", False, (0, 0)), ("cd10", "d2", False, (1, -1)),
+         ("cf90", "filter", False, (-1, 1)), ("cd06", "d1", False, (0, 0)), ("gaussian", "filter", False, (0, 1))]
+
+
+@pytest.mark.parametrize("kind,which,periodic,bc", CASES)
+@pytest.mark.parametrize("n", [24, 25, 37, 75, 129, 200, 257, 301])
+@pytest.mark.parametrize("axis", [1, 2, 3])
+def test_uneven_matches_oracle(kind, which, periodic, bc, n, axis):
+    op, f, fh = setup(kind, n, periodic, axis, n + axis)
+    v = _lib.plan_variant(op._kind, OPER[which], n, 0.05, periodic, axis, 67, 5, *bc)
+    assert v["uneven"] == (n != 37), v           # 33 .. 39 points have no split
+    h = 1.0 if which == "filter" else 0.05
+    D = pd.dense_operator(kind, which, n, h, periodic, *bc)
+    ref = pd.apply_axis(D, fh, axis - 1)
+    out = po.fortran_empty(f.shape, device=DEV)
+    print(f"uneven {kind} {which} periodic {periodic} bc {bc} n {n} axis {axis}", flush=True)
+    op._apply(OPER[which], axis, f, out, 67, 5, *bc)
+    assert rel(out.cpu().numpy(), ref) < 1e-12
+    acc = f.clone()
+    op._apply(OPER[which], axis, f, acc, 67, 5, *bc, alpha=-0.75, beta=1.5)
+    assert rel(acc.cpu().numpy(), -0.75 * ref + 1.5 * fh) < 1e-12
+    op._apply(OPER[which], axis, f, out, 67, 5, *bc, adjoint=True)
+    assert rel(out.cpu().numpy(), pd.apply_axis(D.T, fh, axis - 1)) < 1e-12
+
+
+@pytest.mark.parametrize("n,pencils", [(129, (150, 130)), (300, (150, 130)), (513, (64, 33)), (1023, (40, 33))])
+@pytest.mark.parametrize("axis", [1, 2, 3])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_uneven_throughput_sizes(n, pencils, axis, periodic):
+    """Enough pencils for the throughput partition sizes; FP64 and FP32."""
+    D = pd.dense_operator("cd10", "d1", n, 0.05, periodic, 0, 0)
+    for dtype, tol in ((torch.float64, 1e-12), (torch.float32, 1e-4)):
+        op, f, fh = setup("cd10", n, periodic, axis, n, dtype, pencils)
+        out = po.fortran_empty(f.shape, dtype=dtype, device=DEV)
+        print(f"uneven throughput n {n} axis {axis} periodic {periodic} {dtype}", flush=True)
+        op._apply(_lib.PADE_D1, axis, f, out, *pencils)
+        assert rel(out.cpu().double().numpy(), pd.apply_axis(D, fh, axis - 1)) < tol
+
+
+@pytest.mark.parametrize("oper", ["ddz_E2C", "ddz_C2E", "InterpZ_C2E", "d2dz2_E2E", "ddz_C2C"])
+@pytest.mark.parametrize("n", [25, 70, 129])
+def test_uneven_staggered_bounded(oper, n):
+    name = {"ddz_E2C": "d1_e2c", "ddz_C2E": "d1_c2e", "InterpZ_C2E": "interp_c2e", "d2dz2_E2E": "d2_e2e",
+            "ddz_C2C": "d1_c2c"}[oper]
+    e_in = 1 if oper in ("ddz_E2C", "d2dz2_E2E") else 0
+    e_out = 1 if oper in ("ddz_C2E", "InterpZ_C2E", "d2dz2_E2E") else 0
+    f = np.random.default_rng(n).standard_normal((19, 11, n + e_in))
+    ft = po.as_fortran(torch.tensor(f, device=DEV))
+    for top, bot, tops, bots in ((True, False, False, False), (False, True, True, False), (True, True, True, True)):
+        op = po.cd06stagg()
+        op.init(n, 0.1, top, bot, tops, bots)
+        out = po.fortran_empty((19, 11, n + e_out), device=DEV)
+        print(f"uneven staggered {oper} n {n}", flush=True)
+        getattr(op, oper)(ft, out, 19, 11)
+        D = pd.stagg_bounded_operator(name, n, 0.1, (bot, bots), (top, tops))
+        assert rel(out.cpu().numpy(), pd.apply_axis(D, f, 2)) < 1e-12
+
+
+def test_uneven_in_place_filter3d():
+    """filter3D's last z pass runs in place on uneven partitions too."""
+    from padeops_amd import composite
+    s = (33, 50, 97)
+    fil = po.filters()
+    fil.init(*s, True, True, False, "cf90", "cf90", "cf90")
+    f = np.random.default_rng(1).standard_normal(s)
+    ft = po.as_fortran(torch.tensor(f, device=DEV))
+    print("uneven filter3D", flush=True)
+    composite.filter3D(None, fil, ft)
+    ref = f
+    for a in (1, 0, 2):
+        ref = pd.apply("cf90", "filter", ref, a, 1.0, a < 2, 0, 0)
+    assert rel(ft.cpu().numpy(), ref) < 1e-12
