@@ -261,7 +261,7 @@ int pade_permute3(const void *src, void *dst, int elem_size, int n1, int n2, int
 int pade_plan_export(int kind, int oper, int n, double dx, int periodic, int bc1, int bcn,
                      int adjoint, int M, double *tab, long long tab_len, int *meta);
 
-/* The same for a pencil length that M (16, 32 or 64) does not divide: the
+/* The same for a pencil length that M (16, 24, 32 or 64) does not divide: the
  * table of its uneven partitions (a staggered operator with an edge array:
  * its system form).  meta[64]: as pade_plan_export in [0, 32), [32] = W, the
  * partitions of a reduced-system row, [33 + p] = first row of partition p.

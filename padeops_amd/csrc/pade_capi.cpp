@@ -227,11 +227,12 @@ void add_spike_variants(const pade::OpMatrices &m, std::vector<double> &tab, Pla
         if (build_variant(m, M, tab, v) == 0) pl.spike.push_back(v);
     }
     if (!pl.spike.empty()) return;
-    for (int M : {16, 32, 64}) {
+    for (int M : {16, 24, 32, 64}) {
         pade::UnevenParts parts;
         Variant v;
-        // (those that pick_variant never prefers are not built: 64 rows up to
-        // n = 256, 32 on longer bounded pencils)
+        // (those that pick_variant never prefers are not built: 24 rows where
+        // 32 have a split, 64 up to n = 256, 32 on longer bounded pencils)
+        if (M == 24 && m.n >= 40) continue;
         if (m.n <= 256 ? M == 64 : (M == 32 && !m.periodic)) continue;
         if (pade::uneven_parts(m.n, M, parts) && build_variant(m, M, tab, v, &parts) == 0) pl.spike.push_back(v);
     }
@@ -1127,7 +1128,7 @@ int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, 
     if (kind == pade::CD06STAGG && !periodic && (pade::stagg_edge_in(oper) || pade::stagg_edge_out(oper)))
         if (int rc = pade::build_stagg_system(oper, n, dx, bc1, bcn, m)) return fail(rc, "operator construction failed");
     pade::UnevenParts parts;
-    if ((M != 16 && M != 32 && M != 64) || !pade::uneven_parts(m.n, M, parts))
+    if ((M != 16 && M != 24 && M != 32 && M != 64) || !pade::uneven_parts(m.n, M, parts))
         return fail(21, "no uneven split of this length");
     std::vector<double> t;
     Variant v;

@@ -818,9 +818,9 @@ bool uneven_parts(int n, int M, UnevenParts &out)
     if (n <= M || n % M == 0) return false;
     // Short partitions lose accuracy where A is nearly singular (cf90: the
     // bounded adjoint's error against 128-bit arithmetic grows from 2e-13
-    // with 20 or more rows to 1e-12 with 8 to 12), so 16-row partitions
-    // serve only lengths that two of them hold.
-    if (M == 16 && n > 32) return false;
+    // with 20 or more rows to 1e-12 with 8 to 12), so partitions of 16 and 24
+    // rows serve only lengths that two of them hold.
+    if (M < 32 && n > 2 * M) return false;
     out = UnevenParts();
     out.n = n;
     out.M = M;

@@ -81,7 +81,7 @@ struct UnevenParts {
 };
 // The split of n rows for M slots: false when there is none (M divides n,
 // more than 16 partitions, partitions of fewer than 8 rows, or more than two
-// of 16 slots).
+// of 16 or 24 slots).
 bool uneven_parts(int n, int M, UnevenParts &out);
 
 // Partitioned solve factors (all FP64 on the host).

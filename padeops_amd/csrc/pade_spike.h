@@ -45,8 +45,7 @@
 //
 // Generic path (generic_apply, pade_kernels.hip): one lane per pencil with
 // the whole pencil as one partition in global memory -- for sizes the
-// register path does not cover (n < 24 and 33 .. 39 unless a multiple of 16,
-// n > 1024, or fewer than 128 pencils of an uneven length).
+// register path does not cover (n < 24 unless 16, n > 1024, or fewer than 128 pencils of an uneven length).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -148,7 +147,8 @@ __device__ __forceinline__ void pin(T &x) { asm volatile("" : "+v"(x)); }
 // chunk holds the 4 + 4 window points either side of the partition.
 __host__ __device__ constexpr int xtile_points(int tsize, int M)
 {
-    return (tsize == 8 ? 16 : 32) < M ? (tsize == 8 ? 16 : 32) : M;
+    const int xt = tsize == 8 ? 16 : 32;
+    return M % xt == 0 ? xt : (M == 24 ? 8 : M);
 }
 constexpr int kHaloChunk = 8;
 // How the row segments of a strided-row workgroup (its pencils' values at one

@@ -29,6 +29,7 @@ hipError_t launch_uneven(const ApplyArgs<T> &a, int M, bool adj, int mode, hipSt
         return hipErrorInvalidValue;
     switch (M) {
     case 16: return launch_uneven_m<T, 16>(a, adj, mode, s);
+    case 24: return launch_uneven_m<T, 24>(a, adj, mode, s);
     case 32: return launch_uneven_m<T, 32>(a, adj, mode, s);
     case 64: return launch_uneven_m<T, 64>(a, adj, mode, s);
     default: return hipErrorInvalidValue;

@@ -70,7 +70,7 @@ def solve(tab, m, r):
     return out
 
 
-LENGTHS = [(24, 16), (25, 16), (30, 16), (31, 16), (40, 32), (41, 32), (63, 32), (97, 32),
+LENGTHS = [(24, 16), (25, 16), (30, 16), (31, 16), (33, 24), (36, 24), (39, 24), (40, 32), (41, 32), (63, 32), (97, 32),
            (129, 32), (200, 32), (511, 32), (72, 64), (73, 64), (257, 64), (300, 64), (1023, 64), (544, 64)]
 
 
@@ -125,11 +125,11 @@ def test_splits_keep_their_bounds():
     """Every length: rows per partition, the last partition full, starts a
     multiple of the widest vector that divides the length."""
     for n in range(17, 1100):
-        for M in (16, 32, 64):
+        for M in (16, 24, 32, 64):
             tab, m = export(PADE_CD10, PADE_D1, n, 0.1, True, 0, 0, False, M)
             if tab is None:
                 P = -(-n // M)
-                assert n <= M or n % M == 0 or P > 16 or (n - M) // (P - 1) < 8 + 3 or (M == 16 and n > 32), (n, M)
+                assert n <= M or n % M == 0 or P > 16 or (n - M) // (P - 1) < 8 + 3 or (M < 32 and n > 2 * M), (n, M)
                 continue
             unit = 16 if M == 64 and n % 16 == 0 else 4 if n % 4 == 0 else 2 if n % 2 == 0 else 1
             assert all(s % unit == 0 for s in m["start"]) and m["rows"][-1] == M
