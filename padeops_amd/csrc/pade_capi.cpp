@@ -219,10 +219,12 @@ constexpr int kFilterRhsBc = 100 + pade::FILTER;
 
 // Partition sizes of the register path that serve this operator: those that
 // divide its rows, or else the uneven splits.
-void add_spike_variants(const pade::OpMatrices &m, std::vector<double> &tab, Plan &pl)
+void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double> &tab, Plan &pl)
 {
+    // special rows the kernels hold
+    const int rows = adj ? pade::kBRowsDev : (m.rect ? pade::kBRowsSys : pade::kBRowsFwd);
     for (int M : {16, 32, 64}) {
-        if (m.n % M || m.n / M > pade::kMaxPartitions) continue;
+        if (m.n % M || m.n / M > pade::kMaxPartitions || m.nbl > rows || m.nbr > rows) continue;
         Variant v;
         if (build_variant(m, M, tab, v) == 0) pl.spike.push_back(v);
     }
@@ -232,7 +234,7 @@ void add_spike_variants(const pade::OpMatrices &m, std::vector<double> &tab, Pla
         Variant v;
         // (those that pick_variant never prefers are not built: 24 rows where
         // 32 have a split, 64 up to n = 256, 32 on longer bounded pencils)
-        if (M == 24 && m.n >= 40) continue;
+        if ((M == 24 && m.n >= 40) || m.nbl > rows || m.nbr > rows) continue;
         if (m.n <= 256 ? M == 64 : (M == 32 && !m.periodic)) continue;
         if (pade::uneven_parts(m.n, M, parts) && build_variant(m, M, tab, v, &parts) == 0) pl.spike.push_back(v);
     }
@@ -258,7 +260,7 @@ int build_plan(int kind, int oper, int n, double dx, bool periodic, int bc1, int
         if (int rc = pade::build_stagg_system(oper, n, dx, bc1, bcn, sys)) return fail(rc, "operator construction failed");
     }
     const pade::OpMatrices &pm = sys_form ? sys : pl.mats;
-    add_spike_variants(pm, tab, pl);
+    add_spike_variants(pm, adj, tab, pl);
     if (m >= 4 && build_variant(pl.mats, m, tab, pl.generic) == 0) pl.has_generic = true;
     return 0;
 }
@@ -304,7 +306,7 @@ int build_all_plans(pade_op_s *op)
             if (int rc = operator_matrices(op->kind, pade::FILTER, op->n, op->dx, false, b1, bn, false, pl.mats))
                 return fail(rc, "operator construction failed");
             pl.mats.band = nn.band;      // (bc1, bcn) right-hand side, (0, 0) left-hand side
-            add_spike_variants(pl.mats, tab, pl);
+            add_spike_variants(pl.mats, false, tab, pl);
             if (op->n >= 4 && build_variant(pl.mats, op->n, tab, pl.generic) == 0) pl.has_generic = true;
             op->plans[{kFilterRhsBc, b1, bn, 0}] = std::move(pl);
         }
@@ -551,7 +553,7 @@ int plan_launch(const Plan &pl, bool periodic, int axis, const T *f, T *df, int 
     a.coef_len = v->coef_len;
     a.ncls = v->ncls;
     a.kq = v->kq;
-    for (int k = 0; k < pade::kMaxPartitions; k++) a.cls[k] = v->cls[k];
+    for (int k = 0; k < pade::kMaxPartitions; k++) a.cls4 |= (unsigned long long)v->cls[k] << (4 * k);
     a.ubase = v->parts.base;
     a.uextra = v->parts.extra;
     a.uunit = v->parts.unit;

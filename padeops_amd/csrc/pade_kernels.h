@@ -8,6 +8,12 @@
 namespace pade {
 
 constexpr int kBRowsDev = 8;
+// Special rows of a forward operator at one end, and of a staggered system
+// form (the transposes have up to 8).  Their results stay in registers while
+// the stencil runs: with four rows instead of eight the FP64 M = 32 bounded
+// kernels need 127 registers instead of 145 (four waves per SIMD instead of
+// three: 256^3 bounded y / z 60 / 61 -> 55 / 57 us).
+constexpr int kBRowsFwd = 4, kBRowsSys = 2;
 constexpr int kBColsDev = 16;
 
 // Device table layout of one plan (element offsets):
@@ -20,7 +26,7 @@ constexpr int kBColsDev = 16;
 //       then the reduced-system rows: periodic -> the 4 rows (4P each) of
 //       partition 0 (partition p uses them rotated by p); bounded -> the 4
 //       rows of every partition ([P][4][4P]).
-// Partition p uses block cls[p].  Uneven partitions store of every
+// Partition p uses block cls(p) of the launch arguments.  Uneven partitions store of every
 // partition's reduced-system rows the entries of its window only
 // ([P][4][4W], W = min(2 kq + 1, P); entry j belongs to partition p - kq + j,
 // cyclic when periodic, or to partition j when W = P).
@@ -46,7 +52,9 @@ struct ApplyArgs {
     int coef_len;          // length of the coefficient area
     int ncls;              // number of coefficient blocks
     int kq;                // reduced-system window: partitions p-kq..p+kq (2kq+1 >= P: all)
-    int cls[kMaxPartitions];
+    unsigned long long cls4;   // block of partition p in bits 4p .. 4p + 3 (shifted
+                               // out of a scalar register: an array indexed per
+                               // lane is a load from the argument segment)
     // uneven partitions: partition p < P - 1 has ubase + (p < uextra ? uunit : 0)
     // rows and starts at row p * ubase + min(p, uextra) * uunit, the last has M
     int ubase, uextra, uunit;

@@ -209,12 +209,12 @@ inline size_t spike_lds_bytes(size_t tsize, int M, int P, int PW, bool adj, int 
 // Right rows read the window from its last point (RS = 0: column c is point
 // n - 1 - c) or from the first right-halo point (RS = 1: point n - c, the
 // input of a staggered edge-to-cell operator has one point more).
-template <typename T, int M, int RS = 0>
+template <typename T, int M, int NB, int RS = 0>
 __device__ __forceinline__ void boundary_rows(const T (&w)[M + 8], const T *rows, int nrows, bool right,
-                                              T (&res)[kBRowsDev])
+                                              T (&res)[NB])
 {
 #pragma unroll
-    for (int r = 0; r < kBRowsDev; r++) {
+    for (int r = 0; r < NB; r++) {
         T s = T(0);
         if (r < nrows) {
 #pragma unroll
@@ -228,13 +228,13 @@ __device__ __forceinline__ void boundary_rows(const T (&w)[M + 8], const T *rows
 // B (or B^T) applied in place on the window: w[t+4] is point t on entry,
 // w[t] is row t on exit; special rows at the ends of a bounded pencil replace
 // the interior stencil there.
-template <typename T, int M, int RS = 0>
+template <typename T, int M, int NB, int RS = 0>
 __device__ __forceinline__ void apply_stencil(T (&w)[M + 8], const T *__restrict__ tab, const T *bnd,
                                               bool edge_left, bool edge_right, int nbl, int nbr)
 {
-    T lb[kBRowsDev], rb[kBRowsDev];
-    if (edge_left) boundary_rows<T, M>(w, bnd, nbl, false, lb);
-    if (edge_right) boundary_rows<T, M, RS>(w, bnd + 128, nbr, true, rb);
+    T lb[NB], rb[NB];
+    if (edge_left) boundary_rows<T, M, NB>(w, bnd, nbl, false, lb);
+    if (edge_right) boundary_rows<T, M, NB, RS>(w, bnd + 128, nbr, true, rb);
     T cst[9];
 #pragma unroll
     for (int k = 0; k < 9; k++) cst[k] = tab[k];
@@ -247,24 +247,14 @@ __device__ __forceinline__ void apply_stencil(T (&w)[M + 8], const T *__restrict
     }
     if (edge_left) {
 #pragma unroll
-        for (int r = 0; r < kBRowsDev; r++)
+        for (int r = 0; r < NB; r++)
             if (r < nbl) w[r] = lb[r];
     }
     if (edge_right) {
 #pragma unroll
-        for (int r = 0; r < kBRowsDev; r++)
+        for (int r = 0; r < NB; r++)
             if (r < nbr) w[M - 1 - r] = rb[r];
     }
-}
-
-// Occupancy target per instantiation (waves per SIMD): with it the compiler
-// schedules against the matching register budget (512 / waves VGPRs) instead
-// of hoisting every coefficient read of the unrolled loops.  FP64 M <= 32
-// fits 128 VGPRs, so two workgroups of 8 waves share a CU.
-template <typename T, int M>
-constexpr int spike_waves_per_eu()
-{
-    return sizeof(T) == 8 ? (M >= 64 ? 2 : 4) : (M >= 64 ? 4 : (M >= 32 ? 4 : 8));
 }
 
 template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, bool EPI, bool UNE = false, int ROWS = kWholeLines>
@@ -312,9 +302,24 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     const long long q = q0 + pen;
     const bool inrange = q < a.npencils;
     const bool valid = active && inrange;
-    const long long base0 = (q0 % a.A1) * a.B1 + (q0 / a.A1) * a.B2;
-    const unsigned loff =
-        inrange ? (unsigned)(((q % a.A1) * a.B1 + (q / a.A1) * a.B2 - base0) * (long long)sizeof(T)) : 0u;
+    // Base of the workgroup's first pencil and this lane's byte offset from it.
+    // x and z pencils are one run of npencils; y pencils runs of A1, the
+    // lane's run found from the first pencil's (32-bit: a launch has fewer
+    // than 2^32 pencils).  The 64-bit divisions this replaces were several
+    // hundred instructions before the first load.
+    long long base0;
+    unsigned loff = 0;
+    if (MODE == 1 || a.A1 == a.npencils) {
+        base0 = q0 * a.B1;
+        if (MODE != 1 && inrange) loff = (unsigned)(pen * a.B1 * (long long)sizeof(T));
+    } else {
+        const unsigned run = (unsigned)a.A1, r0 = (unsigned)q0 / run, i0 = (unsigned)q0 - r0 * run;
+        base0 = i0 * a.B1 + r0 * a.B2;
+        const unsigned i = i0 + pen;
+        const unsigned dr = run >= (unsigned)NPEN ? (i >= run ? 1u : 0u) : i / run;
+        if (inrange)
+            loff = (unsigned)((((long long)(i - dr * run) - i0) * a.B1 + (long long)dr * a.B2) * (long long)sizeof(T));
+    }
     const long long stp = a.stride;
     const T *__restrict__ fb = a.f + base0;
     T *__restrict__ ob = a.out + base0;
@@ -588,7 +593,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     }
 
     // coefficient blocks of this lane's partition
-    const int cls = BND || UNE ? a.cls[pc] : 0;
+    const int cls = BND || UNE ? (int)(a.cls4 >> (4 * pc)) & 15 : 0;
     const T *lu = coef + cls * 10 * M;      // [M][6]
     const T *S = lu + 6 * M;                // [M][4]
     const T *Qb = coef + a.ncls * 10 * M;   // periodic: [4][4P] of partition 0; bounded: [P][4][4P];
@@ -607,7 +612,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
                 rtail += bnd[128 + (kBRowsDev - 1) * kBColsDev + c] * w[M + 4 - c];
         }
     }
-    if constexpr (!ADJ) apply_stencil<T, M, MODE == 2 ? 1 : 0>(w, tab, bnd, edge_left, edge_right, a.nbl, a.nbr);
+    if constexpr (!ADJ) apply_stencil<T, M, MODE == 2 ? kBRowsSys : kBRowsFwd, MODE == 2 ? 1 : 0>(w, tab, bnd, edge_left, edge_right, a.nbl, a.nbr);
     // the padding slots of an uneven partition have a zero right-hand side
     if constexpr (UNE) {
 #pragma unroll
@@ -730,7 +735,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
         // rewrites -- every wave reads its halo first
         if constexpr (MODE == 1)
             if (exch) __syncthreads();
-        apply_stencil<T, M>(w, tab, bnd, edge_left, edge_right, a.nbl, a.nbr);
+        apply_stencil<T, M, kBRowsDev>(w, tab, bnd, edge_left, edge_right, a.nbl, a.nbr);
     }
 
     // ---------------------------------------------------------------- store
