@@ -218,7 +218,9 @@ int pade_op_dense_info(pade_op_t op, int oper, int prec, int axis, int f_dtype, 
  * the partition length, PW the partitions per wave, P the partitions per
  * pencil, generic = 1 for the one-lane-per-pencil path (M = n, P = 1), mode
  * 0 strided rows (y, z), 1 x pencils through LDS transposes, 2 the
- * staggered system form, launches the kernel launches of one apply, and
+ * staggered system form, launches the solves of one apply (2: the bounded
+ * cd06 second derivative, the first derivative twice, which the FP64
+ * partitioned kernels run as one kernel launch), and
  * uneven = 1 when M does not divide the rows and the partitions hold at most
  * M of them.  The
  * strided-row kernels address the field with 32-bit per-lane byte offsets (a

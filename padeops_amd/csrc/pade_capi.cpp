@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/padeops_hip.h"
+#include "pade_capi_internal.h"
 #include "pade_dense.h"
 #include "pade_err.h"
 #include "pade_kernels.h"
@@ -512,6 +513,18 @@ struct LaunchPlan {
     pade::ApplyArgs<T> a{};
 };
 
+template <typename T>
+void set_tables(const Variant &v, pade::FieldArgs<T> &fd)
+{
+    fd.nbl = v.nbl;
+    fd.nbr = v.nbr;
+    fd.coef_len = v.coef_len;
+    fd.ncls = v.ncls;
+    fd.kq = v.kq;
+    fd.cls4 = 0;
+    for (int k = 0; k < pade::kMaxPartitions; k++) fd.cls4 |= (unsigned long long)v.cls[k] << (4 * k);
+}
+
 // Variant, partitions per wave and mode of an apply along `axis` over
 // na x nb pencils; the table pointer of `a` is left to the caller.
 template <typename T>
@@ -520,8 +533,9 @@ int plan_launch(const Plan &pl, bool periodic, int axis, const T *f, T *df, int 
     const int n = pl.mats.n;
     pade::ApplyArgs<T> &a = L.a;
     a = pade::ApplyArgs<T>{};
-    a.f = f;
-    a.out = df;
+    a.nfields = 1;
+    a.fld[0].f = f;
+    a.fld[0].out = df;
     a.n = n;
     a.n_in = pl.mats.n_in ? pl.mats.n_in : n;
     a.periodic = periodic ? 1 : 0;
@@ -548,12 +562,7 @@ int plan_launch(const Plan &pl, bool periodic, int axis, const T *f, T *df, int 
     if (v->rect) mode = 2;   // strided rows (axis 3) of a staggered system form
     a.M = v->M;
     a.P = v->P;
-    a.nbl = v->nbl;
-    a.nbr = v->nbr;
-    a.coef_len = v->coef_len;
-    a.ncls = v->ncls;
-    a.kq = v->kq;
-    for (int k = 0; k < pade::kMaxPartitions; k++) a.cls4 |= (unsigned long long)v->cls[k] << (4 * k);
+    set_tables(*v, a.fld[0]);
     a.ubase = v->parts.base;
     a.uextra = v->parts.extra;
     a.uunit = v->parts.unit;
@@ -574,7 +583,7 @@ int apply_one(pade_op_t op, const Plan &pl, int axis, const T *f, T *df, int na,
     if (int rc = plan_launch<T>(pl, op->periodic, axis, f, df, na, nb, L)) return rc;
     pade::ApplyArgs<T> &a = L.a;
     const T *tables = std::is_same<T, double>::value ? (const T *)op->dtab64 : (const T *)op->dtab32;
-    a.tab = tables + L.v->off;
+    a.fld[0].tab = tables + L.v->off;
     const Variant *v = L.v;
     const int pw = L.pw, mode = L.mode, n = v->n;
     const bool use_generic = L.generic;
@@ -619,7 +628,7 @@ int apply_one(pade_op_t op, const Plan &pl, int axis, const T *f, T *df, int na,
             scratch_put<T>(ws, work, s);
             return rc;
         }
-        a.out = tmp;
+        a.fld[0].out = tmp;
     }
     e = pade::launch_generic<T>(a, kadj, work, s);
     if (e == hipSuccess && epi.on) e = pade::launch_axpby<T>(tmp, df, epi.alpha, epi.beta, (long long)count, s);
@@ -627,6 +636,13 @@ int apply_one(pade_op_t op, const Plan &pl, int axis, const T *f, T *df, int na,
     scratch_put<T>(ws, tmp, s);
     if (e != hipSuccess) return hip_fail(e, "generic_apply launch");
     return 0;
+}
+
+// Does one launch apply this operator twice?
+template <typename T>
+bool twice_ok(const LaunchPlan<T> &L)
+{
+    return std::is_same<T, double>::value && !L.generic && L.mode != 2 && (L.pw == 2 || L.pw == 8);
 }
 
 // Argument checks shared by every apply: 0 or the error code.
@@ -683,8 +699,9 @@ int apply_impl(pade_op_t op, int oper, int axis, const T *f, T *df, int na, int 
         return fill_zero(df, count, s);
     }
     if (op->kind == pade::CD06 && oper == pade::D2 && !op->periodic) {
-        // bounded cd06 second derivative: the first derivative applied twice.
-        // Without an epilogue and on the partitioned kernels, the second pass
+        // bounded cd06 second derivative: the first derivative applied twice,
+        // in one launch where the FP64 kernels for that serve the size.
+        // Otherwise, without an epilogue and on the partitioned kernels, the second pass
         // runs in place on df: a workgroup holds every partition of its
         // pencils, and all of a pencil is loaded and consumed before any of
         // it is stored (a workgroup barrier between the two when a pencil
@@ -692,11 +709,30 @@ int apply_impl(pade_op_t op, int oper, int axis, const T *f, T *df, int na, int 
         // every loaded one), so no intermediate array is needed.  The
         // one-lane-per-pencil path overwrites its input as it sweeps and
         // keeps the intermediate.
+        const Plan *p1 = find_plan(op, pade::D1, bc1, bcn, adj);
+        if (!p1) return 21;
+        LaunchPlan<T> L;
+        if (int rc = plan_launch<T>(*p1, op->periodic, axis, f, df, na, nb, L)) return rc;
+        if constexpr (std::is_same<T, double>::value) {
+            if (twice_ok(L)) {
+                // (the allocation-free entry point keeps its size limit, see apply_one)
+                if (ws.on && epi.on) {
+                    const size_t fields = L.v->uneven ? 2 : 1;
+                    T *unused = nullptr;
+                    if (int rc = scratch_get<T>(ws, fields * (size_t)count, s, &unused,
+                                                "cd06 second derivative intermediate"))
+                        return rc;
+                }
+                L.a.fld[0].tab = op->dtab64 + L.v->off;
+                L.a.axpby = epi.on ? 1 : 0;
+                L.a.alpha = epi.alpha;
+                L.a.beta = epi.beta;
+                hipError_t e = pade::launch_twice(L.a, L.v->M, L.pw, L.pw == 8 ? whole_pencil_waves() : 1,
+                                                  L.v->uneven, adj, L.mode, s);
+                return e == hipSuccess ? 0 : hip_fail(e, "spike_apply launch");
+            }
+        }
         if (!epi.on) {
-            const Plan *p1 = find_plan(op, pade::D1, bc1, bcn, adj);
-            if (!p1) return 21;
-            LaunchPlan<T> L;
-            if (int rc = plan_launch<T>(*p1, op->periodic, axis, f, df, na, nb, L)) return rc;
             if (!L.generic) {
                 int rc = apply_one<T>(op, *p1, axis, f, df, na, nb, adj, s, Epilogue<T>(), ws);
                 if (!rc) rc = apply_one<T>(op, *p1, axis, df, df, na, nb, adj, s, Epilogue<T>(), ws);
@@ -1152,6 +1188,63 @@ int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, 
 }  // extern "C"
 
 namespace pade {
+
+int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *flds, int na, int nb, int times, bool acc,
+                 double alpha, double beta, double *tmp, hipStream_t s)
+{
+    if (nf < 1 || nf > kMaxFields || times < 1 || times > 2) return fail(400, "bad batch");
+    for (int k = 0; k < nf; k++) {
+        if (int rc = check_apply(op, oper, axis, na, nb, flds[k].bc1, flds[k].bcn, false)) return rc;
+        if (!flds[k].f || !flds[k].out) return fail(400, "null array");
+    }
+    // one launch for all fields where they share a partitioned kernel
+    const bool composed = op->kind == CD06 && oper == D2 && !op->periodic;
+    if (op->n > 1 && !composed && op->kind != CD06STAGG) {
+        LaunchPlan<double> L;
+        bool one = true;
+        for (int k = 0; k < nf && one; k++) {
+            const Plan *pl = find_plan(op, oper, flds[k].bc1, flds[k].bcn, false);
+            if (!pl) return 21;
+            LaunchPlan<double> Lk;
+            if (int rc = plan_launch<double>(*pl, op->periodic, axis, flds[k].f, flds[k].out, na, nb, Lk)) return rc;
+            one = !Lk.generic && (times == 1 || twice_ok(Lk));
+            if (k == 0) L = Lk;
+            else one = one && Lk.v->M == L.v->M && Lk.v->P == L.v->P && Lk.pw == L.pw && Lk.v->uneven == L.v->uneven;
+            L.a.fld[k] = Lk.a.fld[0];
+            L.a.fld[k].tab = op->dtab64 + Lk.v->off;
+        }
+        if (one) {
+            L.a.nfields = nf;
+            L.a.axpby = acc ? 1 : 0;
+            L.a.alpha = alpha;
+            L.a.beta = beta;
+            const int gw = L.pw == 8 ? whole_pencil_waves() : 1;
+            hipError_t e;
+            if (times == 2) e = launch_twice(L.a, L.v->M, L.pw, gw, L.v->uneven, false, L.mode, s);
+            else if (L.v->uneven) e = launch_uneven<double>(L.a, L.v->M, false, L.mode, s);
+            else e = launch_spike<double>(L.a, L.v->M, L.pw, gw, false, L.mode, s);
+            return e == hipSuccess ? 0 : hip_fail(e, "spike_apply launch");
+        }
+    }
+    for (int k = 0; k < nf; k++) {
+        Epilogue<double> epi;
+        epi.on = acc;
+        epi.alpha = alpha;
+        epi.beta = beta;
+        const double *src = flds[k].f;
+        if (times == 2) {
+            if (!tmp) return fail(400, "no intermediate for a repeated apply");
+            if (int rc = apply_impl<double>(op, oper, axis, src, tmp, na, nb, flds[k].bc1, flds[k].bcn, false, s,
+                                            Epilogue<double>(), Workspace()))
+                return rc;
+            src = tmp;
+        }
+        if (int rc = apply_impl<double>(op, oper, axis, src, flds[k].out, na, nb, flds[k].bc1, flds[k].bcn, false, s,
+                                        epi, Workspace()))
+            return rc;
+    }
+    return 0;
+}
 
 bool apply_in_place_ok(pade_op_t op, int oper, int axis, int na, int nb, int bc1, int bcn)
 {

@@ -2,6 +2,8 @@
 // (internal to libpadeops_hip).
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include "../../include/padeops_hip.h"
 
 namespace pade {
@@ -13,5 +15,21 @@ namespace pade {
 // stored.  The one-lane-per-pencil path (which keeps intermediates in its
 // output), the bounded cd06 second derivative and edge outputs answer false.
 bool apply_in_place_ok(pade_op_t op, int oper, int axis, int na, int nb, int bc1, int bcn);
+
+// One operator along one axis of several FP64 device fields (at most six;
+// each with its own boundary codes), `times` (1 or 2) times each: out =
+// op^times(f), or with acc out = alpha op^times(f) + beta out.  One launch
+// where the fields share a partitioned kernel: a field of a small grid
+// leaves most of the chip idle, and a repeated operator keeps its
+// intermediate in registers; else one apply per field and repetition, with
+// `tmp` (a field, needed for times = 2) as the intermediate.  Outputs must
+// not overlap any input of the call.
+struct BatchField {
+    const double *f;
+    double *out;
+    int bc1, bcn;
+};
+int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *flds, int na, int nb, int times, bool acc,
+                 double alpha, double beta, double *tmp, hipStream_t s);
 
 }  // namespace pade

@@ -27,4 +27,16 @@ int cg_dt_maxima(long long n, const double *rho, const double *u, const double *
                  double dz, double gam, double hmin, unsigned long long *dev4, unsigned long long *host4, double *out,
                  hipStream_t s);
 
+// The three artificial properties before filtering (cgrid.F90:1083-1199) in
+// one pass: fl holds grad(rho), grad(e) and the fourth derivatives of the
+// strain magnitude, the dilatation and e (three planes each, in this order),
+// du the velocity gradients; dil holds the dilatation on entry and the
+// conductivity on return.
+int cg_lad(long long n, double Cmu, double Cbeta, double Ckap, double gam, const double *h, const double *rho,
+           const double *p, const double *T, const double *fl, const double *du, double *mustar, double *bulkstar,
+           double *dil, hipStream_t s);
+
+// The first RK45 stage (A = 0): Q = dt rhs, W += B Q.
+int cg_rk_first(long long n, double dt, double B, const double *rhs, double *Q, double *W, hipStream_t s);
+
 }  // namespace pade

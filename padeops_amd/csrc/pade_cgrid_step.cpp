@@ -15,6 +15,7 @@
 #include <string>
 
 #include "../../include/padeops_hip.h"
+#include "pade_capi_internal.h"
 #include "pade_cgrid.h"
 #include "pade_err.h"
 
@@ -49,11 +50,13 @@ struct pade_cgrid_s {
     // fields (caller's or owned): rho u v w p T e mu bulk kap, and W (5 planes)
     double *f[PADE_CG_NFIELDS] = {};
     bool own[PADE_CG_NFIELDS] = {};
-    // work: two operator-chain fields, du (9), gT (3), fluxes (15), rhs (5),
-    // Qtmp (5), g (3), d4 (3), and the three LAD scratch fields
+    // work: an intermediate (sizes without a partitioned kernel), du (9), gT
+    // (3), fluxes (15, before them the gradients and fourth derivatives of the
+    // LAD, and the filters' intermediates), rhs (5), Qtmp (5) and the three
+    // LAD properties before filtering
     double *work = nullptr;
-    double *t1 = nullptr, *t2 = nullptr, *du = nullptr, *gT = nullptr, *fl = nullptr, *rhs = nullptr,
-           *Q = nullptr, *g = nullptr, *d4 = nullptr, *mustar = nullptr, *func = nullptr, *dil = nullptr;
+    double *t1 = nullptr, *du = nullptr, *gT = nullptr, *fl = nullptr, *rhs = nullptr, *Q = nullptr,
+           *mustar = nullptr, *func = nullptr, *dil = nullptr;
     unsigned long long *dscal = nullptr;    // device: bad index, four maxima
     unsigned long long *hscal = nullptr;    // pinned host copy
     int step = 0;
@@ -65,69 +68,49 @@ namespace {
 double *F(pade_cgrid_t g, int k) { return g->f[k]; }
 double *Wp(pade_cgrid_t g, int k) { return g->f[PADE_CG_W] + (long long)k * g->N; }
 
-// One operator along `axis` (0, 1, 2) of a (nx, ny, nz) field: out = op(f),
-// or out = alpha op(f) + beta out; sign -1 negates the axis's bc pair.
-int apply(pade_cgrid_t g, pade_op_t op, int oper, int axis, const double *f, double *out, int sign, bool acc,
-          double alpha, double beta, hipStream_t s)
+// A field of a batch: its arrays and the sign of the axis's bc pair (-1: odd
+// at the walls).
+struct Item {
+    const double *f;
+    double *out;
+    int sign;
+};
+
+// One operator along `axis` (0, 1, 2) of several (nx, ny, nz) fields, in one
+// launch where the sizes allow: out = op^times(f), or with acc out = alpha
+// op^times(f) + out.
+template <int N>
+int apply(pade_cgrid_t g, pade_op_t op, int oper, int axis, const Item (&items)[N], int times, bool acc, double alpha,
+          hipStream_t s)
 {
     int na, nb;
     if (axis == 0) { na = g->n[1]; nb = g->n[2]; }
     else if (axis == 1) { na = g->n[0]; nb = g->n[2]; }
     else { na = g->n[0]; nb = g->n[1]; }
-    const int b1 = sign * g->bc[axis][0], bn = sign * g->bc[axis][1];
-    if (acc) return pade_op_apply_axpby(op, oper, axis + 1, alpha, f, beta, out, na, nb, b1, bn, s);
-    return pade_op_apply(op, oper, axis + 1, f, out, na, nb, b1, bn, s);
+    pade::BatchField b[N];
+    for (int k = 0; k < N; k++)
+        b[k] = {items[k].f, items[k].out, items[k].sign * g->bc[axis][0], items[k].sign * g->bc[axis][1]};
+    return pade::apply_fields(op, oper, axis + 1, N, b, na, nb, times, acc, alpha, 1.0, g->t1, s);
 }
 
-int d1(pade_cgrid_t g, int axis, const double *f, double *out, int sign, hipStream_t s)
+// cgrid.F90:1259-1336: y, then x, then z, each `times` times, of the N planes
+// src[k], through the work planes fl[0 .. 2N - 1] into dst[k], or added to
+// them; the axis flips[k] takes field k's bc pair negated.
+template <int N>
+int filter(pade_cgrid_t g, const double *const (&src)[N], double *const (&dst)[N], const int (&flips)[N],
+           pade_op_t const *ops, int times, bool add, hipStream_t s)
 {
-    return apply(g, g->der[axis], PADE_D1, axis, f, out, sign, false, 1.0, 0.0, s);
-}
-
-int d2(pade_cgrid_t g, int axis, const double *f, double *out, bool acc, double alpha, hipStream_t s)
-{
-    if (g->der_kind == PADE_CD06) return err(21, "CD06 is incomplete right now");   // derivatives.F90:524-525
-    return apply(g, g->der[axis], PADE_D2, axis, f, out, 1, acc, alpha, 1.0, s);
-}
-
-// cgrid.F90:446-478: the three planes of out (y, x, z order); the axis
-// `flip` takes its bc pair negated (a velocity component along its own axis)
-int gradient(pade_cgrid_t g, const double *f, double *out, int flip, hipStream_t s)
-{
-    for (int a : {1, 0, 2})
-        if (int rc = d1(g, a, f, out + (long long)a * g->N, a == flip ? -1 : 1, s)) return rc;
-    return 0;
-}
-
-// fourth derivative along one axis as the second derivative applied twice
-// (cgrid.F90:1089-1105); with acc, out += scale * d4 f
-int fourth(pade_cgrid_t g, const double *f, int axis, double *out, bool acc, double scale, hipStream_t s)
-{
-    if (int rc = d2(g, axis, f, g->t1, false, 1.0, s)) return rc;
-    return d2(g, axis, g->t1, out, acc, scale, s);
-}
-
-// cgrid.F90:1259-1336: y, then x, then z, each `times` times, buffers
-// alternating; the result replaces arr, or with add_to the last pass adds it
-// there (add_to += filtered)
-int filter(pade_cgrid_t g, double *arr, pade_op_t const *ops, int times, int flip, double *add_to, hipStream_t s)
-{
-    const int order[3] = {1, 0, 2};
-    const int total = 3 * times;
-    double *bufs[2] = {g->t1, g->t2};
-    const double *src = arr;
-    int k = 0;
-    for (int a : order)
-        for (int t = 0; t < times; t++, k++) {
-            const int sign = a == flip ? -1 : 1;
-            const bool last = k == total - 1;
-            if (last && add_to)
-                return apply(g, ops[a], PADE_FILTER, a, src, add_to, sign, true, 1.0, 1.0, s);
-            double *dst = last ? arr : bufs[k % 2];
-            if (int rc = apply(g, ops[a], PADE_FILTER, a, src, dst, sign, false, 1.0, 0.0, s)) return rc;
-            src = dst;
-        }
-    return 0;
+    Item y[N], x[N], z[N];
+    for (int k = 0; k < N; k++) {
+        double *a = g->fl + k * g->N, *b = g->fl + (N + k) * g->N;
+        y[k] = {src[k], a, flips[k] == 1 ? -1 : 1};
+        x[k] = {a, b, flips[k] == 0 ? -1 : 1};
+        z[k] = {b, dst[k], flips[k] == 2 ? -1 : 1};
+    }
+    int rc = apply(g, ops[1], PADE_FILTER, 1, y, times, false, 1.0, s);
+    if (!rc) rc = apply(g, ops[0], PADE_FILTER, 0, x, times, false, 1.0, s);
+    if (!rc) rc = apply(g, ops[2], PADE_FILTER, 2, z, times, add, 1.0, s);
+    return rc;
 }
 
 int transport(pade_cgrid_t g, hipStream_t s)
@@ -143,49 +126,53 @@ int transport(pade_cgrid_t g, hipStream_t s)
                               F(g, PADE_CG_MU), F(g, PADE_CG_BULK), F(g, PADE_CG_KAP), s);
 }
 
-// cgrid.F90:1058-1257 (no species diffusivity for one species)
-int lad(pade_cgrid_t g, hipStream_t s)
-{
-    const long long N = g->N;
-    const double hx = g->h[0], hy = g->h[1], hz = g->h[2];
-    int rc = pade_cg_strain(N, g->du, g->func, g->dil, s);
-    // artificial shear viscosity (:1083-1113): x, z, y as the reference sums
-    if (!rc) rc = pade::cg_fill(g->mustar, N, 0.0, s);
-    for (int a : {0, 2, 1})
-        if (!rc) rc = fourth(g, g->func, a, g->mustar, true, std::pow(g->h[a], 6), s);
-    if (!rc) rc = pade_cg_lad_mu(N, g->Cmu, F(g, PADE_CG_RHO), g->mustar, s);
-    if (!rc) rc = filter(g, g->mustar, g->gfil, 2, -1, F(g, PADE_CG_MU), s);      // (:1252)
-    // artificial bulk viscosity (:1115-1161)
-    if (!rc) rc = gradient(g, F(g, PADE_CG_RHO), g->g, -1, s);
-    for (int a : {0, 2, 1})
-        if (!rc) rc = fourth(g, g->dil, a, g->d4 + (long long)a * N, false, 1.0, s);
-    double *bulkstar = g->func;         // the sensor is no longer needed
-    if (!rc)
-        rc = pade_cg_lad_bulk(N, g->Cbeta, hx, hy, hz, F(g, PADE_CG_RHO), g->g, g->d4, g->du, g->dil, bulkstar, s);
-    if (!rc) rc = filter(g, bulkstar, g->gfil, 2, -1, F(g, PADE_CG_BULK), s);      // (:1253)
-    // artificial conductivity (:1163-1199)
-    if (!rc) rc = gradient(g, F(g, PADE_CG_E), g->g, -1, s);
-    for (int a : {0, 2, 1})
-        if (!rc) rc = fourth(g, F(g, PADE_CG_E), a, g->d4 + (long long)a * N, false, 1.0, s);
-    double *kapstar = g->dil;
-    if (!rc)
-        rc = pade_cg_lad_kap(N, g->Ckap, g->gam, hx, hy, hz, F(g, PADE_CG_RHO), F(g, PADE_CG_P), F(g, PADE_CG_T), g->g,
-                             g->d4, kapstar, s);
-    if (!rc) rc = filter(g, kapstar, g->gfil, 2, -1, F(g, PADE_CG_KAP), s);        // (:1254)
-    return rc;
-}
-
-// cgrid.F90:822-896 with getRHS_x/y/z (:898-1056), get_tau (:1338-1390) and
-// get_q (:1392-1444), into rhs (5 planes)
+// cgrid.F90:822-896 with getLAD (:1058-1257, no species diffusivity for one
+// species), getRHS_x/y/z (:898-1056), get_tau (:1338-1390) and get_q
+// (:1392-1444), into rhs (5 planes).
+//
+// Every operator pass takes all the fields that are ready for it in one
+// launch, and the repeated operators (the fourth derivative, the second
+// derivative twice, cgrid.F90:1089-1105; the Gaussian filter, twice per axis)
+// one launch instead of two: 9 launches for 18 gradient passes, 9 fourth
+// derivatives and 9 filter pairs, 3 for the 15 flux derivatives.  Before the
+// fluxes fill them, the planes fl hold grad(rho) (0-2), grad(e) (3-5) and the
+// fourth derivatives of the strain magnitude (6-8), the dilatation (9-11) and
+// e (12-14), planes x, y, z each.  Bound by memory from 128^3 up; below, by
+// the launch and latency of each pass.  Per step, 256^3 and 96 x 80 x 65
+// (walls in z): one launch per field and pass 39.0 and 4.0 ms, batched and
+// fused 32.4 and 1.72 ms.
 int rhs_impl(pade_cgrid_t g, double *rhs, hipStream_t s)
 {
     const long long N = g->N;
-    int rc = gradient(g, F(g, PADE_CG_U), g->du, 0, s);
-    if (!rc) rc = gradient(g, F(g, PADE_CG_V), g->du + 3 * N, 1, s);
-    if (!rc) rc = gradient(g, F(g, PADE_CG_W_VEL), g->du + 6 * N, 2, s);
-    if (!rc) rc = transport(g, s);
-    if (!rc) rc = lad(g, s);
-    if (!rc) rc = gradient(g, F(g, PADE_CG_T), g->gT, -1, s);
+    int rc = 0;
+    for (int a : {1, 0, 2}) {      // cgrid.F90:446-478: a velocity takes its own axis's bc pair negated
+        const Item grads[6] = {{F(g, PADE_CG_U), g->du + a * N, a == 0 ? -1 : 1},
+                               {F(g, PADE_CG_V), g->du + (3 + a) * N, a == 1 ? -1 : 1},
+                               {F(g, PADE_CG_W_VEL), g->du + (6 + a) * N, a == 2 ? -1 : 1},
+                               {F(g, PADE_CG_RHO), g->fl + a * N, 1},
+                               {F(g, PADE_CG_E), g->fl + (3 + a) * N, 1},
+                               {F(g, PADE_CG_T), g->gT + a * N, 1}};
+        if (!rc) rc = apply(g, g->der[a], PADE_D1, a, grads, 1, false, 1.0, s);
+    }
+    // an inviscid grid's properties are the artificial ones alone, written below
+    if (!rc && !g->inviscid) rc = transport(g, s);
+    if (!rc) rc = pade_cg_strain(N, g->du, g->func, g->dil, s);
+    if (!rc && g->der_kind == PADE_CD06) return err(21, "CD06 is incomplete right now");   // derivatives.F90:524-525
+    for (int a : {0, 2, 1}) {
+        const Item d4[3] = {{g->func, g->fl + (6 + a) * N, 1},
+                            {g->dil, g->fl + (9 + a) * N, 1},
+                            {F(g, PADE_CG_E), g->fl + (12 + a) * N, 1}};
+        if (!rc) rc = apply(g, g->der[a], PADE_D2, a, d4, 2, false, 1.0, s);
+    }
+    if (!rc)
+        rc = pade::cg_lad(N, g->Cmu, g->Cbeta, g->Ckap, g->gam, g->h, F(g, PADE_CG_RHO), F(g, PADE_CG_P),
+                          F(g, PADE_CG_T), g->fl, g->du, g->mustar, g->func, g->dil, s);
+    if (!rc) {                                                                       // (:1113, :1161, :1199, :1252-1254)
+        const double *const stars[3] = {g->mustar, g->func, g->dil};
+        double *const props[3] = {F(g, PADE_CG_MU), F(g, PADE_CG_BULK), F(g, PADE_CG_KAP)};
+        const int flips[3] = {-1, -1, -1};
+        rc = filter(g, stars, props, flips, g->gfil, 2, !g->inviscid, s);
+    }
     if (!rc)
         rc = pade_cg_fluxes(N, F(g, PADE_CG_W), F(g, PADE_CG_U), F(g, PADE_CG_V), F(g, PADE_CG_W_VEL),
                             F(g, PADE_CG_P), g->du, F(g, PADE_CG_MU), F(g, PADE_CG_BULK), F(g, PADE_CG_KAP), g->gT,
@@ -193,11 +180,11 @@ int rhs_impl(pade_cgrid_t g, double *rhs, hipStream_t s)
     // rhs = d(-fx)/dx (the x fluxes come negated), then rhs -= d(fy)/dy,
     // d(fz)/dz, accumulated inside the derivative kernel; every flux is odd at
     // the walls except the momentum flux along the derivative's own axis
-    for (int k = 0; k < 5 && !rc; k++) rc = d1(g, 0, g->fl + k * N, rhs + k * N, k == 1 ? 1 : -1, s);
-    for (int a : {1, 2})
-        for (int k = 0; k < 5 && !rc; k++)
-            rc = apply(g, g->der[a], PADE_D1, a, g->fl + (5LL * a + k) * N, rhs + k * N, k == 1 + a ? 1 : -1, true,
-                       -1.0, 1.0, s);
+    for (int a : {0, 1, 2}) {
+        Item fx[5];
+        for (int k = 0; k < 5; k++) fx[k] = {g->fl + (5LL * a + k) * N, rhs + k * N, k == 1 + a ? 1 : -1};
+        if (!rc) rc = apply(g, g->der[a], PADE_D1, a, fx, 1, a != 0, a == 0 ? 1.0 : -1.0, s);
+    }
     return rc;
 }
 
@@ -299,8 +286,8 @@ int pade_cgrid_create(int nx, int ny, int nz, double dx, double dy, double dz, i
         }
         g->f[k] = p;
     }
-    // t1 t2 | du 9 | gT 3 | fl 15 | rhs 5 | Q 5 | g 3 | d4 3 | mustar func dil
-    const int nwork = 2 + 9 + 3 + 15 + 5 + 5 + 3 + 3 + 3;
+    // t1 | du 9 | gT 3 | fl 15 | rhs 5 | Q 5 | mustar func dil
+    const int nwork = 1 + 9 + 3 + 15 + 5 + 5 + 3;
     hipError_t e = hipMalloc(&g->work, fb * nwork);
     if (e == hipSuccess) e = hipMalloc(&g->dscal, 8 * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipHostMalloc(&g->hscal, 8 * sizeof(unsigned long long), hipHostMallocDefault);
@@ -310,8 +297,8 @@ int pade_cgrid_create(int nx, int ny, int nz, double dx, double dy, double dz, i
     }
     double *w = g->work;
     auto take = [&](int k) { double *p = w; w += (long long)k * g->N; return p; };
-    g->t1 = take(1); g->t2 = take(1); g->du = take(9); g->gT = take(3); g->fl = take(15); g->rhs = take(5);
-    g->Q = take(5); g->g = take(3); g->d4 = take(3); g->mustar = take(1); g->func = take(1); g->dil = take(1);
+    g->t1 = take(1); g->du = take(9); g->gT = take(3); g->fl = take(15); g->rhs = take(5);
+    g->Q = take(5); g->mustar = take(1); g->func = take(1); g->dil = take(1);
     *out = g;
     return 0;
 }
@@ -425,7 +412,6 @@ int pade_cgrid_advance_rk45(pade_cgrid_t g, double dt, pade_cgrid_hook hook_bc, 
     if (dt > 0.0) g->dt = dt;
     int rc = 0;
     if (g->step == 0) rc = post_bc_impl(g, s);         // get_e_from_p, get_T (:675-679)
-    if (!rc) rc = pade::cg_fill(g->Q, 5 * g->N, 0.0, s);
     double Qt = 0.0;
     for (int isub = 0; isub < 5 && !rc; isub++) {
         long long bad = -1;
@@ -442,12 +428,17 @@ int pade_cgrid_advance_rk45(pade_cgrid_t g, double dt, pade_cgrid_hook hook_bc, 
                                 ")");
         }
         rc = rhs_impl(g, g->rhs, s);
-        if (!rc) rc = pade_cg_rk_stage(g->N, g->dt, kRkA[isub], kRkB[isub], g->rhs, g->Q, F(g, PADE_CG_W), s);
+        if (!rc && isub == 0)          // A(1) = 0: Qtmp starts here
+            rc = pade::cg_rk_first(g->N, g->dt, kRkB[0], g->rhs, g->Q, F(g, PADE_CG_W), s);
+        else if (!rc)
+            rc = pade_cg_rk_stage(g->N, g->dt, kRkA[isub], kRkB[isub], g->rhs, g->Q, F(g, PADE_CG_W), s);
         Qt = g->dt + kRkA[isub] * Qt;
         g->tsim += kRkB[isub] * Qt;
         // the momentum component along an axis is odd at its walls (:701-706)
         const int flips[5] = {-1, 0, 1, 2, -1};
-        for (int k = 0; k < 5 && !rc; k++) rc = filter(g, Wp(g, k), g->fil, 1, flips[k], nullptr, s);
+        double *const W[5] = {Wp(g, 0), Wp(g, 1), Wp(g, 2), Wp(g, 3), Wp(g, 4)};
+        const double *const Wc[5] = {W[0], W[1], W[2], W[3], W[4]};
+        if (!rc) rc = filter(g, Wc, W, flips, g->fil, 1, false, s);
         if (!rc) rc = pade_cgrid_get_primitive(g, stream);
         if (!rc && hook_bc) {
             hook_bc(g, user);

@@ -35,26 +35,36 @@ constexpr int kOffBr = 144;
 constexpr int kOffCoef = 272;
 constexpr int kMaxPartitions = 16;
 
+// One field of a launch: its arrays, and the table of its operator (boundary
+// codes may differ between the fields of a launch).
 template <typename T>
-struct ApplyArgs {
+struct FieldArgs {
     const T *f;
     T *out;
     const T *tab;
+    unsigned long long cls4;   // block of partition p in bits 4p .. 4p + 3 (shifted
+                               // out of a scalar register: an array indexed per
+                               // lane is a load from the argument segment)
+    int nbl, nbr;
+    int coef_len;          // length of the coefficient area
+    int ncls;              // number of coefficient blocks
+    int kq;                // reduced-system window: partitions p-kq..p+kq (2kq+1 >= P: all)
+};
+
+constexpr int kMaxFields = 6;
+
+template <typename T>
+struct ApplyArgs {
+    int nfields;           // grid y
     long long npencils;
     long long A1, B1, B2;  // pencil q -> base offset (q % A1)*B1 + (q / A1)*B2
     long long stride;      // element distance between consecutive points of a pencil
-    int n, M, P, periodic, nbl, nbr;
+    int n, M, P, periodic;
     int n_in;              // input points per pencil: n except for the
                            // staggered cell <-> edge operators (generic path:
                            // the right boundary rows read in[n_in - 1 - c];
                            // strided-row mode 2: in[n - c], n_in = n or n + 1)
     int tail;              // mode 2: one more output row after the n solved
-    int coef_len;          // length of the coefficient area
-    int ncls;              // number of coefficient blocks
-    int kq;                // reduced-system window: partitions p-kq..p+kq (2kq+1 >= P: all)
-    unsigned long long cls4;   // block of partition p in bits 4p .. 4p + 3 (shifted
-                               // out of a scalar register: an array indexed per
-                               // lane is a load from the argument segment)
     // uneven partitions: partition p < P - 1 has ubase + (p < uextra ? uunit : 0)
     // rows and starts at row p * ubase + min(p, uextra) * uunit, the last has M
     int ubase, uextra, uunit;
@@ -63,6 +73,8 @@ struct ApplyArgs {
                            // (workgroup i runs on XCD i % 8) takes runs of C
                            // consecutive workgroups; < 0 a contiguous eighth
     T alpha, beta;
+    // last, so that a launch of one field reads one stretch of arguments
+    FieldArgs<T> fld[kMaxFields];
 };
 
 // mode 0: strided rows (y, z); 1: x pencils through LDS transposes; 2:
@@ -75,6 +87,11 @@ hipError_t launch_spike(const ApplyArgs<T> &a, int M, int PW, int GW, bool adj, 
 // of M), two partitions per wave; modes as above.
 template <typename T>
 hipError_t launch_uneven(const ApplyArgs<T> &a, int M, bool adj, int mode, hipStream_t s);
+
+// The operator applied twice in one pass, even or uneven partitions, modes 0
+// and 1, two partitions per wave or whole-pencil x waves (FP64).
+hipError_t launch_twice(const ApplyArgs<double> &a, int M, int PW, int GW, bool uneven, bool adj, int mode,
+                        hipStream_t s);
 
 template <typename T>
 hipError_t launch_generic(const ApplyArgs<T> &a, bool adj, T *work, hipStream_t s);

@@ -15,22 +15,23 @@ __global__ __launch_bounds__(256) void generic_apply(ApplyArgs<T> a, T *__restri
     const long long base = (q % a.A1) * a.B1 + (q / a.A1) * a.B2;
     const long long st = a.stride;
     const int n = a.n;
-    const T *__restrict__ tab = a.tab;
+    const FieldArgs<T> &fd = a.fld[0];
+    const T *__restrict__ tab = fd.tab;
     const T *__restrict__ lu = tab + kOffCoef;          // [n][6]
     const T *__restrict__ S = lu + 6 * n;               // [n][4]
     const T *__restrict__ Q = lu + 10 * n;              // [4][4]
-    T *y = ADJ ? work : a.out;
+    T *y = ADJ ? work : fd.out;
 
     // B applied to `src` (src_n points per pencil) at row i
     auto stencil_row = [&](const T *src, int src_n, int i) -> T {
         if (!a.periodic) {
-            if (i < a.nbl) {
+            if (i < fd.nbl) {
                 T s = T(0);
                 for (int c = 0; c < kBColsDev && c < src_n; c++)
                     s += tab[kOffBl + i * kBColsDev + c] * src[base + (long long)c * st];
                 return s;
             }
-            if (i >= n - a.nbr) {
+            if (i >= n - fd.nbr) {
                 const int r = n - 1 - i;
                 T s = T(0);
                 for (int c = 0; c < kBColsDev && c < src_n; c++)
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(256) void generic_apply(ApplyArgs<T> a, T *__restri
     // row as it goes (f and the output never overlap)
     T zm1 = T(0), zm2 = T(0);
     for (int i = 0; i < n; i++) {
-        const T r = ADJ ? a.f[base + (long long)i * st] : stencil_row(a.f, a.n_in, i);
+        const T r = ADJ ? fd.f[base + (long long)i * st] : stencil_row(fd.f, a.n_in, i);
         const T z = i == 0 ? r : r - lu[i * 6 + 0] * zm1 - lu[i * 6 + 1] * zm2;
         y[base + (long long)i * st] = z;
         zm2 = zm1;
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(256) void generic_apply(ApplyArgs<T> a, T *__restri
         }
     }
     if (ADJ) {
-        for (int i = 0; i < n; i++) a.out[base + (long long)i * st] = stencil_row(work, n, i);
+        for (int i = 0; i < n; i++) fd.out[base + (long long)i * st] = stencil_row(work, n, i);
     }
 }
 

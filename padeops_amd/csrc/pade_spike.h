@@ -257,10 +257,12 @@ __device__ __forceinline__ void apply_stencil(T (&w)[M + 8], const T *__restrict
     }
 }
 
-template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, bool EPI, bool UNE = false, int ROWS = kWholeLines>
+template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, bool EPI, bool UNE = false, int ROWS = kWholeLines,
+          int REP = 1>
 __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
 {
     constexpr int NPEN = 64 / PW;
+    const FieldArgs<T> &fd = a.fld[blockIdx.y];
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T *smem = reinterpret_cast<T *>(smem_raw);
     constexpr bool WHOLE = MODE == 1 && PW >= 4;
@@ -321,9 +323,9 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
             loff = (unsigned)((((long long)(i - dr * run) - i0) * a.B1 + (long long)dr * a.B2) * (long long)sizeof(T));
     }
     const long long stp = a.stride;
-    const T *__restrict__ fb = a.f + base0;
-    T *__restrict__ ob = a.out + base0;
-    const T *__restrict__ tab = a.tab;
+    const T *__restrict__ fb = fd.f + base0;
+    T *__restrict__ ob = fd.out + base0;
+    const T *__restrict__ tab = fd.tab;
     const bool edge_left = BND && p == 0;
     const bool edge_right = BND && p == P - 1;
 
@@ -338,7 +340,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     auto row_pen = [](int r) { return PMAJ ? r % NPEN : r / PW; };
     auto row_part = [](int r) { return PMAJ ? r / NPEN : r % PW; };
     auto tile_row = [](int pn, int pt) { return PMAJ ? pt * NPEN + pn : pn * PW + pt; };
-    T *bnd = smem + (WHOLE ? 0 : (ADJ && MODE != 1 ? 12 : 4) * P * NPEN);   // [256] (bounded)
+    T *bnd = smem + (WHOLE ? 0 : ((ADJ || REP > 1) && MODE != 1 ? 12 : 4) * P * NPEN);   // [256] (bounded)
     T *coef = bnd + (BND ? 256 : 0);                    // [coef_len]
     constexpr int XT = xtile_points(sizeof(T), M), PAD = xtile_row(sizeof(T), M);
     constexpr int VL = 16 / sizeof(T);                  // elements per 16-byte lane
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     // take 64 / LPR consecutive tile rows.
     constexpr bool PINS = WHOLE && XT / VL == NPEN && 64 / LPR == PW;
     auto instr_row = [&](int s_) { return PINS ? tile_row(s_, lane / LPR) : s_ * (64 / LPR) + lane / LPR; };
-    const int xt0 = ((int)(coef - smem) + a.coef_len + VL - 1) / VL * VL;
+    const int xt0 = ((int)(coef - smem) + fd.coef_len + VL - 1) / VL * VL;
     T *xt = smem + xt0 + wave_id * 64 * PAD;
     // [8P][NPEN] adjoint halo: 8P * NPEN <= waves * 64 * PAD since PAD >= 8
     // (a whole-pencil wave: in its own tile, 8P * NPEN <= 64 * PAD)
@@ -390,7 +392,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     // elements.
     {
         const T *g = tab + kOffCoef;
-        const int len = a.coef_len;
+        const int len = fd.coef_len;
         const int nt = blockDim.x;
         constexpr int U = BND ? 16 : 8;
         for (int b0 = threadIdx.x; b0 < len; b0 += U * nt) {
@@ -420,7 +422,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
             for (int t = 4; t < M + 4; t++) w[t] = ld_s<BND && ROWS == kWholeLines>(fb + (long long)(pw0 - 4 + t) * stp, active ? hoff : loff);
             // halo rows (wrapped per partition, or clamped at the ends of a
             // bounded pencil, where the boundary rows replace the stencil)
-            const T *fq = a.f + base0 + (long long)(loff / sizeof(T));
+            const T *fq = fd.f + base0 + (long long)(loff / sizeof(T));
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const int jl = wrap_index(pM - 4 + k, n, !BND);
@@ -593,10 +595,10 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     }
 
     // coefficient blocks of this lane's partition
-    const int cls = BND || UNE ? (int)(a.cls4 >> (4 * pc)) & 15 : 0;
+    const int cls = BND || UNE ? (int)(fd.cls4 >> (4 * pc)) & 15 : 0;
     const T *lu = coef + cls * 10 * M;      // [M][6]
     const T *S = lu + 6 * M;                // [M][4]
-    const T *Qb = coef + a.ncls * 10 * M;   // periodic: [4][4P] of partition 0; bounded: [P][4][4P];
+    const T *Qb = coef + fd.ncls * 10 * M;   // periodic: [4][4P] of partition 0; bounded: [P][4][4P];
                                             // uneven: [P][4][4W], W = min(2 kq + 1, P)
 
     lds_barrier();   // coefficients visible
@@ -612,7 +614,11 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
                 rtail += bnd[128 + (kBRowsDev - 1) * kBColsDev + c] * w[M + 4 - c];
         }
     }
-    if constexpr (!ADJ) apply_stencil<T, M, MODE == 2 ? kBRowsSys : kBRowsFwd, MODE == 2 ? 1 : 0>(w, tab, bnd, edge_left, edge_right, a.nbl, a.nbr);
+    // REP > 1: the operator applied REP times, the intermediate never leaving
+    // the registers (halos through LDS as in the adjoint)
+#pragma unroll 1
+    for (int rep = 0; rep < REP; rep++) {
+    if constexpr (!ADJ) apply_stencil<T, M, MODE == 2 ? kBRowsSys : kBRowsFwd, MODE == 2 ? 1 : 0>(w, tab, bnd, edge_left, edge_right, fd.nbl, fd.nbr);
     // the padding slots of an uneven partition have a zero right-hand side
     if constexpr (UNE) {
 #pragma unroll
@@ -655,7 +661,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
         }
         T u0 = T(0), u1 = T(0), u2 = T(0), u3 = T(0);
         const int m = 4 * P;
-        const int kq = a.kq;
+        const int kq = fd.kq;
         const bool all = 2 * kq + 1 >= P;
         const int d0 = all ? 0 : -kq;
         const int d1 = all ? P - 1 : kq;
@@ -690,10 +696,11 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
         }
     }
 
-    if constexpr (ADJ) {
-        // --------------------------------- B^T of the solved values (halo via LDS)
+    if (ADJ || rep + 1 < REP) {
+        // ------------- the solved values with their halos (via LDS) as a window
         const bool exch = !BND || P > 1;
         if (exch) {
+            if constexpr (WHOLE) wave_lds_sync();        // the tips, in the same place, have been read
             if (active) {
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
@@ -732,10 +739,12 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
                 else if (hasr) w[M + 4 + k] = halo[(8 * pr + M + k - mrows) * NPEN + pen];
         }
         // x: the halo lives in the transpose tiles, which the store phase
-        // rewrites -- every wave reads its halo first
+        // (whole-pencil waves: the next pass's tips) rewrites -- every wave
+        // reads its halo first
         if constexpr (MODE == 1)
             if (exch) __syncthreads();
-        apply_stencil<T, M, kBRowsDev>(w, tab, bnd, edge_left, edge_right, a.nbl, a.nbr);
+        if constexpr (ADJ) apply_stencil<T, M, kBRowsDev>(w, tab, bnd, edge_left, edge_right, fd.nbl, fd.nbr);
+    }
     }
 
     // ---------------------------------------------------------------- store
@@ -885,12 +894,29 @@ inline long long xcd_run_bytes()
     return v;
 }
 
+// The split that the uneven kernels' addressing relies on (UnevenParts).
+template <typename T>
+bool uneven_layout_ok(const ApplyArgs<T> &a, int M)
+{
+    const int inner = (a.P - 1) * a.ubase + std::min(a.P - 1, a.uextra) * a.uunit;
+    return a.P >= 2 && a.P <= kMaxPartitions && a.ubase >= kMinRows && a.ubase + (a.uextra ? a.uunit : 0) <= M &&
+           a.uextra >= 0 && a.uextra < a.P && inner + M == a.n;
+}
+
 // Layout of the row segments of a strided-row launch.
+template <typename T>
+uintptr_t field_bits(const ApplyArgs<T> &a)
+{
+    uintptr_t bits = 0;
+    for (int k = 0; k < a.nfields; k++)
+        bits |= reinterpret_cast<uintptr_t>(a.fld[k].f) | reinterpret_cast<uintptr_t>(a.fld[k].out);
+    return bits;
+}
+
 template <typename T>
 RowLayout row_layout(const ApplyArgs<T> &a)
 {
-    const auto bits = reinterpret_cast<uintptr_t>(a.f) | reinterpret_cast<uintptr_t>(a.out) |
-                      (uintptr_t)(a.stride * (long long)sizeof(T)) | (uintptr_t)(a.B2 * (long long)sizeof(T));
+    const auto bits = field_bits(a) | (uintptr_t)(a.stride * (long long)sizeof(T)) | (uintptr_t)(a.B2 * (long long)sizeof(T));
     if (bits % 128 == 0) return kWholeLines;
     return bits % 64 == 0 ? kHalfLines : kShared;
 }
@@ -898,18 +924,20 @@ RowLayout row_layout(const ApplyArgs<T> &a)
 // Workgroups per XCD run where neighbouring workgroups share lines.
 constexpr int kSharedRun = 64;
 
-template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, bool EPI, bool UNE>
+template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, bool EPI, bool UNE, int REP>
 hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
 {
     constexpr int NPEN = 64 / PW;
     constexpr bool WHOLE = MODE == 1 && PW >= 4;
     ApplyArgs<T> a = a_in;
     const int waves = WHOLE ? gw : (a.P + PW - 1) / PW;
-    const size_t lds = spike_lds_bytes(sizeof(T), M, a.P, PW, ADJ, MODE, a.coef_len, BND, gw);
+    int coef_len = 0;
+    for (int k = 0; k < a.nfields; k++) coef_len = std::max(coef_len, a.fld[k].coef_len);
+    const size_t lds = spike_lds_bytes(sizeof(T), M, a.P, PW, ADJ || REP > 1, MODE, coef_len, BND, gw);
     const long long nblk = (a.npencils + (long long)NPEN * gw - 1) / ((long long)NPEN * gw);
     a.remap = 0;
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(64 * waves), lds, s, a);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nblk, (unsigned)a.nfields), dim3(64 * waves), lds, s, a);
         return hipGetLastError();
     };
     if constexpr (MODE == 1) {
@@ -926,24 +954,24 @@ hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
         // uneven x partitions may start anywhere in a line: cached stores, as
         // for strided rows (129 x 512 x 512 FP64 x 155 -> 229 Gpts/s)
         if constexpr (UNE) {
-            const auto bits = reinterpret_cast<uintptr_t>(a.out) | (uintptr_t)(a.n * sizeof(T)) |
+            const auto bits = field_bits(a) | (uintptr_t)(a.n * sizeof(T)) |
                               (uintptr_t)(a.uunit * sizeof(T));
-            if (bits % 128) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared>);
+            if (bits % 128) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared, REP>);
         }
-        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines>);
+        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines, REP>);
     } else {
         const RowLayout rows = row_layout(a);
-        if (rows == kWholeLines) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines>);
+        if (rows == kWholeLines) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines, REP>);
         int c = kSharedRun;
         while (c > 1 && nblk < 16LL * c) c /= 2;
         if (c >= 2) a.remap = c;
-        if (rows == kShared) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared>);
+        if (rows == kShared) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared, REP>);
         // without an epilogue periodic kernels load alike for whole and half lines
-        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, BND || EPI ? kHalfLines : kWholeLines>);
+        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, (BND || EPI ? kHalfLines : kWholeLines), REP>);
     }
 }
 
-template <typename T, int M, int PW, bool ADJ, int MODE, bool UNE = false>
+template <typename T, int M, int PW, bool ADJ, int MODE, bool UNE = false, int REP = 1>
 hipError_t launch_spike_t(const ApplyArgs<T> &a, int gw, hipStream_t s)
 {
     constexpr bool WHOLE = MODE == 1 && PW >= 4;
@@ -954,18 +982,18 @@ hipError_t launch_spike_t(const ApplyArgs<T> &a, int gw, hipStream_t s)
     if constexpr (MODE == 2) {
         // staggered operators: forward, bounded, strided rows only
         if (ADJ || a.periodic || a.n_in < a.n || a.n_in > a.n + 1) return hipErrorInvalidValue;
-        return epi ? launch_kernel<T, M, PW, false, 2, true, true, UNE>(a, gw, s)
-                   : launch_kernel<T, M, PW, false, 2, true, false, UNE>(a, gw, s);
+        return epi ? launch_kernel<T, M, PW, false, 2, true, true, UNE, REP>(a, gw, s)
+                   : launch_kernel<T, M, PW, false, 2, true, false, UNE, REP>(a, gw, s);
     } else if constexpr (ADJ) {
         // (a periodic adjoint runs the forward kernel on the transposed tables)
         if (a.periodic) return hipErrorInvalidValue;
-        return launch_kernel<T, M, PW, true, MODE, true, false, UNE>(a, gw, s);
+        return launch_kernel<T, M, PW, true, MODE, true, false, UNE, REP>(a, gw, s);
     } else {
         if (a.periodic)
-            return epi ? launch_kernel<T, M, PW, false, MODE, false, true, UNE>(a, gw, s)
-                       : launch_kernel<T, M, PW, false, MODE, false, false, UNE>(a, gw, s);
-        return epi ? launch_kernel<T, M, PW, false, MODE, true, true, UNE>(a, gw, s)
-                   : launch_kernel<T, M, PW, false, MODE, true, false, UNE>(a, gw, s);
+            return epi ? launch_kernel<T, M, PW, false, MODE, false, true, UNE, REP>(a, gw, s)
+                       : launch_kernel<T, M, PW, false, MODE, false, false, UNE, REP>(a, gw, s);
+        return epi ? launch_kernel<T, M, PW, false, MODE, true, true, UNE, REP>(a, gw, s)
+                   : launch_kernel<T, M, PW, false, MODE, true, false, UNE, REP>(a, gw, s);
     }
 }
 

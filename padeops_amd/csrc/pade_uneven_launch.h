@@ -22,11 +22,7 @@ static hipError_t launch_uneven_m(const ApplyArgs<T> &a, bool adj, int mode, hip
 template <typename T>
 hipError_t launch_uneven(const ApplyArgs<T> &a, int M, bool adj, int mode, hipStream_t s)
 {
-    // the layout that the kernel's addressing relies on (UnevenParts)
-    const int inner = (a.P - 1) * a.ubase + std::min(a.P - 1, a.uextra) * a.uunit;
-    if (a.P < 2 || a.P > kMaxPartitions || a.ubase < kMinRows || a.ubase + (a.uextra ? a.uunit : 0) > M ||
-        a.uextra < 0 || a.uextra >= a.P || inner + M != a.n)
-        return hipErrorInvalidValue;
+    if (!uneven_layout_ok(a, M)) return hipErrorInvalidValue;
     switch (M) {
     case 16: return launch_uneven_m<T, 16>(a, adj, mode, s);
     case 24: return launch_uneven_m<T, 24>(a, adj, mode, s);

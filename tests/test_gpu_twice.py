@@ -1,0 +1,114 @@
+"""An operator applied twice in one launch, and several fields in one launch.
+
+The bounded cd06 second derivative (the first derivative twice) is the public
+call that runs the twice-applied kernels directly: forward, accumulating and
+adjoint, even and uneven partitions, every axis, against the dense operator
+squared (FP64, 1e-12).  The compressible step runs both through its batched
+passes; its grids here cover the one-launch path on even and uneven sizes and
+the one-field-at-a-time path of an axis without a partitioned kernel, viscous
+(properties added to) and inviscid (properties written), at the tolerance and
+step of the suite's other step tests."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import cgrid_step as cg
+from oracle import pade_dense as pd
+import padeops_amd as po
+from padeops_amd import _lib
+from padeops_amd import cgrid as gcg
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+@pytest.mark.parametrize("n", [16, 24, 37, 64, 75, 96, 129, 257, 512])
+@pytest.mark.parametrize("axis", [1, 2, 3])
+def test_bounded_cd06_second_derivative(n, axis):
+    op = po.cd06()
+    assert op.init(n, 0.05, False, 0, 0) == 0
+    shape = [67, 5]
+    shape.insert(axis - 1, n)
+    f = po.as_fortran(torch.tensor(np.random.default_rng(n).standard_normal(shape), device=DEV))
+    fh = f.cpu().numpy()
+    D = pd.dense_operator("cd06", "d1", n, 0.05, False, 0, 0)
+    D2 = D @ D
+    ref = pd.apply_axis(D2, fh, axis - 1)
+    out = po.fortran_empty(f.shape, device=DEV)
+    print(f"cd06 d2 bounded n {n} axis {axis}", flush=True)
+    op._apply(_lib.PADE_D2, axis, f, out, 67, 5)
+    assert rel(out.cpu().numpy(), ref) < 1e-12
+    acc = f.clone()
+    op._apply(_lib.PADE_D2, axis, f, acc, 67, 5, alpha=0.5, beta=-2.0)
+    assert rel(acc.cpu().numpy(), 0.5 * ref - 2.0 * fh) < 1e-12
+    op._apply(_lib.PADE_D2, axis, f, out, 67, 5, adjoint=True)
+    assert rel(out.cpu().numpy(), pd.apply_axis(D2.T, fh, axis - 1)) < 1e-12
+
+
+def _state(shape, seed):
+    rng = np.random.default_rng(seed)
+    h = tuple(2 * np.pi / n for n in shape)
+    X = np.meshgrid(*[np.arange(n) * hh for n, hh in zip(shape, h)], indexing="ij")
+
+    def wave(amp, mean):
+        k, ph = rng.integers(1, 3, size=(4, 3)), rng.uniform(0, 2 * np.pi, 4)
+        return mean + amp * sum(np.cos(k[m, 0] * X[0] + k[m, 1] * X[1] + k[m, 2] * X[2] + ph[m]) for m in range(4)) / 4
+    return dict(rho=wave(0.1, 1.0), u=wave(0.3, 0.1), v=wave(0.3, -0.2), w=wave(0.3, 0.15), p=wave(0.1, 1.0)), h
+
+
+@pytest.mark.parametrize("shape,periodic,bc", [
+    ((32, 40, 25), (True, True, True), ((0, 0),) * 3),
+    ((48, 24, 33), (True, True, False), ((0, 0), (0, 0), (0, 0)))])
+@pytest.mark.parametrize("inviscid", [True, False])
+def test_batched_step_matches_oracle(shape, periodic, bc, inviscid):
+    s0, h = _state(shape, sum(shape))
+    h = tuple(1.0 / (n - 1) if not p else hh for n, p, hh in zip(shape, periodic, h))
+    kw = dict(gam=1.4, Rgas=1.0, inviscid=inviscid, mu_ref=0.01, T_ref=1.0, visc_n=0.75, Pr=0.7, periodic=periodic, bc=bc)
+    og = cg.Grid(shape, h, **kw)
+    s1 = og.advance(s0, 1e-4)
+    g = gcg.cgrid(*shape, *h, **kw)
+    for c in ("rho", "u", "v", "w", "p"):
+        getattr(g, c).copy_(torch.tensor(s0[c], device=DEV))
+    g.mu.fill_(7.0)              # an inviscid grid overwrites what its properties held
+    g.post_bc()
+    g.get_conserved()
+    print(f"batched step {shape} periodic {periodic} inviscid {inviscid}", flush=True)
+    g.advance_RK45(1e-4)
+    torch.cuda.synchronize()
+    vscale = max(np.abs(s1[c]).max() for c in ("u", "v", "w"))
+    for c in ("rho", "u", "v", "w", "p", "T", "e"):
+        scale = vscale if c in ("u", "v", "w") else np.abs(s1[c]).max()
+        err = np.abs(getattr(g, c).cpu().numpy() - s1[c]).max() / scale
+        assert err < 1e-12, (c, err)
+    g.destroy()
+
+
+@pytest.mark.parametrize("shape,periodic,bc", [
+    ((20, 64, 37), (False, True, False), ((0, 0), (0, 0), (1, -1))),
+    ((129, 16, 40), (False, False, True), ((1, 1), (-1, 0), (0, 0)))])
+@pytest.mark.parametrize("inviscid", [True, False])
+def test_batched_rhs_matches_oracle(shape, periodic, bc, inviscid):
+    """Bounded axes with mixed closures (the fields of a batch then differ in
+    their tables), one of them without a partitioned kernel (x = 20)."""
+    s0, h = _state(shape, sum(shape))
+    h = tuple(1.0 / (n - 1) if not p else hh for n, p, hh in zip(shape, periodic, h))
+    kw = dict(gam=1.4, Rgas=1.0, inviscid=inviscid, mu_ref=0.01, T_ref=1.0, visc_n=0.75, Pr=0.7, periodic=periodic, bc=bc)
+    og = cg.Grid(shape, h, **kw)
+    s = og.from_p(dict(s0))
+    ref = og.rhs(og.conserved(s), s)
+    g = gcg.cgrid(*shape, *h, **kw)
+    for c in ("rho", "u", "v", "w", "p"):
+        getattr(g, c).copy_(torch.tensor(s0[c], device=DEV))
+    g.post_bc()
+    g.get_conserved()
+    rhs = po.fortran_empty((*shape, 5), device=DEV)
+    print(f"batched rhs {shape} inviscid {inviscid}", flush=True)
+    g.getRHS(rhs)
+    got = rhs.cpu().numpy()
+    for k in range(5):
+        assert rel(got[..., k], ref[..., k]) < 1e-12, k
+    g.destroy()
