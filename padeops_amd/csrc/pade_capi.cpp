@@ -15,6 +15,7 @@
 
 #include "../../include/padeops_hip.h"
 #include "pade_capi_internal.h"
+#include "pade_cgrid.h"
 #include "pade_dense.h"
 #include "pade_err.h"
 #include "pade_kernels.h"
@@ -1189,10 +1190,21 @@ int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, 
 
 namespace pade {
 
-int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *flds, int na, int nb, int times, bool acc,
-                 double alpha, double beta, double *tmp, hipStream_t s)
+// The stage of apply_fields as a pass of its own.
+static int run_stage(pade_op_t op, int nf, const BatchField *flds, int na, int nb, const Stage *stage, hipStream_t s)
 {
-    if (nf < 1 || nf > kMaxFields || times < 1 || times > 2) return fail(400, "bad batch");
+    for (int k = 0; stage && k < nf; k++)
+        if (int rc = cg_rk_stage((long long)na * nb * op->n, stage->dt, stage->A, stage->B, flds[k].out, flds[k].Q,
+                                 flds[k].W, s))
+            return rc;
+    return 0;
+}
+
+int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *flds, int na, int nb, int times, bool acc,
+                 double alpha, double beta, double *tmp, hipStream_t s, const Stage *stage)
+{
+    if (nf < 1 || nf > kMaxFields || times < 1 || times > 2 || (stage && (!acc || times != 1)))
+        return fail(400, "bad batch");
     for (int k = 0; k < nf; k++) {
         if (int rc = check_apply(op, oper, axis, na, nb, flds[k].bc1, flds[k].bcn, false)) return rc;
         if (!flds[k].f || !flds[k].out) return fail(400, "null array");
@@ -1220,10 +1232,22 @@ int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *fld
             L.a.beta = beta;
             const int gw = L.pw == 8 ? whole_pencil_waves() : 1;
             hipError_t e;
+            if (stage && L.mode == 0 && L.pw == 2) {
+                for (int k = 0; k < nf; k++) {
+                    L.a.fld[k].stage_q = flds[k].Q;
+                    L.a.fld[k].stage_w = flds[k].W;
+                }
+                L.a.stage_dt = stage->dt;
+                L.a.stage_a = stage->A;
+                L.a.stage_b = stage->B;
+                e = launch_stage(L.a, L.v->M, L.v->uneven, s);
+                return e == hipSuccess ? 0 : hip_fail(e, "spike_apply launch");
+            }
             if (times == 2) e = launch_twice(L.a, L.v->M, L.pw, gw, L.v->uneven, false, L.mode, s);
             else if (L.v->uneven) e = launch_uneven<double>(L.a, L.v->M, false, L.mode, s);
             else e = launch_spike<double>(L.a, L.v->M, L.pw, gw, false, L.mode, s);
-            return e == hipSuccess ? 0 : hip_fail(e, "spike_apply launch");
+            if (e != hipSuccess) return hip_fail(e, "spike_apply launch");
+            return run_stage(op, nf, flds, na, nb, stage, s);
         }
     }
     for (int k = 0; k < nf; k++) {
@@ -1243,7 +1267,7 @@ int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *fld
                                         epi, Workspace()))
             return rc;
     }
-    return 0;
+    return run_stage(op, nf, flds, na, nb, stage, s);
 }
 
 bool apply_in_place_ok(pade_op_t op, int oper, int axis, int na, int nb, int bc1, int bcn)

@@ -24,12 +24,20 @@ bool apply_in_place_ok(pade_op_t op, int oper, int axis, int na, int nb, int bc1
 // intermediate in registers; else one apply per field and repetition, with
 // `tmp` (a field, needed for times = 2) as the intermediate.  Outputs must
 // not overlap any input of the call.
+//
+// A stage (Runge-Kutta, low storage) may end an accumulating apply: with r =
+// alpha op(f) + beta out, Q = dt r + A Q and W += B Q for every field; `out`
+// then holds r or its old values, as the kernels serve it.
 struct BatchField {
     const double *f;
     double *out;
     int bc1, bcn;
+    double *Q = nullptr, *W = nullptr;   // of the stage
+};
+struct Stage {
+    double dt, A, B;
 };
 int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *flds, int na, int nb, int times, bool acc,
-                 double alpha, double beta, double *tmp, hipStream_t s);
+                 double alpha, double beta, double *tmp, hipStream_t s, const Stage *stage = nullptr);
 
 }  // namespace pade

@@ -29,14 +29,23 @@ int cg_dt_maxima(long long n, const double *rho, const double *u, const double *
 
 // The three artificial properties before filtering (cgrid.F90:1083-1199) in
 // one pass: fl holds grad(rho), grad(e) and the fourth derivatives of the
-// strain magnitude, the dilatation and e (three planes each, in this order),
-// du the velocity gradients; dil holds the dilatation on entry and the
-// conductivity on return.
+// strain magnitude, the dilatation and e (three planes each, in this order);
+// mustar holds the bulk viscosity's switch on entry.
 int cg_lad(long long n, double Cmu, double Cbeta, double Ckap, double gam, const double *h, const double *rho,
-           const double *p, const double *T, const double *fl, const double *du, double *mustar, double *bulkstar,
-           double *dil, hipStream_t s);
+           const double *p, const double *T, const double *fl, double *mustar, double *bulkstar, double *kapstar,
+           hipStream_t s);
 
-// The first RK45 stage (A = 0): Q = dt rhs, W += B Q.
-int cg_rk_first(long long n, double dt, double B, const double *rhs, double *Q, double *W, hipStream_t s);
+// An RK45 stage of n values: Q = dt rhs + A Q, W += B Q.
+int cg_rk_stage(long long n, double dt, double A, double B, const double *rhs, double *Q, double *W, hipStream_t s);
+
+// The magnitude of the strain rate, the dilatation and the bulk viscosity's
+// switch (cgrid.F90:1085-1087, :1140-1155) from the velocity gradients.
+int cg_strain_switch(long long n, const double *du, double *func, double *dil, double *fsw, hipStream_t s);
+
+// get_primitive and post_bc, then get_conserved of the result (the state
+// between two substeps when nothing comes between them), with pade_cg_conserved's
+// test of W.
+int cg_primitive_conserved(long long n, double *W, double gam, double Rgas, double *rho, double *u, double *v,
+                           double *w, double *e, double *p, double *T, unsigned long long *bad_index, hipStream_t s);
 
 }  // namespace pade

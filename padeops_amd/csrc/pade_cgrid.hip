@@ -89,6 +89,46 @@ __global__ __launch_bounds__(kBlock) void k_primitive(long long n, const double 
     }
 }
 
+// k_primitive, then k_conserved of its result, in one pass (5 fields read
+// instead of 10).
+__global__ __launch_bounds__(kBlock) void k_primitive_conserved(long long n, double *W, double gam, double Rgas,
+                                                                double *__restrict__ rho, double *__restrict__ u,
+                                                                double *__restrict__ v, double *__restrict__ w,
+                                                                double *__restrict__ e, double *__restrict__ p,
+                                                                double *__restrict__ T,
+                                                                unsigned long long *__restrict__ bad_index)
+{
+    unsigned long long first = ~0ull;
+    GRID_STRIDE(i, n)
+    {
+        const double r = W[i];
+        const double onebyrho = 1.0 / r;
+        const double uu = W[n + i] * onebyrho, vv = W[2 * n + i] * onebyrho, ww = W[3 * n + i] * onebyrho;
+        const double ee = W[4 * n + i] * onebyrho - 0.5 * (uu * uu + vv * vv + ww * ww);
+        const double pp = (gam - 1.0) * r * ee;
+        const double e2 = pp / (gam - 1.0) / r;
+        rho[i] = r;
+        u[i] = uu;
+        v[i] = vv;
+        w[i] = ww;
+        p[i] = pp;
+        e[i] = e2;
+        T[i] = e2 * ((gam - 1.0) / Rgas);
+        const double w1 = r * uu, w2 = r * vv, w3 = r * ww;
+        const double w4 = r * (e2 + 0.5 * (uu * uu + vv * vv + ww * ww));
+        W[n + i] = w1;
+        W[2 * n + i] = w2;
+        W[3 * n + i] = w3;
+        W[4 * n + i] = w4;
+        if (bad_value(r) | bad_value(w1) | bad_value(w2) | bad_value(w3) | bad_value(w4)) {
+            const int l = bad_value(r) ? 0 : bad_value(w1) ? 1 : bad_value(w2) ? 2 : bad_value(w3) ? 3 : 4;
+            const unsigned long long idx = (unsigned long long)(l * n + i);
+            first = idx < first ? idx : first;
+        }
+    }
+    if (first != ~0ull) atomicMin(bad_index, first);
+}
+
 // LAD shear-viscosity sensor: magnitude of the strain rate (cgrid.F90:1085-1087);
 // du planes: du/dx du/dy du/dz dv/dx ... dw/dz
 __global__ __launch_bounds__(kBlock) void k_strain(long long n, const double *__restrict__ du,
@@ -160,19 +200,41 @@ __global__ __launch_bounds__(kBlock) void k_lad_kap(long long n, double Ckap, do
     }
 }
 
-// k_lad_mu, k_lad_bulk and k_lad_kap in one pass: 27 fields read and 3
+// k_strain with the bulk viscosity's switch, which reads the same velocity
+// gradients: one plane written here instead of seven read by k_lad.
+__global__ __launch_bounds__(kBlock) void k_strain_switch(long long n, const double *__restrict__ du,
+                                                          double *__restrict__ func, double *__restrict__ dil,
+                                                          double *__restrict__ fsw)
+{
+    GRID_STRIDE(i, n)
+    {
+        const double ux = du[i], uy = du[n + i], uz = du[2 * n + i];
+        const double vx = du[3 * n + i], vy = du[4 * n + i], vz = du[5 * n + i];
+        const double wx = du[6 * n + i], wy = du[7 * n + i], wz = du[8 * n + i];
+        func[i] = sqrt(ux * ux + 0.5 * (vx + uy) * (vx + uy) + 0.5 * (wx + uz) * (wx + uz) + vy * vy +
+                       0.5 * (wy + vz) * (wy + vz) + wz * wz);
+        const double f = ux + vy + wz;
+        dil[i] = f;
+        const double c1 = wy - vz, c2 = uz - wx, c3 = vx - uy;
+        const double curl2 = c1 * c1 + c2 * c2 + c3 * c3;
+        const double d2 = f * f;
+        fsw[i] = f >= 0.0 ? 0.0 : d2 / (d2 + curl2 + 1.0e-32);
+    }
+}
+
+// k_lad_mu, k_lad_bulk and k_lad_kap in one pass: 19 fields read and 3
 // written instead of 33 and 3 (and no accumulating passes for mustar).
 __global__ __launch_bounds__(kBlock) void k_lad(long long n, double Cmu, double Cbeta, double Ckap, double gam,
                                                 double hx, double hy, double hz, const double *__restrict__ rho,
                                                 const double *__restrict__ p, const double *__restrict__ T,
-                                                const double *__restrict__ fl, const double *__restrict__ du,
-                                                double *__restrict__ mustar, double *__restrict__ bulkstar, double *dil)
+                                                const double *__restrict__ fl, double *mustar,
+                                                double *__restrict__ bulkstar, double *__restrict__ kapstar)
 {
     const double hx4 = hx * hx * hx * hx, hy4 = hy * hy * hy * hy, hz4 = hz * hz * hz * hz;
     const double hx6 = hx4 * hx * hx, hy6 = hy4 * hy * hy, hz6 = hz4 * hz * hz;
     GRID_STRIDE(i, n)
     {
-        const double r = rho[i];
+        const double r = rho[i], fsw = mustar[i];
         double m = hx6 * fl[6 * n + i];
         m = m + hz6 * fl[8 * n + i];
         m = m + hy6 * fl[7 * n + i];
@@ -183,13 +245,6 @@ __global__ __launch_bounds__(kBlock) void k_lad(long long n, double Cmu, double 
         double b = fl[9 * n + i] * hx4 * (ax * ax);
         b = b + fl[11 * n + i] * hz4 * (az * az);
         b = b + fl[10 * n + i] * hy4 * (ay * ay);
-        const double uy = du[n + i], uz = du[2 * n + i], vx = du[3 * n + i], vz = du[5 * n + i];
-        const double wx = du[6 * n + i], wy = du[7 * n + i];
-        const double c1 = wy - vz, c2 = uz - wx, c3 = vx - uy;
-        const double curl2 = c1 * c1 + c2 * c2 + c3 * c3;
-        const double f = dil[i];
-        const double d2 = f * f;
-        const double fsw = f >= 0.0 ? 0.0 : d2 / (d2 + curl2 + 1.0e-32);
         bulkstar[i] = Cbeta * r * fsw * fabs(b);
         g1 = fl[3 * n + i] * fl[3 * n + i];
         g2 = fl[4 * n + i] * fl[4 * n + i];
@@ -199,7 +254,7 @@ __global__ __launch_bounds__(kBlock) void k_lad(long long n, double Cmu, double 
         k = k + fl[14 * n + i] * hz4 * (hz * g3 / den);
         k = k + fl[13 * n + i] * hy4 * (hy * g2 / den);
         const double sos = sqrt(gam * p[i] / r);
-        dil[i] = Ckap * r * sos * fabs(k) / T[i];
+        kapstar[i] = Ckap * r * sos * fabs(k) / T[i];
     }
 }
 
@@ -256,18 +311,6 @@ __global__ __launch_bounds__(kBlock) void k_rk(long long n5, double dt, double A
     GRID_STRIDE(i, n5)
     {
         const double q = dt * rhs[i] + A * Q[i];
-        Q[i] = q;
-        W[i] = W[i] + B * q;
-    }
-}
-
-// its first stage, A = 0
-__global__ __launch_bounds__(kBlock) void k_rk_first(long long n5, double dt, double B, const double *__restrict__ rhs,
-                                                     double *__restrict__ Q, double *__restrict__ W)
-{
-    GRID_STRIDE(i, n5)
-    {
-        const double q = dt * rhs[i];
         Q[i] = q;
         W[i] = W[i] + B * q;
     }
@@ -378,20 +421,36 @@ int cg_fill(double *x, long long n, double v, hipStream_t s)
 }
 
 int cg_lad(long long n, double Cmu, double Cbeta, double Ckap, double gam, const double *h, const double *rho,
-           const double *p, const double *T, const double *fl, const double *du, double *mustar, double *bulkstar,
-           double *dil, hipStream_t s)
+           const double *p, const double *T, const double *fl, double *mustar, double *bulkstar, double *kapstar,
+           hipStream_t s)
 {
     (void)hipGetLastError();
     hipLaunchKernelGGL(k_lad, dim3(grid_for(n)), dim3(kBlock), 0, s, n, Cmu, Cbeta, Ckap, gam, h[0], h[1], h[2], rho, p,
-                       T, fl, du, mustar, bulkstar, dil);
+                       T, fl, mustar, bulkstar, kapstar);
     return launched("artificial-property launch");
 }
 
-int cg_rk_first(long long n, double dt, double B, const double *rhs, double *Q, double *W, hipStream_t s)
+int cg_strain_switch(long long n, const double *du, double *func, double *dil, double *fsw, hipStream_t s)
 {
     (void)hipGetLastError();
-    hipLaunchKernelGGL(k_rk_first, dim3(grid_for(5 * n)), dim3(kBlock), 0, s, 5 * n, dt, B, rhs, Q, W);
-    return launched("first RK stage launch");
+    hipLaunchKernelGGL(k_strain_switch, dim3(grid_for(n)), dim3(kBlock), 0, s, n, du, func, dil, fsw);
+    return launched("strain launch");
+}
+
+int cg_rk_stage(long long n, double dt, double A, double B, const double *rhs, double *Q, double *W, hipStream_t s)
+{
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_rk, dim3(grid_for(n)), dim3(kBlock), 0, s, n, dt, A, B, rhs, Q, W);
+    return launched("RK stage launch");
+}
+
+int cg_primitive_conserved(long long n, double *W, double gam, double Rgas, double *rho, double *u, double *v,
+                           double *w, double *e, double *p, double *T, unsigned long long *bad_index, hipStream_t s)
+{
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_primitive_conserved, dim3(grid_for(n)), dim3(kBlock), 0, s, n, W, gam, Rgas, rho, u, v, w, e,
+                       p, T, bad_index);
+    return launched("state update launch");
 }
 
 int cg_transport(long long n, const double *T, double mu_ref, double T_ref, double visc_n, double cp_by_pr,

@@ -74,6 +74,7 @@ struct Item {
     const double *f;
     double *out;
     int sign;
+    double *Q = nullptr, *W = nullptr;   // of a Runge-Kutta stage
 };
 
 // One operator along `axis` (0, 1, 2) of several (nx, ny, nz) fields, in one
@@ -81,7 +82,7 @@ struct Item {
 // op^times(f) + out.
 template <int N>
 int apply(pade_cgrid_t g, pade_op_t op, int oper, int axis, const Item (&items)[N], int times, bool acc, double alpha,
-          hipStream_t s)
+          hipStream_t s, const pade::Stage *stage = nullptr)
 {
     int na, nb;
     if (axis == 0) { na = g->n[1]; nb = g->n[2]; }
@@ -89,8 +90,9 @@ int apply(pade_cgrid_t g, pade_op_t op, int oper, int axis, const Item (&items)[
     else { na = g->n[0]; nb = g->n[1]; }
     pade::BatchField b[N];
     for (int k = 0; k < N; k++)
-        b[k] = {items[k].f, items[k].out, items[k].sign * g->bc[axis][0], items[k].sign * g->bc[axis][1]};
-    return pade::apply_fields(op, oper, axis + 1, N, b, na, nb, times, acc, alpha, 1.0, g->t1, s);
+        b[k] = {items[k].f, items[k].out, items[k].sign * g->bc[axis][0], items[k].sign * g->bc[axis][1], items[k].Q,
+                items[k].W};
+    return pade::apply_fields(op, oper, axis + 1, N, b, na, nb, times, acc, alpha, 1.0, g->t1, s, stage);
 }
 
 // cgrid.F90:1259-1336: y, then x, then z, each `times` times, of the N planes
@@ -140,8 +142,13 @@ int transport(pade_cgrid_t g, hipStream_t s)
 // e (12-14), planes x, y, z each.  Bound by memory from 128^3 up; below, by
 // the launch and latency of each pass.  Per step, 256^3 and 96 x 80 x 65
 // (walls in z): one launch per field and pass 39.0 and 4.0 ms, batched and
-// fused 32.4 and 1.72 ms.
-int rhs_impl(pade_cgrid_t g, double *rhs, hipStream_t s)
+// fused 32.4 and 1.72 ms, with the stage in the last flux derivative, the
+// bulk switch beside the strain and one pass for the state update 31.1 and
+// 1.68 ms.
+//
+// With a stage the last flux derivative also advances Q and W (rhs then holds
+// an unfinished sum).
+int rhs_impl(pade_cgrid_t g, double *rhs, hipStream_t s, const pade::Stage *stage = nullptr)
 {
     const long long N = g->N;
     int rc = 0;
@@ -156,7 +163,7 @@ int rhs_impl(pade_cgrid_t g, double *rhs, hipStream_t s)
     }
     // an inviscid grid's properties are the artificial ones alone, written below
     if (!rc && !g->inviscid) rc = transport(g, s);
-    if (!rc) rc = pade_cg_strain(N, g->du, g->func, g->dil, s);
+    if (!rc) rc = pade::cg_strain_switch(N, g->du, g->func, g->dil, g->mustar, s);
     if (!rc && g->der_kind == PADE_CD06) return err(21, "CD06 is incomplete right now");   // derivatives.F90:524-525
     for (int a : {0, 2, 1}) {
         const Item d4[3] = {{g->func, g->fl + (6 + a) * N, 1},
@@ -166,7 +173,7 @@ int rhs_impl(pade_cgrid_t g, double *rhs, hipStream_t s)
     }
     if (!rc)
         rc = pade::cg_lad(N, g->Cmu, g->Cbeta, g->Ckap, g->gam, g->h, F(g, PADE_CG_RHO), F(g, PADE_CG_P),
-                          F(g, PADE_CG_T), g->fl, g->du, g->mustar, g->func, g->dil, s);
+                          F(g, PADE_CG_T), g->fl, g->mustar, g->func, g->dil, s);
     if (!rc) {                                                                       // (:1113, :1161, :1199, :1252-1254)
         const double *const stars[3] = {g->mustar, g->func, g->dil};
         double *const props[3] = {F(g, PADE_CG_MU), F(g, PADE_CG_BULK), F(g, PADE_CG_KAP)};
@@ -182,8 +189,9 @@ int rhs_impl(pade_cgrid_t g, double *rhs, hipStream_t s)
     // the walls except the momentum flux along the derivative's own axis
     for (int a : {0, 1, 2}) {
         Item fx[5];
-        for (int k = 0; k < 5; k++) fx[k] = {g->fl + (5LL * a + k) * N, rhs + k * N, k == 1 + a ? 1 : -1};
-        if (!rc) rc = apply(g, g->der[a], PADE_D1, a, fx, 1, a != 0, a == 0 ? 1.0 : -1.0, s);
+        for (int k = 0; k < 5; k++)
+            fx[k] = {g->fl + (5LL * a + k) * N, rhs + k * N, k == 1 + a ? 1 : -1, g->Q + k * N, Wp(g, k)};
+        if (!rc) rc = apply(g, g->der[a], PADE_D1, a, fx, 1, a != 0, a == 0 ? 1.0 : -1.0, s, a == 2 ? stage : nullptr);
     }
     return rc;
 }
@@ -195,20 +203,30 @@ int post_bc_impl(pade_cgrid_t g, hipStream_t s)
                             F(g, PADE_CG_T), s);
 }
 
-int conserved_impl(pade_cgrid_t g, bool check, long long *bad, hipStream_t s)
+// The word that the kernels lower to the first bad index of W: all ones
+// before, read back after them.
+int reset_bad(pade_cgrid_t g, hipStream_t s)
 {
-    if (check) {
-        hipError_t e = hipMemsetAsync(g->dscal, 0xff, sizeof(unsigned long long), s);
-        if (e != hipSuccess) return err(1000 + int(e), "bad-index reset");
-    }
-    int rc = pade_cg_conserved(g->N, F(g, PADE_CG_RHO), F(g, PADE_CG_U), F(g, PADE_CG_V), F(g, PADE_CG_W_VEL),
-                               F(g, PADE_CG_E), F(g, PADE_CG_W), check ? g->dscal : nullptr, s);
-    if (rc || !check) return rc;
+    hipError_t e = hipMemsetAsync(g->dscal, 0xff, sizeof(unsigned long long), s);
+    return e == hipSuccess ? 0 : err(1000 + int(e), "bad-index reset");
+}
+
+int read_bad(pade_cgrid_t g, long long *bad, hipStream_t s)
+{
     hipError_t e = hipMemcpyAsync(g->hscal, g->dscal, sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return err(1000 + int(e), "bad-index read");
     *bad = g->hscal[0] == ~0ull ? -1 : (long long)g->hscal[0];
     return 0;
+}
+
+int conserved_impl(pade_cgrid_t g, bool check, long long *bad, hipStream_t s)
+{
+    if (check)
+        if (int rc = reset_bad(g, s)) return rc;
+    int rc = pade_cg_conserved(g->N, F(g, PADE_CG_RHO), F(g, PADE_CG_U), F(g, PADE_CG_V), F(g, PADE_CG_W_VEL),
+                               F(g, PADE_CG_E), F(g, PADE_CG_W), check ? g->dscal : nullptr, s);
+    return rc || !check ? rc : read_bad(g, bad, s);
 }
 
 void release(pade_cgrid_t g)
@@ -412,10 +430,13 @@ int pade_cgrid_advance_rk45(pade_cgrid_t g, double dt, pade_cgrid_hook hook_bc, 
     if (dt > 0.0) g->dt = dt;
     int rc = 0;
     if (g->step == 0) rc = post_bc_impl(g, s);         // get_e_from_p, get_T (:675-679)
+    if (!rc) rc = pade::cg_fill(g->Q, 5 * g->N, 0.0, s);
     double Qt = 0.0;
     for (int isub = 0; isub < 5 && !rc; isub++) {
         long long bad = -1;
-        rc = conserved_impl(g, true, &bad, s);
+        // (without a hook the state update of the substep before formed W and
+        // its test already)
+        rc = isub == 0 || hook_bc ? conserved_impl(g, true, &bad, s) : read_bad(g, &bad, s);
         if (rc) break;
         if (bad >= 0) {                                  // nancheck, :684-692
             if (bad_substep) *bad_substep = isub + 1;
@@ -427,11 +448,8 @@ int pade_cgrid_advance_rk45(pade_cgrid_t g, double dt, pade_cgrid_hook hook_bc, 
                                 std::to_string(j + 1) + "," + std::to_string(k + 1) + "," + std::to_string(l + 1) +
                                 ")");
         }
-        rc = rhs_impl(g, g->rhs, s);
-        if (!rc && isub == 0)          // A(1) = 0: Qtmp starts here
-            rc = pade::cg_rk_first(g->N, g->dt, kRkB[0], g->rhs, g->Q, F(g, PADE_CG_W), s);
-        else if (!rc)
-            rc = pade_cg_rk_stage(g->N, g->dt, kRkA[isub], kRkB[isub], g->rhs, g->Q, F(g, PADE_CG_W), s);
+        const pade::Stage stage = {g->dt, kRkA[isub], kRkB[isub]};
+        rc = rhs_impl(g, g->rhs, s, &stage);
         Qt = g->dt + kRkA[isub] * Qt;
         g->tsim += kRkB[isub] * Qt;
         // the momentum component along an axis is odd at its walls (:701-706)
@@ -439,7 +457,15 @@ int pade_cgrid_advance_rk45(pade_cgrid_t g, double dt, pade_cgrid_hook hook_bc, 
         double *const W[5] = {Wp(g, 0), Wp(g, 1), Wp(g, 2), Wp(g, 3), Wp(g, 4)};
         const double *const Wc[5] = {W[0], W[1], W[2], W[3], W[4]};
         if (!rc) rc = filter(g, Wc, W, flips, g->fil, 1, false, s);
-        if (!rc) rc = pade_cgrid_get_primitive(g, stream);
+        if (!rc && !hook_bc && isub < 4) {
+            rc = reset_bad(g, s);
+            if (!rc)
+                rc = pade::cg_primitive_conserved(g->N, F(g, PADE_CG_W), g->gam, g->Rgas, F(g, PADE_CG_RHO),
+                                                  F(g, PADE_CG_U), F(g, PADE_CG_V), F(g, PADE_CG_W_VEL),
+                                                  F(g, PADE_CG_E), F(g, PADE_CG_P), F(g, PADE_CG_T), g->dscal, s);
+        } else if (!rc) {
+            rc = pade_cgrid_get_primitive(g, stream);
+        }
         if (!rc && hook_bc) {
             hook_bc(g, user);
             rc = post_bc_impl(g, s);

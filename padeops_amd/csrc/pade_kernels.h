@@ -49,6 +49,7 @@ struct FieldArgs {
     int coef_len;          // length of the coefficient area
     int ncls;              // number of coefficient blocks
     int kq;                // reduced-system window: partitions p-kq..p+kq (2kq+1 >= P: all)
+    T *stage_q, *stage_w;  // Runge-Kutta stage epilogue: register and state
 };
 
 constexpr int kMaxFields = 6;
@@ -73,6 +74,7 @@ struct ApplyArgs {
                            // (workgroup i runs on XCD i % 8) takes runs of C
                            // consecutive workgroups; < 0 a contiguous eighth
     T alpha, beta;
+    T stage_dt, stage_a, stage_b;
     // last, so that a launch of one field reads one stretch of arguments
     FieldArgs<T> fld[kMaxFields];
 };
@@ -92,6 +94,11 @@ hipError_t launch_uneven(const ApplyArgs<T> &a, int M, bool adj, int mode, hipSt
 // and 1, two partitions per wave or whole-pencil x waves (FP64).
 hipError_t launch_twice(const ApplyArgs<double> &a, int M, int PW, int GW, bool uneven, bool adj, int mode,
                         hipStream_t s);
+
+// The accumulating apply along z finished by a Runge-Kutta stage: r = alpha
+// op(f) + beta out (not written), Q = stage_dt r + stage_a Q, W += stage_b Q.
+// Mode 0, two partitions per wave.
+hipError_t launch_stage(const ApplyArgs<double> &a, int M, bool uneven, hipStream_t s);
 
 template <typename T>
 hipError_t launch_generic(const ApplyArgs<T> &a, bool adj, T *work, hipStream_t s);

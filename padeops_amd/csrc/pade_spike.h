@@ -169,6 +169,8 @@ constexpr int kHaloChunk = 8;
 // overlap so that every 32-byte sector is stored whole by one workgroup:
 // 242 / 208.)
 enum RowLayout { kWholeLines = 0, kHalfLines = 1, kShared = 2 };
+// Epilogue: store op(f); alpha op(f) + beta out; a Runge-Kutta stage on that.
+enum Epi { kStore = 0, kAxpby = 1, kStage = 2 };
 // rows every partition has (UnevenParts keeps to it)
 constexpr int kMinRows = 8;
 // 16-byte lanes: VL elements per lane, XT / VL lanes per tile row; tile rows
@@ -257,7 +259,7 @@ __device__ __forceinline__ void apply_stencil(T (&w)[M + 8], const T *__restrict
     }
 }
 
-template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, bool EPI, bool UNE = false, int ROWS = kWholeLines,
+template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, int EPI, bool UNE = false, int ROWS = kWholeLines,
           int REP = 1>
 __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
 {
@@ -751,7 +753,41 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     if constexpr (MODE != 1) {
         const unsigned hoff = loff + (unsigned)((long long)(UNE ? pM - pw0 : half * M) * stp * (long long)sizeof(T));
         if (valid) {
-            if constexpr (EPI) {
+            if constexpr (EPI == kStage) {
+                // low-storage Runge-Kutta stage on the finished right-hand
+                // side r = alpha op(f) + beta out: Q = dt r + A Q, W += B Q
+                // (r itself is not written), in batches as below
+                constexpr int KB = kEpiRows / 2;
+                const long long qd = fd.stage_q - fd.out, wd = fd.stage_w - fd.out;
+                T cur[3][KB], nxt[3][KB];
+                auto load = [&](T (&o)[3][KB], int t0) {
+#pragma unroll
+                    for (int k = 0; k < KB; k++) {
+                        T *row = ob + (long long)(pw0 + t0 + k) * stp;
+                        o[0][k] = ld_s<ROWS == kWholeLines>(row, hoff);
+                        o[1][k] = ld_s<ROWS == kWholeLines>(row + qd, hoff);
+                        o[2][k] = ld_s<ROWS == kWholeLines>(row + wd, hoff);
+                    }
+                };
+                load(cur, 0);
+#pragma unroll
+                for (int t0 = 0; t0 < M; t0 += KB) {
+                    if (t0 + KB < M) load(nxt, t0 + KB);
+#pragma unroll
+                    for (int k = 0; k < KB; k++)
+                        if (!UNE || t0 + k < mrows) {
+                            T *row = ob + (long long)(pw0 + t0 + k) * stp;
+                            const T r = a.alpha * w[t0 + k] + a.beta * cur[0][k];
+                            const T q = a.stage_dt * r + a.stage_a * cur[1][k];
+                            put(row + qd, hoff, q);
+                            put(row + wd, hoff, cur[2][k] + a.stage_b * q);
+                        }
+#pragma unroll
+                    for (int k = 0; k < KB; k++)
+#pragma unroll
+                        for (int j = 0; j < 3; j++) cur[j][k] = nxt[j][k];
+                }
+            } else if constexpr (EPI) {
                 // Old values are loaded in batches of rows, the next batch
                 // before the current one is stored: the compiler cannot show
                 // that the store of row t and the load of row t + 1 touch
@@ -909,7 +945,8 @@ uintptr_t field_bits(const ApplyArgs<T> &a)
 {
     uintptr_t bits = 0;
     for (int k = 0; k < a.nfields; k++)
-        bits |= reinterpret_cast<uintptr_t>(a.fld[k].f) | reinterpret_cast<uintptr_t>(a.fld[k].out);
+        bits |= reinterpret_cast<uintptr_t>(a.fld[k].f) | reinterpret_cast<uintptr_t>(a.fld[k].out) |
+                reinterpret_cast<uintptr_t>(a.fld[k].stage_q) | reinterpret_cast<uintptr_t>(a.fld[k].stage_w);
     return bits;
 }
 
@@ -924,7 +961,7 @@ RowLayout row_layout(const ApplyArgs<T> &a)
 // Workgroups per XCD run where neighbouring workgroups share lines.
 constexpr int kSharedRun = 64;
 
-template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, bool EPI, bool UNE, int REP>
+template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, int EPI, bool UNE, int REP>
 hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
 {
     constexpr int NPEN = 64 / PW;
@@ -982,18 +1019,18 @@ hipError_t launch_spike_t(const ApplyArgs<T> &a, int gw, hipStream_t s)
     if constexpr (MODE == 2) {
         // staggered operators: forward, bounded, strided rows only
         if (ADJ || a.periodic || a.n_in < a.n || a.n_in > a.n + 1) return hipErrorInvalidValue;
-        return epi ? launch_kernel<T, M, PW, false, 2, true, true, UNE, REP>(a, gw, s)
-                   : launch_kernel<T, M, PW, false, 2, true, false, UNE, REP>(a, gw, s);
+        return epi ? launch_kernel<T, M, PW, false, 2, true, kAxpby, UNE, REP>(a, gw, s)
+                   : launch_kernel<T, M, PW, false, 2, true, kStore, UNE, REP>(a, gw, s);
     } else if constexpr (ADJ) {
         // (a periodic adjoint runs the forward kernel on the transposed tables)
         if (a.periodic) return hipErrorInvalidValue;
-        return launch_kernel<T, M, PW, true, MODE, true, false, UNE, REP>(a, gw, s);
+        return launch_kernel<T, M, PW, true, MODE, true, kStore, UNE, REP>(a, gw, s);
     } else {
         if (a.periodic)
-            return epi ? launch_kernel<T, M, PW, false, MODE, false, true, UNE, REP>(a, gw, s)
-                       : launch_kernel<T, M, PW, false, MODE, false, false, UNE, REP>(a, gw, s);
-        return epi ? launch_kernel<T, M, PW, false, MODE, true, true, UNE, REP>(a, gw, s)
-                   : launch_kernel<T, M, PW, false, MODE, true, false, UNE, REP>(a, gw, s);
+            return epi ? launch_kernel<T, M, PW, false, MODE, false, kAxpby, UNE, REP>(a, gw, s)
+                       : launch_kernel<T, M, PW, false, MODE, false, kStore, UNE, REP>(a, gw, s);
+        return epi ? launch_kernel<T, M, PW, false, MODE, true, kAxpby, UNE, REP>(a, gw, s)
+                   : launch_kernel<T, M, PW, false, MODE, true, kStore, UNE, REP>(a, gw, s);
     }
 }
 
