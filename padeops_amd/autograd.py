@@ -17,14 +17,14 @@ import torch
 import torch.utils.checkpoint
 
 from ._lib import PADE_D1, PADE_D2, PADE_FILTER
-from .operators import fortran_empty
+from .operators import _is_dense_block, fortran_empty
 
 __all__ = ["compact_apply", "ddx", "ddy", "ddz", "d2dx2", "d2dy2", "d2dz2", "filterx", "filtery", "filterz",
            "checkpointed_steps"]
 
 
 def _fortran(t):
-    if t.dim() == 3 and t.permute(2, 1, 0).is_contiguous():
+    if t.dim() == 3 and _is_dense_block(t):
         return t
     out = fortran_empty(tuple(t.shape), dtype=t.dtype, device=t.device)
     out.copy_(t)

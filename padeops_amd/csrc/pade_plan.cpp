@@ -869,13 +869,19 @@ int dense_operator(const OpMatrices &op, std::vector<double> &D)
     }
     if (int rc = invert(A, n)) return rc;
     D.assign((size_t)n * n, 0.0);
+    // the entries of B's rows, a stencil each
+    std::vector<int> first(n + 1, 0), col;
+    for (int k = 0; k < n; k++) {
+        for (int j = 0; j < n; j++)
+            if (B[(size_t)k * n + j] != 0.0) col.push_back(j);
+        first[k + 1] = (int)col.size();
+    }
     for (int i = 0; i < n; i++)
         for (int k = 0; k < n; k++) {
             const double a = A[(size_t)i * n + k];
-            if (a == 0.0) continue;
             const double *b = &B[(size_t)k * n];
             double *d = &D[(size_t)i * n];
-            for (int j = 0; j < n; j++) d[j] += a * b[j];
+            for (int q = first[k]; q < first[k + 1]; q++) d[col[q]] += a * b[col[q]];
         }
     return 0;
 }

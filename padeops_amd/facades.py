@@ -20,9 +20,12 @@ methods and the least-squares filter are outside this library and raise
 from __future__ import annotations
 
 from ._lib import PadeError
-from .operators import cd06, cd10, cf90, gaussian
+from .operators import cd06, cd10, cf90, gaussian, torch
 
 _AXES = ("x", "y", "z")
+_INDEX = {"x": 0, "y": 1, "z": 2}
+_OTHERS = ((1, 2), (0, 2), (0, 1))          # the two other axes
+_DD, _D2D, _FILTER = (("dd1", "dd2", "dd3"), ("d2d1", "d2d2", "d2d3"), ("filter1", "filter2", "filter3"))
 
 
 def _sizes(args):
@@ -38,7 +41,10 @@ def _sizes(args):
 
 def _check_shape(arr, sz):
     count = sz[0] * sz[1] * sz[2]
-    size = arr.size if hasattr(arr, "size") and not callable(arr.size) else arr.numel()
+    if torch is not None and isinstance(arr, torch.Tensor):
+        size = arr.numel()
+    else:
+        size = arr.size if hasattr(arr, "size") and not callable(arr.size) else arr.numel()
     if size != count:
         raise ValueError(f"array of {size} values where the pencil layout {list(sz)} has {count}")
 
@@ -106,13 +112,12 @@ class derivatives:
         return self._method.get("z")
 
     def _d1(self, axis, f, df, bc1, bcn):
-        sz = {"x": self.xsz, "y": self.ysz, "z": self.zsz}[axis]
+        k = _INDEX[axis]
+        sz = (self.xsz, self.ysz, self.zsz)[k]
         _check_shape(f, sz)
         _check_shape(df, sz)
-        k = _AXES.index(axis)
-        na, nb = [s for i, s in enumerate(sz) if i != k]
-        op = self._ops[axis]
-        fn = getattr(op, f"dd{k + 1}")
+        na, nb = sz[_OTHERS[k][0]], sz[_OTHERS[k][1]]
+        fn = getattr(self._ops[axis], _DD[k])
         if self._method[axis] == "cd10" and bc1 is not None and bcn is not None:
             return fn(f, df, na, nb, bc1, bcn)          # derivatives.F90:455-458
         return fn(f, df, na, nb)
@@ -120,12 +125,12 @@ class derivatives:
     def _d2(self, axis, f, df, bc1, bcn):
         if self._method[axis] == "cd06":                 # derivatives.F90:524-525
             raise PadeError(21, "CD06 is incomplete right now")
-        sz = {"x": self.xsz, "y": self.ysz, "z": self.zsz}[axis]
+        k = _INDEX[axis]
+        sz = (self.xsz, self.ysz, self.zsz)[k]
         _check_shape(f, sz)
         _check_shape(df, sz)
-        k = _AXES.index(axis)
-        na, nb = [s for i, s in enumerate(sz) if i != k]
-        return getattr(self._ops[axis], f"d2d{k + 1}")(f, df, na, nb, bc1, bcn)
+        na, nb = sz[_OTHERS[k][0]], sz[_OTHERS[k][1]]
+        return getattr(self._ops[axis], _D2D[k])(f, df, na, nb, bc1, bcn)
 
     def ddx(self, f, dfdx, bc1=None, bcn=None):
         """derivatives.F90:447-468"""
@@ -210,12 +215,12 @@ class filters:
         return self._method.get("z")
 
     def _filter(self, axis, f, ff, bc1, bcn):
-        sz = {"x": self.xsz, "y": self.ysz, "z": self.zsz}[axis]
+        k = _INDEX[axis]
+        sz = (self.xsz, self.ysz, self.zsz)[k]
         _check_shape(f, sz)
         _check_shape(ff, sz)
-        k = _AXES.index(axis)
-        na, nb = [s for i, s in enumerate(sz) if i != k]
-        return getattr(self._ops[axis], f"filter{k + 1}")(f, ff, na, nb, bc1, bcn)
+        na, nb = sz[_OTHERS[k][0]], sz[_OTHERS[k][1]]
+        return getattr(self._ops[axis], _FILTER[k])(f, ff, na, nb, bc1, bcn)
 
     def filterx(self, f, ff, bc1=None, bcn=None):
         """filters.F90:220-235"""

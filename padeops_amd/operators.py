@@ -56,19 +56,27 @@ def _is_dense_block(t):
     """A flat (1-D) contiguous tensor, or an N-D tensor with Fortran strides.
     A C-ordered (n1, n2, n3) tensor is refused: its memory read as Fortran
     order would put the derivative on the wrong axis."""
-    if t.dim() <= 1:
+    shape, stride = t.shape, t.stride()
+    # the usual case, three extents with exactly Fortran strides, without
+    # building a view (the checks of a call on a 64^3 field cost as much host
+    # time as its kernel runs)
+    if len(shape) == 3 and stride == (1, shape[0], shape[0] * shape[1]):
+        return True
+    if len(shape) <= 1:
         return t.is_contiguous()
-    return t.permute(*reversed(range(t.dim()))).is_contiguous()
+    return t.permute(*reversed(range(len(shape)))).is_contiguous()
 
 
 def _stream_ptr():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device, as the address ctypes passes."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _check_device_arrays(f, df, count):
-    if f.dtype != df.dtype:
+    dtype = f.dtype
+    if dtype != df.dtype:
         raise TypeError("f and df must have the same dtype")
-    if f.dtype not in (torch.float64, torch.float32):
+    if dtype != torch.float64 and dtype != torch.float32:
         raise TypeError("f must be float64 or float32")
     if not (f.is_cuda and df.is_cuda):
         raise TypeError("device arrays must live on the GPU")
@@ -154,15 +162,16 @@ class _CompactOp:
             a = 1.0 if alpha is None else float(alpha)
             b = 0.0 if beta is None else float(beta)
             fn = lib.pade_op_apply_axpby if f.dtype == torch.float64 else lib.pade_op_apply_axpby_f32
-            _lib.check(fn(self._h, oper, axis, a, ctypes.c_void_p(f.data_ptr()), b, ctypes.c_void_p(df.data_ptr()),
-                          int(na), int(nb), b1, bn, _stream_ptr()))
+            _lib.check(fn(self._h, oper, axis, a, f.data_ptr(), b, df.data_ptr(), int(na), int(nb), b1, bn,
+                          _stream_ptr()))
             return df
         if f.dtype == torch.float64:
             fn = lib.pade_op_apply_adjoint if adjoint else lib.pade_op_apply
         else:
             fn = lib.pade_op_apply_adjoint_f32 if adjoint else lib.pade_op_apply_f32
-        _lib.check(fn(self._h, oper, axis, ctypes.c_void_p(f.data_ptr()), ctypes.c_void_p(df.data_ptr()),
-                      int(na), int(nb), b1, bn, _stream_ptr()))
+        rc = fn(self._h, oper, axis, f.data_ptr(), df.data_ptr(), int(na), int(nb), b1, bn, _stream_ptr())
+        if rc:
+            _lib.check(rc)
         return df
 
     def dense_apply(self, oper, axis, f, df, na, nb, prec, bc1=None, bcn=None):
