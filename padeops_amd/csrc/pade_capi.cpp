@@ -61,8 +61,8 @@ struct PlanKey {
 };
 
 struct Plan {
-    std::vector<Variant> spike;  // register-path variants (M in {16,32,64}), ascending M; the
-                                 // uneven ones only where no M divides the rows
+    std::vector<Variant> spike;  // register-path variants: M of 16, 32, 64 (48) dividing the rows,
+                                 // then the uneven ones
     Variant generic;             // whole pencil as one partition
     bool has_generic = false;
     pade::OpMatrices mats;       // for the dense form
@@ -230,14 +230,25 @@ void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double>
         Variant v;
         if (build_variant(m, M, tab, v) == 0) pl.spike.push_back(v);
     }
-    if (!pl.spike.empty()) return;
-    for (int M : {16, 24, 32, 64}) {
+    // Uneven partitions, of the sizes that pick_variant prefers: everywhere
+    // that no size divides the rows, for lengths of 144 .. 240 that 16 alone
+    // divides, and 40 or 48 slots from n = 257 to 384.
+    const int n = m.n;
+    const bool mid = n > 256 && n <= 384;
+    if (mid && m.periodic && n == 8 * 48) {         // whole-pencil x waves
+        Variant v;
+        if (build_variant(m, 48, tab, v) == 0) pl.spike.push_back(v);
+    }
+    if (!pl.spike.empty() && !(n % 32 == 16 && n >= 144) && !mid) return;
+    const bool none = pl.spike.empty();
+    for (int M : {16, 24, 32, 40, 48, 64}) {
         pade::UnevenParts parts;
         Variant v;
-        // (those that pick_variant never prefers are not built: 24 rows where
-        // 32 have a split, 64 up to n = 256, 32 on longer bounded pencils)
-        if ((M == 24 && m.n >= 40) || m.nbl > rows || m.nbr > rows) continue;
-        if (m.n <= 256 ? M == 64 : (M == 32 && !m.periodic)) continue;
+        bool want;
+        if (mid) want = M == 48 || (M == 40 && n <= 320);
+        else if (n <= 256) want = M == 32 || (none && (M == 16 || (M == 24 && n < 40)));
+        else want = M == 64 || (M == 32 && m.periodic);
+        if (!want || m.nbl > rows || m.nbr > rows) continue;
         if (pade::uneven_parts(m.n, M, parts) && build_variant(m, M, tab, v, &parts) == 0) pl.spike.push_back(v);
     }
 }
@@ -401,7 +412,32 @@ const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mod
     // / 330-331 / 330-332, n = 128 283 / 317-318 / 321 vs 325-329 / 364-368 /
     // 367-371, n = 256 306-308 / 311 / 293 vs 314-316 / 340-343 / 319-320;
     // bounded n = 512 337-338 / 322 / 303-304 vs 242 / 258 / 240).
-    const int pref_m = pl.mats.n <= 256 ? 32 : ((mode == 1 || !pl.mats.periodic) ? 64 : 32);
+    // From 257 to 384 points x takes 48 slots and strided rows 40 up to 320
+    // and then 48: at most eight partitions, four waves per workgroup (512 x
+    // 256 pencils, FP64, us, x / y / z, with 32, 40, 48, 64 slots: periodic n =
+    // 260 223 / 138 / 138, 162 / 119 / 122, 153 / 116 / 121, 181 / 151 / 154;
+    // n = 320 195 / 144 / 153, 164 / 130 / 136, 136 / 135 / 141, 140 / 146 /
+    // 161; n = 384 215 / 164 / 175, 302 / 225 / 229, 157 / 153 / 160, 162 /
+    // 164 / 184; bounded n = 288 202 / 153 / 157, 167 / 130 / 138, 145 / 139 /
+    // 142, 172 / 173 / 175), but for bounded x that 64 divides (n = 320 152
+    // with 64, 163 with 48; n = 384 169, 172).  Nine or more partitions of 40
+    // or 48 rows lose a workgroup per CU, so longer pencils return to 64 and
+    // 32.  (Even bounded rows of n = 512 measure 235 / 255 us with 64 and 230 /
+    // 239 with 32 slots since those fit four waves per SIMD; they keep the
+    // reported 64.)
+    // FP32, whose even kernels have twice the waves in flight, stays with
+    // these where they exist, but for bounded strided rows (512 x 512 pencils,
+    // us, even and uneven: periodic n = 288 135 / 128 / 132 and 150 / 135 /
+    // 138, n = 352 160 / 158 / 162 and 177 / 166 / 167; bounded 195 / 155 /
+    // 158 and 172 / 140 / 140, n = 320 147 / 151 / 154 and 182 / 145 / 147).
+    const int n = pl.mats.n;
+    const bool even = std::any_of(pl.spike.begin(), pl.spike.end(), [](const Variant &v) { return !v.uneven; });
+    const bool beside = fp64 || !even || (mode != 1 && !pl.mats.periodic);
+    const bool mid = n > 256 && n <= 384 && beside;
+    const int pref_m = n <= 256 ? 32
+                       : !mid   ? (mode == 1 || !pl.mats.periodic ? 64 : 32)
+                       : mode == 1 ? (!pl.mats.periodic && n % 64 == 0 ? 64 : 48)
+                                   : (n <= 320 ? 40 : 48);
     // Whole pencils per wave (x, 8 partitions of 32 or 64 points) read every
     // line once and stream their loads: preferred for periodic x when the
     // pencil fills all 8 partition slots of the wave (512^3: FP64 +1.5-2 %;
@@ -421,7 +457,11 @@ const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mod
         // uneven kernels take two partitions per wave
         if (v.uneven && (pw != 2 || npencils < kUnevenPencils)) return -1;
         if ((v.P + pw - 1) / pw > 8) return -1;
-        if (pw == 8 && (mode != 1 || v.P > 8 || (v.M != 32 && v.M != 64))) return -1;
+        if (pw == 8 && (mode != 1 || v.P > 8 || (v.M != 32 && v.M != 48 && v.M != 64))) return -1;
+        if (v.M == 48 && !v.uneven && (pw != 8 || !fp64)) return -1;        // whole pencils only
+        // (FP32 x beside 16 from eleven partitions of 16 rows: n = 144 90 ->
+        // 91 us, 176 116 -> 96, bounded 108 -> 113, 134 -> 108)
+        if (v.uneven && !beside && !(mode == 1 && n > 160 && n <= 256)) return -1;
         // four partitions per wave: strided rows only, by request (tuning)
         if (pw == 4 && (mode != 0 || envPW != 4 || (v.M != 32 && v.M != 64))) return -1;
         if (envM && v.M != envM) return -1;
@@ -431,19 +471,33 @@ const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mod
         const long long waves = groups * ((v.P + pw - 1) / pw);
         return waves * 64 > kMaxLaunchThreads ? -1 : waves;
     };
-    // a latency-bound size (no variant reaches 4096 waves) takes the variant
+    // A latency-bound size (no variant reaches 4096 waves) takes the variant
     // with the most waves (the shortest partitions); otherwise the throughput
-    // preferences below
-    long long max_waves = -1;
+    // preferences below.  x above 256 points (FP32: 384) takes these as soon
+    // as they give two waves per CU (9216 pencils of 512 points: FP64 21 us
+    // with 64 rows, 31 with 32, FP32 15 and 19; of 288 FP64 17 with 48, 22
+    // with 32, strided rows 15.9 and 15.4; of 384 FP32 13.8 with 64, 12.6).
+    // And with the chip filled, more than ten partitions of 16 rows lose to 32
+    // by their reduced system (FP64, 96^2 pencils, bounded x n = 192 19 -> 14
+    // us, 176 20 -> 17, y 13.7 -> 12.6; 40^2 pencils 9.1 -> 10.1, kept, as is
+    // periodic x beside uneven 32, 13.5 and 15.8).
+    long long max_waves = -1, pref_waves = -1;
     for (const Variant &v : pl.spike)
-        for (int pw : {1, 2, 4, 8}) max_waves = std::max(max_waves, waves_of(v, pw));
-    const bool small = max_waves < 4096;
+        for (int pw : {1, 2, 4, 8}) {
+            max_waves = std::max(max_waves, waves_of(v, pw));
+            if (v.M == pref_m) pref_waves = std::max(pref_waves, waves_of(v, pw));
+        }
+    const bool small = max_waves < 4096 && !(mode == 1 && n > (fp64 ? 256 : 384) && pref_waves >= 512);
+    auto small_rank = [&](const Variant &v) {
+        const bool keep16 = mode == 1 && pl.mats.periodic && n % 32;
+        return v.M == 16 && v.P > 10 && !keep16 && fp64 && max_waves >= 1024 ? 33 : v.M;
+    };
     for (const Variant &v : pl.spike)
         for (int pw : {1, 2, 4, 8}) {
             if (waves_of(v, pw) < 0) continue;
             int score = (pw == 2 ? 100 : 0) + (pw == 8 && prefer_whole && v.P == 8 ? 300 : 0) +
                         (v.M == pref_m ? 50 : (v.M == 64 ? 30 : (v.M == 32 ? 20 : 10)));
-            if (small) score = 1000 - v.M + (pw == 2 ? 1 : 0);
+            if (small) score = 1000 - 2 * small_rank(v) + (pw == 2 ? 1 : 0);
             if (score > best_score) { best_score = score; best = &v; best_pw = pw; }
         }
     *pw_out = best_pw;
@@ -1167,7 +1221,7 @@ int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, 
     if (kind == pade::CD06STAGG && !periodic && (pade::stagg_edge_in(oper) || pade::stagg_edge_out(oper)))
         if (int rc = pade::build_stagg_system(oper, n, dx, bc1, bcn, m)) return fail(rc, "operator construction failed");
     pade::UnevenParts parts;
-    if ((M != 16 && M != 24 && M != 32 && M != 64) || !pade::uneven_parts(m.n, M, parts))
+    if (M < 16 || M > 64 || M % 8 || M == 56 || !pade::uneven_parts(m.n, M, parts))
         return fail(21, "no uneven split of this length");
     std::vector<double> t;
     Variant v;

@@ -815,7 +815,10 @@ int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
 
 bool uneven_parts(int n, int M, UnevenParts &out)
 {
-    if (n <= M || n % M == 0) return false;
+    // (40 and 48 slots serve the lengths that they divide as well: those have
+    // no even kernels of that size but for whole pencils)
+    const bool mid = M == 40 || M == 48;
+    if (n <= M || (n % M == 0 && !mid)) return false;
     // Short partitions lose accuracy where A is nearly singular (cf90: the
     // bounded adjoint's error against 128-bit arithmetic grows from 2e-13
     // with 20 or more rows to 1e-12 with 8 to 12), so partitions of 16 and 24
@@ -825,7 +828,7 @@ bool uneven_parts(int n, int M, UnevenParts &out)
     out.n = n;
     out.M = M;
     out.P = (n + M - 1) / M;
-    out.unit = n % 16 == 0 && M == 64 ? 16 : (n % 4 == 0 ? 4 : (n % 2 == 0 ? 2 : 1));
+    out.unit = n % 16 == 0 && (M == 64 || M == 48) ? 16 : (n % 4 == 0 ? 4 : (n % 2 == 0 ? 2 : 1));
     const int units = (n - M) / out.unit;             // the unit divides n and M
     out.base = units / (out.P - 1) * out.unit;
     out.extra = units % (out.P - 1);

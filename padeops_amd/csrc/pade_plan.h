@@ -64,12 +64,12 @@ struct OpMatrices {
     double tail_dn = 0.0, tail_idg = 0.0;
 };
 
-// Split of n rows into P partitions of M register slots each when M does not
-// divide n.  Partition p < P - 1 holds `base` (+ `unit` for p < extra) rows
+// Split of n rows into P partitions of M register slots each, mostly where M
+// does not divide n.  Partition p < P - 1 holds `base` (+ `unit` for p < extra) rows
 // and its remaining slots are padding; the last holds M rows, so that the
 // special rows of a bounded pencil keep their slots at both ends.  `unit` is
 // the largest of 4, 2, 1 that divides n (16-byte starts for x pencils), or 16
-// for M = 64 and n a multiple of 16 (whole-line starts of FP64 x pencils).  A
+// for M = 48 or 64 and n a multiple of 16 (whole-line starts of FP64 x pencils).  A
 // padding slot t carries the equation y_t = y_{t-2}, which stays inside the
 // band: the last two slots of every partition then repeat its last two rows
 // (exchanged when the number of padding slots is odd), and the kernels' tip
@@ -79,8 +79,8 @@ struct UnevenParts {
     int rows(int p) const { return p == P - 1 ? M : base + (p < extra ? unit : 0); }
     int start(int p) const { return p * base + (p < extra ? p : extra) * unit; }
 };
-// The split of n rows for M slots: false when there is none (M divides n,
-// more than 16 partitions, partitions of fewer than 8 rows, or more than two
+// The split of n rows for M slots: false when there is none (M other than 40
+// or 48 divides n, more than 16 partitions, partitions of fewer than 8 rows, or more than two
 // of 16 or 24 slots).
 bool uneven_parts(int n, int M, UnevenParts &out);
 

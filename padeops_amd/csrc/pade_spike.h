@@ -143,12 +143,13 @@ __device__ __forceinline__ void pin(T &x) { asm volatile("" : "+v"(x)); }
 
 // x-pencil transpose tile: XT points of a row per chunk (aligned segments
 // of 64 bytes for FP64, 128 bytes for FP32 -- the widths that keep the FP64
-// M = 64 kernel within 256 registers and the FP32 one within 128); the halo
+// M = 64 kernel within 256 registers and the FP32 one within 128; partitions
+// that those do not divide take 16 or 8 points); the halo
 // chunk holds the 4 + 4 window points either side of the partition.
 __host__ __device__ constexpr int xtile_points(int tsize, int M)
 {
     const int xt = tsize == 8 ? 16 : 32;
-    return M % xt == 0 ? xt : (M == 24 ? 8 : M);
+    return M % xt == 0 ? xt : (M % 16 == 0 ? 16 : 8);
 }
 constexpr int kHaloChunk = 8;
 // How the row segments of a strided-row workgroup (its pencils' values at one

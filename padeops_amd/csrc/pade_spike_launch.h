@@ -44,6 +44,10 @@ hipError_t launch_spike(const ApplyArgs<T> &a, int M, int PW, int GW, bool adj, 
         switch (M) {
         case 32:
             return adj ? launch_spike_t<T, 32, 8, true, 1>(a, GW, s) : launch_spike_t<T, 32, 8, false, 1>(a, GW, s);
+        case 48:
+            if constexpr (sizeof(T) == 8)       // (periodic: no adjoint form)
+                return adj ? hipErrorInvalidValue : launch_spike_t<T, 48, 8, false, 1>(a, GW, s);
+            return hipErrorInvalidValue;
         case 64:
             return adj ? launch_spike_t<T, 64, 8, true, 1>(a, GW, s) : launch_spike_t<T, 64, 8, false, 1>(a, GW, s);
         default: return hipErrorInvalidValue;

@@ -20,6 +20,8 @@ hipError_t launch_stage(const ApplyArgs<double> &a, int M, bool uneven, hipStrea
     case 16: return uneven ? stage_m<16, true>(a, s) : stage_m<16, false>(a, s);
     case 24: return uneven ? stage_m<24, true>(a, s) : hipErrorInvalidValue;
     case 32: return uneven ? stage_m<32, true>(a, s) : stage_m<32, false>(a, s);
+    case 40: return uneven ? stage_m<40, true>(a, s) : hipErrorInvalidValue;
+    case 48: return uneven ? stage_m<48, true>(a, s) : hipErrorInvalidValue;
     case 64: return uneven ? stage_m<64, true>(a, s) : stage_m<64, false>(a, s);
     default: return hipErrorInvalidValue;
     }

@@ -24,6 +24,8 @@ hipError_t launch_twice(const ApplyArgs<double> &a, int M, int PW, int GW, bool 
     case 16: return PW == 2 ? launch_twice_16(a, uneven, adj, mode, s) : hipErrorInvalidValue;
     case 24: return uneven ? launch_twice_24(a, adj, mode, s) : hipErrorInvalidValue;
     case 32: return uneven ? launch_twice_32u(a, adj, mode, s) : launch_twice_32(a, PW, GW, adj, mode, s);
+    case 40:
+    case 48: return launch_twice_mid(a, M, PW, GW, uneven, adj, mode, s);
     case 64: return uneven ? launch_twice_64u(a, adj, mode, s) : launch_twice_64(a, PW, GW, adj, mode, s);
     default: return hipErrorInvalidValue;
     }

@@ -33,6 +33,8 @@ hipError_t launch_twice_16(const ApplyArgs<double> &a, bool uneven, bool adj, in
 hipError_t launch_twice_24(const ApplyArgs<double> &a, bool adj, int mode, hipStream_t s);
 hipError_t launch_twice_32(const ApplyArgs<double> &a, int PW, int GW, bool adj, int mode, hipStream_t s);
 hipError_t launch_twice_32u(const ApplyArgs<double> &a, bool adj, int mode, hipStream_t s);
+hipError_t launch_twice_mid(const ApplyArgs<double> &a, int M, int PW, int GW, bool uneven, bool adj, int mode,
+                            hipStream_t s);
 hipError_t launch_twice_64(const ApplyArgs<double> &a, int PW, int GW, bool adj, int mode, hipStream_t s);
 hipError_t launch_twice_64u(const ApplyArgs<double> &a, bool adj, int mode, hipStream_t s);
 

@@ -19,6 +19,10 @@ static hipError_t launch_uneven_m(const ApplyArgs<T> &a, bool adj, int mode, hip
                      : launch_spike_t<T, M, 2, true, 1, true>(a, 1, s);
 }
 
+// 40 and 48 slots, in translation units of their own
+template <typename T>
+hipError_t launch_uneven_mid(const ApplyArgs<T> &a, int M, bool adj, int mode, hipStream_t s);
+
 template <typename T>
 hipError_t launch_uneven(const ApplyArgs<T> &a, int M, bool adj, int mode, hipStream_t s)
 {
@@ -27,6 +31,8 @@ hipError_t launch_uneven(const ApplyArgs<T> &a, int M, bool adj, int mode, hipSt
     case 16: return launch_uneven_m<T, 16>(a, adj, mode, s);
     case 24: return launch_uneven_m<T, 24>(a, adj, mode, s);
     case 32: return launch_uneven_m<T, 32>(a, adj, mode, s);
+    case 40:
+    case 48: return launch_uneven_mid<T>(a, M, adj, mode, s);
     case 64: return launch_uneven_m<T, 64>(a, adj, mode, s);
     default: return hipErrorInvalidValue;
     }

@@ -26,7 +26,7 @@ def rel(a, b):
     return float(np.abs(a - b).max() / np.abs(b).max())
 
 
-@pytest.mark.parametrize("n", [16, 24, 37, 64, 75, 96, 129, 257, 512])
+@pytest.mark.parametrize("n", [16, 24, 37, 64, 75, 96, 129, 257, 336, 512])
 @pytest.mark.parametrize("axis", [1, 2, 3])
 def test_bounded_cd06_second_derivative(n, axis):
     op = po.cd06()
@@ -62,7 +62,10 @@ def _state(shape, seed):
 
 @pytest.mark.parametrize("shape,periodic,bc", [
     ((32, 40, 25), (True, True, True), ((0, 0),) * 3),
-    ((48, 24, 33), (True, True, False), ((0, 0), (0, 0), (0, 0)))])
+    ((48, 24, 33), (True, True, False), ((0, 0), (0, 0), (0, 0))),
+    ((16, 24, 300), (True, True, True), ((0, 0),) * 3),
+    ((384, 64, 64), (True, True, True), ((0, 0),) * 3),
+    ((16, 24, 336), (True, True, True), ((0, 0),) * 3)])
 @pytest.mark.parametrize("inviscid", [True, False])
 def test_batched_step_matches_oracle(shape, periodic, bc, inviscid):
     s0, h = _state(shape, sum(shape))
@@ -89,7 +92,8 @@ def test_batched_step_matches_oracle(shape, periodic, bc, inviscid):
 
 @pytest.mark.parametrize("shape,periodic,bc", [
     ((20, 64, 37), (False, True, False), ((0, 0), (0, 0), (1, -1))),
-    ((129, 16, 40), (False, False, True), ((1, 1), (-1, 0), (0, 0)))])
+    ((129, 16, 40), (False, False, True), ((1, 1), (-1, 0), (0, 0))),
+    ((24, 336, 384), (True, True, True), ((0, 0),) * 3)])
 @pytest.mark.parametrize("inviscid", [True, False])
 def test_batched_rhs_matches_oracle(shape, periodic, bc, inviscid):
     """Bounded axes with mixed closures (the fields of a batch then differ in

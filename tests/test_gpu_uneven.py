@@ -58,7 +58,8 @@ def test_uneven_matches_oracle(kind, which, periodic, bc, n, axis):
     assert rel(out.cpu().numpy(), pd.apply_axis(D.T, fh, axis - 1)) < 1e-12
 
 
-@pytest.mark.parametrize("n,pencils", [(129, (150, 130)), (300, (150, 130)), (513, (64, 33)), (1023, (40, 33))])
+@pytest.mark.parametrize("n,pencils", [(129, (150, 130)), (176, (70, 65)), (300, (150, 130)), (320, (41, 40)),
+                                       (384, (41, 40)), (513, (64, 33)), (1023, (40, 33))])
 @pytest.mark.parametrize("axis", [1, 2, 3])
 @pytest.mark.parametrize("periodic", [True, False])
 def test_uneven_throughput_sizes(n, pencils, axis, periodic):

@@ -71,7 +71,8 @@ def solve(tab, m, r):
 
 
 LENGTHS = [(24, 16), (25, 16), (30, 16), (31, 16), (33, 24), (36, 24), (39, 24), (40, 32), (41, 32), (63, 32), (97, 32),
-           (129, 32), (200, 32), (511, 32), (72, 64), (73, 64), (257, 64), (300, 64), (1023, 64), (544, 64)]
+           (129, 32), (200, 32), (511, 32), (72, 64), (73, 64), (257, 64), (300, 64), (1023, 64), (544, 64),
+           (257, 40), (300, 40), (320, 40), (258, 48), (321, 48), (336, 48), (383, 48), (384, 48)]
 
 
 @pytest.mark.parametrize("kind,which", [("cd06", "d1"), ("cd06", "d2"), ("cd10", "d1"), ("cd10", "d2"),
@@ -125,13 +126,13 @@ def test_splits_keep_their_bounds():
     """Every length: rows per partition, the last partition full, starts a
     multiple of the widest vector that divides the length."""
     for n in range(17, 1100):
-        for M in (16, 24, 32, 64):
+        for M in (16, 24, 32, 40, 48, 64):
             tab, m = export(PADE_CD10, PADE_D1, n, 0.1, True, 0, 0, False, M)
             if tab is None:
                 P = -(-n // M)
-                assert n <= M or n % M == 0 or P > 16 or (n - M) // (P - 1) < 8 + 3 or (M < 32 and n > 2 * M), (n, M)
+                assert n <= M or (n % M == 0 and M not in (40, 48)) or P > 16 or (n - M) // (P - 1) < 8 + 3 or (M < 32 and n > 2 * M), (n, M)
                 continue
-            unit = 16 if M == 64 and n % 16 == 0 else 4 if n % 4 == 0 else 2 if n % 2 == 0 else 1
+            unit = 16 if M in (48, 64) and n % 16 == 0 else 4 if n % 4 == 0 else 2 if n % 2 == 0 else 1
             assert all(s % unit == 0 for s in m["start"]) and m["rows"][-1] == M
             assert all(8 <= k <= M for k in m["rows"]) and sum(m["rows"]) == n
             assert all(s + M <= n for s in m["start"])          # windows stay inside the pencil
