@@ -65,6 +65,11 @@ struct Plan {
                                  // then the uneven ones
     Variant generic;             // whole pencil as one partition
     bool has_generic = false;
+    // does a partition size divide the rows?
+    bool even() const
+    {
+        return std::any_of(spike.begin(), spike.end(), [](const Variant &v) { return !v.uneven; });
+    }
     pade::OpMatrices mats;       // for the dense form
 };
 
@@ -431,8 +436,7 @@ const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mod
     // 138, n = 352 160 / 158 / 162 and 177 / 166 / 167; bounded 195 / 155 /
     // 158 and 172 / 140 / 140, n = 320 147 / 151 / 154 and 182 / 145 / 147).
     const int n = pl.mats.n;
-    const bool even = std::any_of(pl.spike.begin(), pl.spike.end(), [](const Variant &v) { return !v.uneven; });
-    const bool beside = fp64 || !even || (mode != 1 && !pl.mats.periodic);
+    const bool beside = fp64 || !pl.even() || (mode != 1 && !pl.mats.periodic);
     const bool mid = n > 256 && n <= 384 && beside;
     const int pref_m = n <= 256 ? 32
                        : !mid   ? (mode == 1 || !pl.mats.periodic ? 64 : 32)
@@ -657,9 +661,9 @@ int apply_one(pade_op_t op, const Plan &pl, int axis, const T *f, T *df, int na,
         }
         if (v->uneven) {
             // The allocation-free entry point refuses accumulating applies
-            // whose one-lane form would not fit its array; lengths that take
-            // uneven partitions keep that documented limit.
-            if (ws.on && epi.on) {
+            // whose one-lane form would not fit its array; lengths that no
+            // partition size divides keep that documented limit.
+            if (ws.on && epi.on && !pl.even()) {
                 T *unused = nullptr;
                 if (int rc = scratch_get<T>(ws, (size_t)a.npencils * n, s, &unused, "accumulate temporary")) return rc;
             }
@@ -772,7 +776,7 @@ int apply_impl(pade_op_t op, int oper, int axis, const T *f, T *df, int na, int 
             if (twice_ok(L)) {
                 // (the allocation-free entry point keeps its size limit, see apply_one)
                 if (ws.on && epi.on) {
-                    const size_t fields = L.v->uneven ? 2 : 1;
+                    const size_t fields = p1->even() ? 1 : 2;
                     T *unused = nullptr;
                     if (int rc = scratch_get<T>(ws, fields * (size_t)count, s, &unused,
                                                 "cd06 second derivative intermediate"))

@@ -4,6 +4,8 @@ the dense oracle, at the edges of the splits (shortest partitions, odd and
 even padding, one and two partitions in the last wave) with pencil counts
 that leave the last workgroup partly empty.  FP64 to 1e-12, FP32 to the
 suite's banded tolerance."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -106,3 +108,22 @@ def test_uneven_in_place_filter3d():
     for a in (1, 0, 2):
         ref = pd.apply("cf90", "filter", ref, a, 1.0, a < 2, 0, 0)
     assert rel(ft.cpu().numpy(), ref) < 1e-12
+
+
+@pytest.mark.parametrize("kind,which,n,side,periodic", [("cd10", "d1", 320, 165, True), ("cd10", "d1", 240, 190, False),
+                                                        ("cd06", "d2", 320, 130, False)])
+def test_noalloc_limit_of_divided_lengths(kind, which, n, side, periodic):
+    """Lengths that a partition size divides need no scratch array to
+    accumulate (cd06's bounded second derivative one field of it), also where
+    they run uneven partitions: fields above that limit are taken."""
+    op, f, _ = setup(kind, n, periodic, 3, n, pencils=(side, side))
+    v = _lib.plan_variant(op._kind, OPER[which], n, 0.05, periodic, 3, side, side, 0, 0)
+    assert f.numel() * 8 * (2 if which == "d2" else 1) > _lib.PADE_NOALLOC_SCRATCH_BYTES
+    ref, out = f.clone(), f.clone()
+    op._apply(OPER[which], 3, f, ref, side, side, alpha=0.5, beta=-2.0)
+    print(f"noalloc {kind} {which} n {n} {v}", flush=True)
+    rc = _lib.load().pade_op_apply_axpby_noalloc(op._h, OPER[which], 3, 0.5, ctypes.c_void_p(f.data_ptr()), -2.0,
+                                                 ctypes.c_void_p(out.data_ptr()), side, side, 0, 0,
+                                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    assert torch.equal(ref, out)
