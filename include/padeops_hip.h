@@ -267,12 +267,12 @@ int pade_plan_export(int kind, int oper, int n, double dx, int periodic, int bc1
  * that M = 40 or 48 serves: the table of its uneven partitions (a staggered
  * operator with an edge array: its system form).  meta[64]: as
  * pade_plan_export in [0, 32), [32] = W, the partitions of a reduced-system
- * row, [33 + p] = first row of partition p.  Every partition occupies M slots:
- * its rows, then padding slots with y_t = y_{t-2} and a zero right-hand side;
- * the last partition has M rows.  The reduced-system rows hold, for every
- * partition, 4 rows of 4 W values: entry j for partition p - kq + j (cyclic
- * when periodic), or partition j when W = P.  Returns 21 when the length has
- * no such split.  Used by tests. */
+ * row, [33 + p] = first row of partition p, [54 + p - 16] = class of p > 15.
+ * Every partition occupies M slots: its rows, then padding slots with y_t =
+ * y_{t-2} and a zero right-hand side; the last partition has M rows.  The
+ * reduced-system rows hold, for every partition, 4 rows of 4 W values: entry
+ * j for partition p - kq + j (cyclic when periodic), or partition j when W =
+ * P.  Returns 21 when the length has no such split.  Used by tests. */
 int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, int bc1, int bcn,
                             int adjoint, int M, double *tab, long long tab_len, int *meta);
 

@@ -46,7 +46,7 @@ struct Variant {
     long long off = 0;  // element offset of this variant's table in the plan buffer
     int nbl = 0, nbr = 0;
     int coef_len = 0, ncls = 0, kq = 0;
-    int cls[pade::kMaxPartitions] = {0};
+    int cls[pade::kMaxLongPartitions] = {0};
     int len = 0;
     bool uneven = false;   // partitions of `parts`
     pade::UnevenParts parts;
@@ -111,7 +111,7 @@ int build_variant(const pade::OpMatrices &m, int M, std::vector<double> &tab, Va
         for (int k = 0; k < (int)reps.size(); k++)
             if (same(reps[k], p)) { c = k; break; }
         if (c < 0) { c = (int)reps.size(); reps.push_back(p); }
-        if (p < pade::kMaxPartitions) v.cls[p] = c;
+        if (p < pade::kMaxLongPartitions) v.cls[p] = c;
     }
     if (periodic && !parts && reps.size() != 1) return 3;  // even periodic blocks are identical by construction
     v.ncls = (int)reps.size();
@@ -254,7 +254,9 @@ void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double>
         else if (n <= 256) want = M == 32 || (none && (M == 16 || (M == 24 && n < 40)));
         else want = M == 64 || (M == 32 && m.periodic);
         if (!want || m.nbl > rows || m.nbr > rows) continue;
-        if (pade::uneven_parts(m.n, M, parts) && build_variant(m, M, tab, v, &parts) == 0) pl.spike.push_back(v);
+        if (!pade::uneven_parts(m.n, M, parts) || build_variant(m, M, tab, v, &parts) != 0) continue;
+        if (v.P > pade::kMaxPartitions && v.ncls > 8) continue;     // three bits per partition
+        pl.spike.push_back(v);
     }
 }
 
@@ -458,8 +460,8 @@ const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mod
     const bool prefer_whole = mode == 1 && pl.mats.periodic;
     // eligible (variant, partitions per wave) pairs and their wave counts
     auto waves_of = [&](const Variant &v, int pw) -> long long {
-        // uneven kernels take two partitions per wave
-        if (v.uneven && (pw != 2 || npencils < kUnevenPencils)) return -1;
+        // uneven kernels take two partitions per wave, four of more than sixteen
+        if (v.uneven && (pw != (v.P > pade::kMaxPartitions ? 4 : 2) || npencils < kUnevenPencils)) return -1;
         if ((v.P + pw - 1) / pw > 8) return -1;
         if (pw == 8 && (mode != 1 || v.P > 8 || (v.M != 32 && v.M != 48 && v.M != 64))) return -1;
         if (v.M == 48 && !v.uneven && (pw != 8 || !fp64)) return -1;        // whole pencils only
@@ -467,7 +469,7 @@ const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mod
         // 91 us, 176 116 -> 96, bounded 108 -> 113, 134 -> 108)
         if (v.uneven && !beside && !(mode == 1 && n > 160 && n <= 256)) return -1;
         // four partitions per wave: strided rows only, by request (tuning)
-        if (pw == 4 && (mode != 0 || envPW != 4 || (v.M != 32 && v.M != 64))) return -1;
+        if (pw == 4 && !v.uneven && (mode != 0 || envPW != 4 || (v.M != 32 && v.M != 64))) return -1;
         if (envM && v.M != envM) return -1;
         if (envPW && pw != envPW) return -1;
         if (!offsets_fit(a, v.rect ? 2 : mode, v.M, pw)) return -1;
@@ -581,7 +583,8 @@ void set_tables(const Variant &v, pade::FieldArgs<T> &fd)
     fd.ncls = v.ncls;
     fd.kq = v.kq;
     fd.cls4 = 0;
-    for (int k = 0; k < pade::kMaxPartitions; k++) fd.cls4 |= (unsigned long long)v.cls[k] << (4 * k);
+    const int bits = v.P > pade::kMaxPartitions ? 3 : 4;
+    for (int k = 0; k < v.P; k++) fd.cls4 |= (unsigned long long)v.cls[k] << (bits * k);
 }
 
 // Variant, partitions per wave and mode of an apply along `axis` over
@@ -1233,7 +1236,7 @@ int pade_plan_export_uneven(int kind, int oper, int n, double dx, int periodic, 
     const int cols = m.n_in ? m.n_in : m.n;
     int vals[64] = {m.n, v.M, v.P, periodic ? 1 : 0, v.nbl, v.nbr, pade::kOffBl, pade::kOffBr,
                     pade::kOffCoef, v.coef_len, v.ncls, v.kq, v.len, cols, m.rect ? 1 : 0, m.tail ? 1 : 0};
-    for (int k = 0; k < pade::kMaxPartitions; k++) vals[16 + k] = v.cls[k];
+    for (int k = 0; k < v.P; k++) vals[k < 16 ? 16 + k : 54 + k - 16] = v.cls[k];
     vals[32] = std::min(2 * v.kq + 1, v.P);
     for (int p = 0; p < v.P; p++) vals[33 + p] = parts.start(p);
     std::memcpy(meta, vals, sizeof(vals));

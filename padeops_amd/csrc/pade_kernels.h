@@ -34,6 +34,9 @@ constexpr int kOffBl = 16;
 constexpr int kOffBr = 144;
 constexpr int kOffCoef = 272;
 constexpr int kMaxPartitions = 16;
+// Uneven partitions of 64 slots go on to 21, four per wave (three bits of class
+// each in the 64 of FieldArgs): pencils of up to 1344 points.
+constexpr int kMaxLongPartitions = 21;
 
 // One field of a launch: its arrays, and the table of its operator (boundary
 // codes may differ between the fields of a launch).
@@ -42,9 +45,10 @@ struct FieldArgs {
     const T *f;
     T *out;
     const T *tab;
-    unsigned long long cls4;   // block of partition p in bits 4p .. 4p + 3 (shifted
-                               // out of a scalar register: an array indexed per
-                               // lane is a load from the argument segment)
+    unsigned long long cls4;   // block of partition p in bits 4p .. 4p + 3, 3p .. 3p + 2
+                               // where P > 16 (shifted out of a scalar register:
+                               // an array indexed per lane is a load from the
+                               // argument segment)
     int nbl, nbr;
     int coef_len;          // length of the coefficient area
     int ncls;              // number of coefficient blocks

@@ -815,10 +815,11 @@ int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
 
 bool uneven_parts(int n, int M, UnevenParts &out)
 {
-    // (40 and 48 slots serve the lengths that they divide as well: those have
-    // no even kernels of that size but for whole pencils)
+    // (40 and 48 slots serve the lengths that they divide as well, those have
+    // no even kernels of that size but for whole pencils, and so do more than
+    // sixteen of 64)
     const bool mid = M == 40 || M == 48;
-    if (n <= M || (n % M == 0 && !mid)) return false;
+    if (n <= M || (n % M == 0 && !mid && n <= 16 * M)) return false;
     // Short partitions lose accuracy where A is nearly singular (cf90: the
     // bounded adjoint's error against 128-bit arithmetic grows from 2e-13
     // with 20 or more rows to 1e-12 with 8 to 12), so partitions of 16 and 24
@@ -832,7 +833,7 @@ bool uneven_parts(int n, int M, UnevenParts &out)
     const int units = (n - M) / out.unit;             // the unit divides n and M
     out.base = units / (out.P - 1) * out.unit;
     out.extra = units % (out.P - 1);
-    return out.P <= 16 && out.base >= 8;
+    return out.P <= (M == 64 ? 21 : 16) && out.base >= 8;
 }
 
 int spike_factor_uneven(const OpMatrices &op, const UnevenParts &u, SpikeFactors &out)

@@ -45,7 +45,7 @@
 //
 // Generic path (generic_apply, pade_kernels.hip): one lane per pencil with
 // the whole pencil as one partition in global memory -- for sizes the
-// register path does not cover (n < 24 unless 16, n > 1024, or fewer than 128 pencils of an uneven length).
+// register path does not cover (n < 24 unless 16, n > 1344, or fewer than 128 pencils of an uneven length).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -192,7 +192,7 @@ __host__ __device__ inline int lds_elems(int M, int P, int PW, bool adj, int mod
                                          int gw)
 {
     const int npen = 64 / PW;
-    const bool whole = mode == 1 && PW >= 4;      // tips in the tile area
+    const bool whole = mode == 1 && PW == 8;      // tips in the tile area
     const int waves = whole ? gw : (P + PW - 1) / PW;
     // (x pencils exchange the adjoint halo through their transpose tiles)
     int e = (whole ? 0 : (adj && mode != 1 ? 12 : 4) * P * npen) + (bnd ? 256 : 0) + coef_len;
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     const FieldArgs<T> &fd = a.fld[blockIdx.y];
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T *smem = reinterpret_cast<T *>(smem_raw);
-    constexpr bool WHOLE = MODE == 1 && PW >= 4;
+    constexpr bool WHOLE = MODE == 1 && PW == 8;
     const int lane = threadIdx.x & 63;
     const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Waves of a workgroup serve consecutive partitions of the same NPEN
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
         //     first partition and the right halo of its second (of the first
         //     when the pair has no second); the boundary inside the pair
         //     comes from the main chunks in LDS;
-        //   PW == 1: both sides, 4 + 4 points;
+        //   PW == 1 or 4: both sides, 4 + 4 points;
         //   PW == 8 (whole pencils per wave, P <= 8): none -- every halo is
         //     in the wave's own tile.
         constexpr int G = 64 / LPR;                      // rows per load instruction
@@ -466,12 +466,12 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
                 const bool ok = q0 + rp < a.npencils && part < P;
                 const int j = part_start(ok ? part : 0) + c * XT + VL * (lane % LPR);
                 const unsigned xo = ok ? (unsigned)((rp * (long long)n + j) * (long long)sizeof(T)) : 0u;
-                const vec_t v = PW >= 4 ? ldg_nt(fb, xo) : ldg(fb, xo);
+                const vec_t v = WHOLE ? ldg_nt(fb, xo) : ldg(fb, xo);
 #pragma unroll
                 for (int e = 0; e < VL; e++) w[W0 + c * XT + s * VL + e] = v[e];
             }
         }
-        if constexpr (!ADJ && PW <= 2) {   // (whole-pencil waves need no halo loads)
+        if constexpr (!ADJ && !WHOLE) {    // (whole-pencil waves need no halo loads)
             constexpr int HC = PW == 2 ? 4 : kHaloChunk;     // halo values per tile row
             constexpr int GH = 64 / HC;
 #pragma unroll
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
                         if (half == 1) w[k] = t;
                     }
                 }
-            } else if constexpr (PW >= 4 && !ADJ) {
+            } else if constexpr (WHOLE && !ADJ) {
                 // whole pencils in the wave (P <= PW): every halo is the end of
                 // a neighbouring partition in the tile, across the periodic
                 // wrap too (at the ends of a bounded pencil the boundary rows
@@ -566,7 +566,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
             }
             wave_lds_sync();
         }
-        if constexpr (!ADJ && PW <= 2) {
+        if constexpr (!ADJ && !WHOLE) {
             constexpr int HC = PW == 2 ? 4 : kHaloChunk;
             constexpr int GH = 64 / HC;
 #pragma unroll
@@ -598,7 +598,9 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
     }
 
     // coefficient blocks of this lane's partition
-    const int cls = BND || UNE ? (int)(fd.cls4 >> (4 * pc)) & 15 : 0;
+    // (four partitions per wave of a long uneven pencil: three bits each)
+    constexpr int CB = UNE && PW == 4 ? 3 : 4;
+    const int cls = BND || UNE ? (int)(fd.cls4 >> (CB * pc)) & ((1 << CB) - 1) : 0;
     const T *lu = coef + cls * 10 * M;      // [M][6]
     const T *S = lu + 6 * M;                // [M][4]
     const T *Qb = coef + fd.ncls * 10 * M;   // periodic: [4][4P] of partition 0; bounded: [P][4][4P];
@@ -936,7 +938,7 @@ template <typename T>
 bool uneven_layout_ok(const ApplyArgs<T> &a, int M)
 {
     const int inner = (a.P - 1) * a.ubase + std::min(a.P - 1, a.uextra) * a.uunit;
-    return a.P >= 2 && a.P <= kMaxPartitions && a.ubase >= kMinRows && a.ubase + (a.uextra ? a.uunit : 0) <= M &&
+    return a.P >= 2 && a.P <= (M == 64 ? kMaxLongPartitions : kMaxPartitions) && a.ubase >= kMinRows && a.ubase + (a.uextra ? a.uunit : 0) <= M &&
            a.uextra >= 0 && a.uextra < a.P && inner + M == a.n;
 }
 
@@ -966,7 +968,7 @@ template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, int EPI, bool
 hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
 {
     constexpr int NPEN = 64 / PW;
-    constexpr bool WHOLE = MODE == 1 && PW >= 4;
+    constexpr bool WHOLE = MODE == 1 && PW == 8;
     ApplyArgs<T> a = a_in;
     const int waves = WHOLE ? gw : (a.P + PW - 1) / PW;
     int coef_len = 0;
@@ -1012,7 +1014,7 @@ hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
 template <typename T, int M, int PW, bool ADJ, int MODE, bool UNE = false, int REP = 1>
 hipError_t launch_spike_t(const ApplyArgs<T> &a, int gw, hipStream_t s)
 {
-    constexpr bool WHOLE = MODE == 1 && PW >= 4;
+    constexpr bool WHOLE = MODE == 1 && PW == 8;
     if (!WHOLE) gw = 1;
     // the accumulate epilogue exists for the forward operator only
     if (ADJ && a.axpby) return hipErrorInvalidValue;

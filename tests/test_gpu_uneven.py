@@ -40,7 +40,7 @@ CASES = [("cd10", "d1", True, (0, 0)), ("cd10", "d2", True, (0, 0)), ("cf90", "f
 
 
 @pytest.mark.parametrize("kind,which,periodic,bc", CASES)
-@pytest.mark.parametrize("n", [24, 25, 37, 75, 129, 200, 257, 301])
+@pytest.mark.parametrize("n", [24, 25, 37, 75, 129, 200, 257, 301, 1025, 1100])
 @pytest.mark.parametrize("axis", [1, 2, 3])
 def test_uneven_matches_oracle(kind, which, periodic, bc, n, axis):
     op, f, fh = setup(kind, n, periodic, axis, n + axis)
@@ -61,7 +61,8 @@ def test_uneven_matches_oracle(kind, which, periodic, bc, n, axis):
 
 
 @pytest.mark.parametrize("n,pencils", [(129, (150, 130)), (176, (70, 65)), (300, (150, 130)), (320, (41, 40)),
-                                       (384, (41, 40)), (513, (64, 33)), (1023, (40, 33))])
+                                       (384, (41, 40)), (513, (64, 33)), (1023, (40, 33)), (1088, (40, 33)),
+                                       (1343, (25, 21))])
 @pytest.mark.parametrize("axis", [1, 2, 3])
 @pytest.mark.parametrize("periodic", [True, False])
 def test_uneven_throughput_sizes(n, pencils, axis, periodic):
@@ -76,7 +77,7 @@ def test_uneven_throughput_sizes(n, pencils, axis, periodic):
 
 
 @pytest.mark.parametrize("oper", ["ddz_E2C", "ddz_C2E", "InterpZ_C2E", "d2dz2_E2E", "ddz_C2C"])
-@pytest.mark.parametrize("n", [25, 70, 129])
+@pytest.mark.parametrize("n", [25, 70, 129, 1041])
 def test_uneven_staggered_bounded(oper, n):
     name = {"ddz_E2C": "d1_e2c", "ddz_C2E": "d1_c2e", "InterpZ_C2E": "interp_c2e", "d2dz2_E2E": "d2_e2e",
             "ddz_C2C": "d1_c2c"}[oper]

@@ -27,7 +27,7 @@ def export(kind, oper, n, dx, periodic, bc1, bcn, adjoint, M):
     keys = ["n", "M", "P", "periodic", "nbl", "nbr", "off_bl", "off_br", "off_coef", "coef_len", "ncls", "kq", "len",
             "n_in", "sys", "tail"]
     m = dict(zip(keys, list(meta)[:16]))
-    m["cls"], m["W"], m["start"] = list(meta)[16:32], meta[32], list(meta)[33:33 + m["P"]]
+    m["cls"], m["W"], m["start"] = list(meta)[16:32] + list(meta)[54:59], meta[32], list(meta)[33:33 + m["P"]]
     m["rows"] = [b - a for a, b in zip(m["start"], m["start"][1:] + [m["n"]])]
     return tab, m
 
@@ -72,7 +72,8 @@ def solve(tab, m, r):
 
 LENGTHS = [(24, 16), (25, 16), (30, 16), (31, 16), (33, 24), (36, 24), (39, 24), (40, 32), (41, 32), (63, 32), (97, 32),
            (129, 32), (200, 32), (511, 32), (72, 64), (73, 64), (257, 64), (300, 64), (1023, 64), (544, 64),
-           (257, 40), (300, 40), (320, 40), (258, 48), (321, 48), (336, 48), (383, 48), (384, 48)]
+           (257, 40), (300, 40), (320, 40), (258, 48), (321, 48), (336, 48), (383, 48), (384, 48),
+           (1025, 64), (1088, 64), (1100, 64), (1344, 64)]
 
 
 @pytest.mark.parametrize("kind,which", [("cd06", "d1"), ("cd06", "d2"), ("cd10", "d1"), ("cd10", "d2"),
@@ -125,12 +126,12 @@ def test_uneven_staggered_system_form(op, n, M):
 def test_splits_keep_their_bounds():
     """Every length: rows per partition, the last partition full, starts a
     multiple of the widest vector that divides the length."""
-    for n in range(17, 1100):
+    for n in range(17, 1360):
         for M in (16, 24, 32, 40, 48, 64):
             tab, m = export(PADE_CD10, PADE_D1, n, 0.1, True, 0, 0, False, M)
             if tab is None:
                 P = -(-n // M)
-                assert n <= M or (n % M == 0 and M not in (40, 48)) or P > 16 or (n - M) // (P - 1) < 8 + 3 or (M < 32 and n > 2 * M), (n, M)
+                assert n <= M or (n % M == 0 and M not in (40, 48)) or P > (21 if M == 64 else 16) or (n - M) // (P - 1) < 8 + 3 or (M < 32 and n > 2 * M), (n, M)
                 continue
             unit = 16 if M in (48, 64) and n % 16 == 0 else 4 if n % 4 == 0 else 2 if n % 2 == 0 else 1
             assert all(s % unit == 0 for s in m["start"]) and m["rows"][-1] == M
@@ -149,5 +150,6 @@ def test_variant_choice():
             assert v["uneven"] and not v["generic"] and v["PW"] == 2
             assert not pv(128, axis, 200, 200, periodic=periodic)["uneven"]
     assert pv(129, 2, 8, 16)["uneven"] and pv(129, 2, 127, 1)["generic"]
-    assert pv(23, 1, 64, 64)["generic"] and pv(1025, 1, 64, 64)["generic"]
+    assert pv(23, 1, 64, 64)["generic"] and pv(1345, 1, 64, 64)["generic"]
+    assert pv(1025, 1, 64, 64)["PW"] == 4 and pv(1344, 2, 64, 64)["PW"] == 4 and pv(1024, 3, 64, 64)["PW"] == 2
     assert _lib.plan_variant(PADE_CF90, PADE_FILTER, 272, 1.0, False, 3, 64, 64)["uneven"]
