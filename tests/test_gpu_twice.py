@@ -65,7 +65,8 @@ def _state(shape, seed):
     ((48, 24, 33), (True, True, False), ((0, 0), (0, 0), (0, 0))),
     ((16, 24, 300), (True, True, True), ((0, 0),) * 3),
     ((384, 64, 64), (True, True, True), ((0, 0),) * 3),
-    ((16, 24, 336), (True, True, True), ((0, 0),) * 3)])
+    ((16, 24, 336), (True, True, True), ((0, 0),) * 3),
+    ((16, 24, 1041), (True, True, True), ((0, 0),) * 3)])
 @pytest.mark.parametrize("inviscid", [True, False])
 def test_batched_step_matches_oracle(shape, periodic, bc, inviscid):
     s0, h = _state(shape, sum(shape))
