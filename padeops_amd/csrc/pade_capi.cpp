@@ -74,12 +74,15 @@ struct Plan {
 };
 
 // Assemble the table of one variant; returns 0 or an error code.
-// parts: the uneven partitions to use, or null for an even split into M rows.
+// parts: the uneven partitions to use (known: factors at hand), or null for an
+// even split into M rows.
 int build_variant(const pade::OpMatrices &m, int M, std::vector<double> &tab, Variant &v,
-                  const pade::UnevenParts *parts = nullptr)
+                  const pade::UnevenParts *parts = nullptr, std::vector<pade::PartFactors> *known = nullptr)
 {
     pade::SpikeFactors sf;
-    if (int rc = parts ? pade::spike_factor_uneven(m, *parts, sf) : pade::spike_factor(m, M, sf)) return rc;
+    std::vector<pade::PartFactors> none;
+    if (int rc = parts ? pade::spike_factor_uneven(m, *parts, known ? *known : none, sf) : pade::spike_factor(m, M, sf))
+        return rc;
     if (parts) {
         v.uneven = true;
         v.parts = *parts;
@@ -226,7 +229,8 @@ constexpr int kFilterRhsBc = 100 + pade::FILTER;
 
 // Partition sizes of the register path that serve this operator: those that
 // divide its rows, or else the uneven splits.
-void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double> &tab, Plan &pl)
+void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double> &tab,
+                        std::vector<pade::PartFactors> &known, Plan &pl)
 {
     // special rows the kernels hold
     const int rows = adj ? pade::kBRowsDev : (m.rect ? pade::kBRowsSys : pade::kBRowsFwd);
@@ -254,7 +258,7 @@ void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double>
         else if (n <= 256) want = M == 32 || (none && (M == 16 || (M == 24 && n < 40)));
         else want = M == 64 || (M == 32 && m.periodic);
         if (!want || m.nbl > rows || m.nbr > rows) continue;
-        if (!pade::uneven_parts(m.n, M, parts) || build_variant(m, M, tab, v, &parts) != 0) continue;
+        if (!pade::uneven_parts(m.n, M, parts) || build_variant(m, M, tab, v, &parts, &known) != 0) continue;
         if (v.P > pade::kMaxPartitions && v.ncls > 8) continue;     // three bits per partition
         pl.spike.push_back(v);
     }
@@ -265,7 +269,7 @@ void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double>
 // one-lane-per-pencil form.  bc1 / bcn are the codes that build the
 // operator (init-time for cd06 and cd06stagg).
 int build_plan(int kind, int oper, int n, double dx, bool periodic, int bc1, int bcn, bool adj,
-               std::vector<double> &tab, Plan &pl)
+               std::vector<double> &tab, std::vector<pade::PartFactors> &known, Plan &pl)
 {
     if (int rc = operator_matrices(kind, oper, n, dx, periodic, bc1, bcn, adj, pl.mats))
         return fail(rc, "operator construction failed");
@@ -280,7 +284,7 @@ int build_plan(int kind, int oper, int n, double dx, bool periodic, int bc1, int
         if (int rc = pade::build_stagg_system(oper, n, dx, bc1, bcn, sys)) return fail(rc, "operator construction failed");
     }
     const pade::OpMatrices &pm = sys_form ? sys : pl.mats;
-    add_spike_variants(pm, adj, tab, pl);
+    add_spike_variants(pm, adj, tab, known, pl);
     if (m >= 4 && build_variant(pl.mats, m, tab, pl.generic) == 0) pl.has_generic = true;
     return 0;
 }
@@ -289,6 +293,7 @@ int build_plan(int kind, int oper, int n, double dx, bool periodic, int bc1, int
 int build_all_plans(pade_op_s *op)
 {
     std::vector<double> tab;
+    std::vector<pade::PartFactors> known;
     std::vector<int> opers;
     if (op->kind == pade::CF90 || op->kind == pade::GAUSSIAN) opers = {pade::FILTER};
     else if (op->kind == pade::CD06STAGG) {
@@ -311,7 +316,7 @@ int build_all_plans(pade_op_s *op)
                 const int cb1 = init_bc ? op->init_bc1 : b1;
                 const int cbn = init_bc ? op->init_bcn : bn;
                 Plan pl;
-                if (int rc = build_plan(op->kind, oper, op->n, op->dx, op->periodic, cb1, cbn, adj != 0, tab, pl))
+                if (int rc = build_plan(op->kind, oper, op->n, op->dx, op->periodic, cb1, cbn, adj != 0, tab, known, pl))
                     return rc;
                 op->plans[{oper, b1, bn, adj}] = std::move(pl);
             }
@@ -326,7 +331,7 @@ int build_all_plans(pade_op_s *op)
             if (int rc = operator_matrices(op->kind, pade::FILTER, op->n, op->dx, false, b1, bn, false, pl.mats))
                 return fail(rc, "operator construction failed");
             pl.mats.band = nn.band;      // (bc1, bcn) right-hand side, (0, 0) left-hand side
-            add_spike_variants(pl.mats, false, tab, pl);
+            add_spike_variants(pl.mats, false, tab, known, pl);
             if (op->n >= 4 && build_variant(pl.mats, op->n, tab, pl.generic) == 0) pl.has_generic = true;
             op->plans[{kFilterRhsBc, b1, bn, 0}] = std::move(pl);
         }
@@ -1108,9 +1113,10 @@ int pade_plan_variant(int kind, int oper, int n, double dx, int periodic, int bc
         info[5] = 2;
     }
     std::vector<double> tab;
+    std::vector<pade::PartFactors> known;
     Plan pl;
     const bool filter_kind = kind == pade::CF90 || kind == pade::GAUSSIAN;
-    if (int rc = build_plan(kind, oper, n, filter_kind ? 1.0 : dx, periodic != 0, bc1, bcn, adjoint != 0, tab, pl))
+    if (int rc = build_plan(kind, oper, n, filter_kind ? 1.0 : dx, periodic != 0, bc1, bcn, adjoint != 0, tab, known, pl))
         return rc;
     int rc;
     int M = 0, pw = 1, P = 0, generic = 0, mode = 0, uneven = 0;

@@ -12,6 +12,7 @@
 // matching RHS rows).  bc = 0 rows are the one-sided closures.
 #include "pade_plan.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -625,19 +626,20 @@ namespace {
 // Band LU (no pivoting) of rows [r0, r0+rows) restricted to that block, in
 // M >= rows slots (the slots beyond the rows hold y_t = y_{t-2}).
 // lu[t*5 + {0..4}] = l1, l2, 1/pivot, u1/pivot, u2/pivot.
-int band_lu_block(const OpMatrices &op, int r0, int rows, int M, double *lu)
+template <typename Real>
+int band_lu_block(const OpMatrices &op, int r0, int rows, int M, Real *lu)
 {
-    std::vector<double> U((size_t)M * 3, 0.0);  // U rows: offsets 0..2
+    std::vector<Real> U((size_t)M * 3, Real(0));  // U rows: offsets 0..2
     for (int t = 0; t < M; t++) {
         const int i = r0 + t;
-        double row[5] = {-1.0, 0.0, 1.0, 0.0, 0.0};
+        Real row[5] = {-1.0, 0.0, 1.0, 0.0, 0.0};
         for (int o = -2; o <= 2 && t < rows; o++) {
             const int tt = t + o;
             row[o + 2] = (tt >= 0 && tt < rows) ? op.band[(size_t)i * 5 + o + 2] : 0.0;
         }
-        double l1 = 0.0, l2 = 0.0;
+        Real l1 = 0.0, l2 = 0.0;
         if (t >= 2) {
-            const double *u = &U[(size_t)(t - 2) * 3];
+            const Real *u = &U[(size_t)(t - 2) * 3];
             l2 = row[0] / u[0];
             // row t-2 spans columns t-2 .. t  -> offsets -2..0 of row t
             row[0] -= l2 * u[0];
@@ -645,7 +647,7 @@ int band_lu_block(const OpMatrices &op, int r0, int rows, int M, double *lu)
             row[2] -= l2 * u[2];
         }
         if (t >= 1) {
-            const double *u = &U[(size_t)(t - 1) * 3];
+            const Real *u = &U[(size_t)(t - 1) * 3];
             l1 = row[1] / u[0];
             row[1] -= l1 * u[0];
             row[2] -= l1 * u[1];
@@ -655,7 +657,7 @@ int band_lu_block(const OpMatrices &op, int r0, int rows, int M, double *lu)
         U[(size_t)t * 3 + 0] = row[2];
         U[(size_t)t * 3 + 1] = row[3];
         U[(size_t)t * 3 + 2] = row[4];
-        const double ip = 1.0 / row[2];
+        const Real ip = Real(1) / row[2];
         lu[t * 5 + 0] = l1;
         lu[t * 5 + 1] = l2;
         lu[t * 5 + 2] = ip;
@@ -665,16 +667,17 @@ int band_lu_block(const OpMatrices &op, int r0, int rows, int M, double *lu)
     return 0;
 }
 
-void band_lu_solve(const double *lu, int M, double *x)
+template <typename Real>
+void band_lu_solve(const Real *lu, int M, Real *x)
 {
     for (int t = 0; t < M; t++) {
-        double z = x[t];
+        Real z = x[t];
         if (t >= 1) z -= lu[t * 5 + 0] * x[t - 1];
         if (t >= 2) z -= lu[t * 5 + 1] * x[t - 2];
         x[t] = z;
     }
     for (int t = M - 1; t >= 0; t--) {
-        double g = x[t] * lu[t * 5 + 2];
+        Real g = x[t] * lu[t * 5 + 2];
         if (t + 1 < M) g -= lu[t * 5 + 3] * x[t + 1];
         if (t + 2 < M) g -= lu[t * 5 + 4] * x[t + 2];
         x[t] = g;
@@ -720,14 +723,104 @@ int invert(std::vector<double> &a, int m)
     return 0;
 }
 
-}  // namespace
-
-namespace {
+// The same in place for a matrix given to 64 bits whose rows have few entries,
+// each entry of the inverse rounded once: banded elimination in double (a
+// pivot row and a row above it meet only where the first has entries), one
+// correction from the residual in long double.
+int invert(std::vector<long double> &r, int m)
+{
+    std::vector<double> a(r.begin(), r.end()), x((size_t)m * m, 0.0), e((size_t)m * m);
+    std::vector<int> piv(m);
+    std::vector<int> list((size_t)2 * m * m), nright(m), nbelow(m);   // entries of U's rows, multipliers of L's columns
+    auto right = [&](int c) { return &list[(size_t)c * m]; };
+    auto below = [&](int c) { return &list[(size_t)(m + c) * m]; };
+    for (int c = 0; c < m; c++) {
+        int p = c;
+        for (int i = c + 1; i < m; i++)
+            if (std::fabs(a[(size_t)i * m + c]) > std::fabs(a[(size_t)p * m + c])) p = i;
+        if (a[(size_t)p * m + c] == 0.0) return 2;
+        piv[c] = p;
+        if (p != c) std::swap_ranges(&a[(size_t)p * m + c], &a[(size_t)p * m] + m, &a[(size_t)c * m + c]);
+        for (int k = c + 1; k < m; k++) {
+            if (a[(size_t)c * m + k] != 0.0) right(c)[nright[c]++] = k;
+            if (a[(size_t)k * m + c] != 0.0) below(c)[nbelow[c]++] = k;
+        }
+        for (int q = 0; q < nbelow[c]; q++) {
+            const int i = below(c)[q];
+            const double f = a[(size_t)i * m + c] /= a[(size_t)c * m + c];
+            for (int u = 0; u < nright[c]; u++) a[(size_t)i * m + right(c)[u]] -= f * a[(size_t)c * m + right(c)[u]];
+        }
+    }
+    // m right-hand sides; row i of b has entries in [lo[i], hi[i]) only (they
+    // decay away from the diagonal, and those below 1e-30 are dropped: the
+    // reduced systems' windows end at 1e-18, and products of smaller ones are
+    // subnormal, some hundred cycles each)
+    std::vector<int> lo(m), hi(m);
+    auto trim = [&](std::vector<double> &b, int i) {
+        auto small = [&](int j) { return std::fabs(b[(size_t)i * m + j]) < 1e-30; };
+        for (; lo[i] < hi[i] && small(lo[i]); lo[i]++) b[(size_t)i * m + lo[i]] = 0.0;
+        for (; lo[i] < hi[i] && small(hi[i] - 1); hi[i]--) b[(size_t)i * m + hi[i] - 1] = 0.0;
+    };
+    auto solve = [&](std::vector<double> &b) {
+        auto sub = [&](int i, double f, int k) {
+            lo[i] = std::min(lo[i], lo[k]);
+            hi[i] = std::max(hi[i], hi[k]);
+            double *__restrict__ d = &b[(size_t)i * m];
+            const double *__restrict__ s = &b[(size_t)k * m];
+            for (int j = lo[k]; j < hi[k]; j++) d[j] -= f * s[j];
+        };
+        for (int c = 0; c < m; c++) {
+            if (piv[c] != c) {
+                std::swap_ranges(&b[(size_t)c * m], &b[(size_t)c * m] + m, &b[(size_t)piv[c] * m]);
+                std::swap(lo[c], lo[piv[c]]);
+                std::swap(hi[c], hi[piv[c]]);
+            }
+            trim(b, c);
+            for (int q = 0; q < nbelow[c]; q++) sub(below(c)[q], a[(size_t)below(c)[q] * m + c], c);
+        }
+        for (int c = m - 1; c >= 0; c--) {
+            for (int q = 0; q < nright[c]; q++) sub(c, a[(size_t)c * m + right(c)[q]], right(c)[q]);
+            const double d = 1.0 / a[(size_t)c * m + c];
+            for (int j = lo[c]; j < hi[c]; j++) b[(size_t)c * m + j] *= d;
+            trim(b, c);
+        }
+    };
+    for (int i = 0; i < m; i++) {
+        x[(size_t)i * m + i] = 1.0;
+        lo[i] = i;
+        hi[i] = i + 1;
+    }
+    solve(x);
+    std::vector<int> nz;
+    std::vector<int> xlo(lo), xhi(hi);
+    for (int i = 0; i < m; i++) {
+        nz.clear();
+        lo[i] = i;
+        hi[i] = i + 1;
+        for (int k = 0; k < m; k++)
+            if (r[(size_t)i * m + k] != 0.0) {
+                nz.push_back(k);
+                lo[i] = std::min(lo[i], xlo[k]);
+                hi[i] = std::max(hi[i], xhi[k]);
+            }
+        for (int j = lo[i]; j < hi[i]; j++) {
+            long double s = i == j ? 1.0 : 0.0;
+            for (int k : nz) s -= r[(size_t)i * m + k] * x[(size_t)k * m + j];
+            e[(size_t)i * m + j] = (double)s;
+        }
+        trim(e, i);
+    }
+    solve(e);
+    for (size_t k = 0; k < x.size(); k++) r[k] = (long double)x[k] + e[k];
+    return 0;
+}
 
 // The factors of P partitions of M slots: partition p holds rows start(p) ..
-// start(p) + rows(p) - 1 in its first slots.
-template <typename Start, typename Rows>
-int factor_parts(const OpMatrices &op, int M, int P, Start start, Rows rows, SpikeFactors &out)
+// start(p) + rows(p) - 1 in its first slots.  Computed in Real, stored in
+// double.
+template <typename Real, typename Start, typename Rows>
+int factor_parts(const OpMatrices &op, int M, int P, Start start, Rows rows, std::vector<PartFactors> &known,
+                 SpikeFactors &out)
 {
     const int n = op.n;
     out = SpikeFactors();
@@ -738,38 +831,56 @@ int factor_parts(const OpMatrices &op, int M, int P, Start start, Rows rows, Spi
     out.lu.assign((size_t)P * M * 5, 0.0);
     out.S.assign((size_t)P * M * 4, 0.0);
     out.Q.assign((size_t)P * 4 * 4 * P, 0.0);
-    std::vector<double> col(M);
+    const int trow[4] = {0, 1, M - 2, M - 1};           // slots of the tips
+    std::vector<Real> lu((size_t)M * 5), col(M), tips((size_t)P * 16);   // tips: S at trow
     for (int p = 0; p < P; p++) {
-        double *lu = &out.lu[(size_t)p * M * 5];
         const int mp = rows(p);
-        if (int rc = band_lu_block(op, start(p), mp, M, lu)) return rc;
-        // coupling columns: rows of this block that reference columns outside it
-        for (int c = 0; c < 4; c++) {
-            std::fill(col.begin(), col.end(), 0.0);
-            bool any = false;
-            for (int t = 0; t < mp; t++) {
-                const int i = start(p) + t;
-                for (int o = -2; o <= 2; o++) {
-                    const int tt = t + o;
-                    if (tt >= 0 && tt < mp) continue;
-                    const double v = op.band[(size_t)i * 5 + o + 2];
-                    if (v == 0.0) continue;
-                    // tt = -2,-1 -> tail of left neighbour (c = 0,1);
-                    // tt = rows, rows+1 -> head of right neighbour (c = 2,3)
-                    const int cc = tt < 0 ? tt + 2 : 2 + (tt - mp);
-                    if (cc == c) { col[t] += v; any = true; }
+        const double *band = &op.band[(size_t)start(p) * 5];
+        // partitions with the same rows of A have the same factors
+        auto kn = std::find_if(known.begin(), known.end(), [&](const PartFactors &k) {
+            return k.M == M && (int)k.band.size() == 5 * mp && std::equal(k.band.begin(), k.band.end(), band);
+        });
+        if (kn == known.end()) {
+            PartFactors k;
+            k.M = M;
+            k.band.assign(band, band + 5 * mp);
+            k.S.assign((size_t)M * 4, 0.0);
+            if (int rc = band_lu_block(op, start(p), mp, M, lu.data())) return rc;
+            k.lu.assign(lu.begin(), lu.end());
+            // coupling columns: rows of this block that reference columns outside it
+            for (int c = 0; c < 4; c++) {
+                std::fill(col.begin(), col.end(), Real(0));
+                bool any = false;
+                for (int t = 0; t < mp; t++) {
+                    if (t == 2 && mp > 4) t = mp - 2;      // the first and last two reach outside
+                    for (int o = -2; o <= 2; o++) {
+                        const int tt = t + o;
+                        if (tt >= 0 && tt < mp) continue;
+                        const double v = band[(size_t)t * 5 + o + 2];
+                        if (v == 0.0) continue;
+                        // tt = -2,-1 -> tail of left neighbour (c = 0,1);
+                        // tt = rows, rows+1 -> head of right neighbour (c = 2,3)
+                        const int cc = tt < 0 ? tt + 2 : 2 + (tt - mp);
+                        if (cc == c) { col[t] += v; any = true; }
+                    }
                 }
+                if (!any) continue;
+                band_lu_solve(lu.data(), M, col.data());
+                for (int t = 0; t < M; t++) k.S[(size_t)t * 4 + c] = (double)col[t];
+                for (int q = 0; q < 4; q++) k.tips[4 * q + c] = col[trow[q]];
             }
-            if (any) band_lu_solve(lu, M, col.data());
-            for (int t = 0; t < M; t++) out.S[((size_t)p * M + t) * 4 + c] = any ? col[t] : 0.0;
+            kn = known.insert(known.end(), std::move(k));
         }
+        std::copy(kn->lu.begin(), kn->lu.end(), &out.lu[(size_t)p * M * 5]);
+        std::copy(kn->S.begin(), kn->S.end(), &out.S[(size_t)p * M * 4]);
+        std::copy(kn->tips, kn->tips + 16, &tips[(size_t)p * 16]);
     }
     if (!op.periodic && P == 1) return 0;
     // reduced system over the tips: unknown 4q + k, k = 0,1 head slots (0,1),
     // k = 2,3 tail slots (M-2, M-1), which hold the last two rows, exchanged
     // when the partition has an odd number of padding slots
     const int m = 4 * P;
-    std::vector<double> R((size_t)m * m, 0.0);
+    std::vector<Real> R((size_t)m * m, Real(0));
     auto nbr_index = [&](int p, int c) -> int {
         if (c < 2) {
             int q = p - 1;
@@ -780,7 +891,6 @@ int factor_parts(const OpMatrices &op, int M, int P, Start start, Rows rows, Spi
         if (q >= P) { if (!op.periodic) return -1; q -= P; }
         return 4 * q + (c - 2);
     };
-    const int trow[4] = {0, 1, M - 2, M - 1};
     for (int p = 0; p < P; p++)
         for (int k = 0; k < 4; k++) {
             const int r = 4 * p + k;
@@ -788,7 +898,7 @@ int factor_parts(const OpMatrices &op, int M, int P, Start start, Rows rows, Spi
             for (int c = 0; c < 4; c++) {
                 const int j = nbr_index(p, c);
                 if (j < 0) continue;
-                R[(size_t)r * m + j] += out.S[((size_t)p * M + trow[k]) * 4 + c];
+                R[(size_t)r * m + j] += tips[(size_t)p * 16 + 4 * k + c];
             }
         }
     if (int rc = invert(R, m)) return rc;
@@ -796,7 +906,7 @@ int factor_parts(const OpMatrices &op, int M, int P, Start start, Rows rows, Spi
         for (int c = 0; c < 4; c++) {
             const int j = nbr_index(p, c);
             for (int k = 0; k < m; k++)
-                out.Q[((size_t)p * 4 + c) * m + k] = j < 0 ? 0.0 : R[(size_t)j * m + k];
+                out.Q[((size_t)p * 4 + c) * m + k] = j < 0 ? 0.0 : (double)R[(size_t)j * m + k];
         }
     return 0;
 }
@@ -810,7 +920,8 @@ int spike_factor(const OpMatrices &op, int M, SpikeFactors &out)
     // operators on n = 5..7 cells)
     const bool whole_bounded = !op.periodic && M == op.n && op.n >= 4;
     if ((M < 8 && !whole_bounded) || op.n % M != 0) return 1;
-    return factor_parts(op, M, op.n / M, [&](int p) { return p * M; }, [&](int) { return M; }, out);
+    std::vector<PartFactors> known;
+    return factor_parts<double>(op, M, op.n / M, [&](int p) { return p * M; }, [&](int) { return M; }, known, out);
 }
 
 bool uneven_parts(int n, int M, UnevenParts &out)
@@ -836,10 +947,17 @@ bool uneven_parts(int n, int M, UnevenParts &out)
     return out.P <= (M == 64 ? 21 : 16) && out.base >= 8;
 }
 
-int spike_factor_uneven(const OpMatrices &op, const UnevenParts &u, SpikeFactors &out)
+int spike_factor_uneven(const OpMatrices &op, const UnevenParts &u, std::vector<PartFactors> &known, SpikeFactors &out)
 {
     if (op.n != u.n || u.P < 2) return 1;
-    return factor_parts(op, u.M, u.P, [&](int p) { return u.start(p); }, [&](int p) { return u.rows(p); }, out);
+    // In 80-bit arithmetic, each entry rounded once: otherwise the tables
+    // alone set the FP64 kernels' error on these lengths (white noise, root
+    // mean square over the largest output, against 64-bit mantissas: cd10 d2,
+    // n = 321, codes (1, -1), 6.0e-17 with tables from 64-bit arithmetic and
+    // 3.5e-17 with these, 3.5e-17 as one partition; cf90, n = 129, periodic,
+    // 1.2e-14, 1.06e-14 and 1.0e-14).
+    return factor_parts<long double>(op, u.M, u.P, [&](int p) { return u.start(p); }, [&](int p) { return u.rows(p); },
+                                     known, out);
 }
 
 int dense_operator(const OpMatrices &op, std::vector<double> &D)

@@ -112,8 +112,17 @@ void transpose_operator(const OpMatrices &fwd, OpMatrices &adj);
 
 // Factor A for a partitioned solve with partition size M (n % M == 0).
 int spike_factor(const OpMatrices &op, int M, SpikeFactors &out);
+// Factors of one partition of M slots, with the rows of A that they belong to.
+struct PartFactors {
+    int M = 0;
+    std::vector<double> band, lu, S;
+    long double tips[16] = {0};   // S at the tip slots, before rounding
+};
 // The same over uneven partitions; lu, S and Q are per slot (P * M of them).
-int spike_factor_uneven(const OpMatrices &op, const UnevenParts &parts, SpikeFactors &out);
+// `known`: partitions factored before (an operator's plans differ at the ends
+// of the pencil only), extended by the new ones.
+int spike_factor_uneven(const OpMatrices &op, const UnevenParts &parts, std::vector<PartFactors> &known,
+                        SpikeFactors &out);
 
 // Error code init() returns for this size (0 ok, 2/3/7 as the reference).
 int init_error(int kind, int n, bool periodic);

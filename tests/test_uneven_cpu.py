@@ -153,3 +153,44 @@ def test_variant_choice():
     assert pv(23, 1, 64, 64)["generic"] and pv(1345, 1, 64, 64)["generic"]
     assert pv(1025, 1, 64, 64)["PW"] == 4 and pv(1344, 2, 64, 64)["PW"] == 4 and pv(1024, 3, 64, 64)["PW"] == 2
     assert _lib.plan_variant(PADE_CF90, PADE_FILTER, 272, 1.0, False, 3, 64, 64)["uneven"]
+
+
+def extended(A, b):
+    """A^-1 b to the 64-bit mantissas of long double, by refinement."""
+    x = np.linalg.solve(A, b.astype(float)).astype(np.longdouble)
+    for _ in range(3):
+        x += np.linalg.solve(A, (b - A.astype(np.longdouble) @ x).astype(float))
+    return x
+
+
+def rms_error(kind, which, n, periodic, bc, adj, M, v, ref):
+    """Of the kernels' arithmetic in 64 bits; M = n: one partition."""
+    dx, k, o = 0.3 if which != "filter" else 1.0, se.KIND[kind], se.OPER[which]
+    tab, m = (se.export(kind, which, n, dx, periodic, *bc, adj, n) if M == n
+              else export(k, o, n, dx, periodic, *bc, adj, M))
+    run = se._solve if M == n else solve
+    pad, sq = "wrap" if periodic else "clamp", 0.0
+    for j in range(v.shape[1]):
+        y = (se._stencil(tab, m, run(tab, m, v[:, j]), pad) if adj and not periodic
+             else run(tab, m, se._stencil(tab, m, v[:, j].copy(), pad)))
+        sq += float(((y - ref[:, j]) ** 2).sum())
+    return sq ** 0.5
+
+
+@pytest.mark.parametrize("kind,which,periodic,bc,adj", [
+    ("cd10", "d1", True, (0, 0), False), ("cd10", "d1", False, (1, -1), False), ("cd10", "d2", False, (1, -1), False),
+    ("cd10", "d2", False, (1, -1), True), ("cd06", "d1", False, (0, 0), False), ("cf90", "filter", True, (0, 0), False),
+    ("cf90", "filter", False, (0, 0), False)])
+@pytest.mark.parametrize("n,M", [(65, 32), (129, 32), (321, 48)])
+def test_error_is_that_of_one_partition(kind, which, periodic, bc, adj, n, M):
+    """FP64 against long double: the partitioned solve adds one rounding per
+    value (the correction) to the five or more of the stencil and the two
+    sweeps, a tenth in the root mean square; with the sampling error of a few
+    thousand correlated values, less than 1.2 times one partition's error."""
+    A, B = (x.astype(float) for x in pd.assemble(kind, which, n, 0.3 if which != "filter" else 1.0, periodic, *bc)[:2])
+    v = np.random.default_rng(n).standard_normal((n, 48))
+    vl, Bl = v.astype(np.longdouble), B.astype(np.longdouble)
+    ref = Bl.T @ extended(A.T, vl) if adj else extended(A, Bl @ vl)
+    one = rms_error(kind, which, n, periodic, bc, adj, n, v, ref)
+    parts = rms_error(kind, which, n, periodic, bc, adj, M, v, ref)
+    assert parts < 1.2 * one, parts / one
