@@ -229,7 +229,15 @@ constexpr int kFilterRhsBc = 100 + pade::FILTER;
 
 // Partition sizes of the register path that serve this operator: those that
 // divide its rows, or else the uneven splits.
-void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double> &tab,
+// The bounded cf90 adjoint (inverse: A^-T before B^T) takes no uneven split
+// that is less exact than what else serves the length: A is nearly singular at
+// the shortest wave, which only B^T removes, so what a partition's ends add to
+// its rounding stays (white noise, root mean square over the largest output,
+// FP64 / FP32: n = 129 as one partition 6.0e-15 / 2.8e-6, in 32 slots 1.0e-14
+// / 5.9e-6; n = 320 in 64 rows 8.6e-15 / 4.4e-6, in 40 slots 1.04e-14 /
+// 4.8e-6; but n = 176 in 16 rows 1.8e-14 / 6.8e-6, in 32 slots 1.0e-14 /
+// 5.3e-6).
+void add_spike_variants(const pade::OpMatrices &m, bool adj, bool inverse, std::vector<double> &tab,
                         std::vector<pade::PartFactors> &known, Plan &pl)
 {
     // special rows the kernels hold
@@ -250,6 +258,7 @@ void add_spike_variants(const pade::OpMatrices &m, bool adj, std::vector<double>
     }
     if (!pl.spike.empty() && !(n % 32 == 16 && n >= 144) && !mid) return;
     const bool none = pl.spike.empty();
+    if (inverse && (none || n % 64 == 0)) return;
     for (int M : {16, 24, 32, 40, 48, 64}) {
         pade::UnevenParts parts;
         Variant v;
@@ -284,7 +293,7 @@ int build_plan(int kind, int oper, int n, double dx, bool periodic, int bc1, int
         if (int rc = pade::build_stagg_system(oper, n, dx, bc1, bcn, sys)) return fail(rc, "operator construction failed");
     }
     const pade::OpMatrices &pm = sys_form ? sys : pl.mats;
-    add_spike_variants(pm, adj, tab, known, pl);
+    add_spike_variants(pm, adj, kind == pade::CF90 && adj && !periodic, tab, known, pl);
     if (m >= 4 && build_variant(pl.mats, m, tab, pl.generic) == 0) pl.has_generic = true;
     return 0;
 }
@@ -331,7 +340,7 @@ int build_all_plans(pade_op_s *op)
             if (int rc = operator_matrices(op->kind, pade::FILTER, op->n, op->dx, false, b1, bn, false, pl.mats))
                 return fail(rc, "operator construction failed");
             pl.mats.band = nn.band;      // (bc1, bcn) right-hand side, (0, 0) left-hand side
-            add_spike_variants(pl.mats, false, tab, known, pl);
+            add_spike_variants(pl.mats, false, false, tab, known, pl);
             if (op->n >= 4 && build_variant(pl.mats, op->n, tab, pl.generic) == 0) pl.has_generic = true;
             op->plans[{kFilterRhsBc, b1, bn, 0}] = std::move(pl);
         }

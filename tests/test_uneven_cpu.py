@@ -194,3 +194,20 @@ def test_error_is_that_of_one_partition(kind, which, periodic, bc, adj, n, M):
     one = rms_error(kind, which, n, periodic, bc, adj, n, v, ref)
     parts = rms_error(kind, which, n, periodic, bc, adj, M, v, ref)
     assert parts < 1.2 * one, parts / one
+
+
+def test_bounded_cf90_adjoint_keeps_the_more_exact_form():
+    """Lengths that no partition size divides, and those that 64 divides, run
+    the bounded cf90 adjoint as before uneven partitions, on every axis; the
+    forward filter and the other adjoints take them."""
+    def pv(n, axis, adjoint, kind=PADE_CF90, oper=PADE_FILTER, periodic=False, dtype=_lib.PADE_F64):
+        return _lib.plan_variant(kind, oper, n, 0.1, periodic, axis, 200, 200, adjoint=adjoint, dtype=dtype)
+    for axis in (1, 2, 3):
+        for dtype in (_lib.PADE_F64, _lib.PADE_F32):
+            for n in (25, 39, 65, 129, 257, 321, 700, 1025):
+                assert pv(n, axis, True, dtype=dtype)["generic"] and pv(n, axis, False, dtype=dtype)["uneven"]
+                assert pv(n, axis, True, PADE_CD10, PADE_D1, dtype=dtype)["uneven"]
+                assert pv(n, axis, True, periodic=True, dtype=dtype)["uneven"]
+            for n in (320, 384):
+                v = pv(n, axis, True, dtype=dtype)
+                assert v["M"] == 64 and not v["uneven"] and not v["generic"]
