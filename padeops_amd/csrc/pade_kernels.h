@@ -58,8 +58,9 @@ struct FieldArgs {
 
 constexpr int kMaxFields = 6;
 
+// What the fields of a launch share.
 template <typename T>
-struct ApplyArgs {
+struct SolveArgs {
     int nfields;           // grid y
     long long npencils;
     long long A1, B1, B2;  // pencil q -> base offset (q % A1)*B1 + (q / A1)*B2
@@ -79,7 +80,10 @@ struct ApplyArgs {
                            // consecutive workgroups; < 0 a contiguous eighth
     T alpha, beta;
     T stage_dt, stage_a, stage_b;
-    // last, so that a launch of one field reads one stretch of arguments
+};
+
+template <typename T>
+struct ApplyArgs : SolveArgs<T> {
     FieldArgs<T> fld[kMaxFields];
 };
 
@@ -88,6 +92,10 @@ struct ApplyArgs {
 // GW: whole-pencil x waves (PW = 8) per workgroup (other variants: 1).
 template <typename T>
 hipError_t launch_spike(const ApplyArgs<T> &a, int M, int PW, int GW, bool adj, int mode, hipStream_t s);
+
+// launch_spike of several fields: forward, modes 0 and 1, two partitions per
+// wave or whole-pencil x waves (FP64).
+hipError_t launch_fields(const ApplyArgs<double> &a, int M, int PW, int GW, int mode, hipStream_t s);
 
 // The same solve over uneven partitions (a pencil length that is no multiple
 // of M), two partitions per wave; modes as above.

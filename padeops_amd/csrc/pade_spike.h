@@ -260,12 +260,25 @@ __device__ __forceinline__ void apply_stencil(T (&w)[M + 8], const T *__restrict
     }
 }
 
+// The fields of a launch, grid y.  A launch of one field has a kernel of its
+// own (NF = 1), whose arguments are all at known places: a struct indexed by
+// the field stays in memory as a whole, so it is an argument beside the others
+// (one struct for both: FP64 x, M = 32, periodic, 132 registers instead of 128,
+// three waves per SIMD instead of four), and the dependent read of its entries
+// stands before the first load of every workgroup (FP64 cd06 64^3 x / z 5.7 /
+// 5.6 us indexed, 5.5 / 5.3 not; cd10 512^3 z 421.9 and 417.4, FP32 x 187.5 and
+// 186.0).
+template <typename T, int NF>
+struct FieldSet {
+    FieldArgs<T> fld[NF];
+};
+
 template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, int EPI, bool UNE = false, int ROWS = kWholeLines,
-          int REP = 1>
-__global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
+          int REP = 1, int NF = 1>
+__global__ __launch_bounds__(512) void spike_apply(SolveArgs<T> a, FieldSet<T, NF> fields)
 {
     constexpr int NPEN = 64 / PW;
-    const FieldArgs<T> &fd = a.fld[blockIdx.y];
+    const FieldArgs<T> &fd = fields.fld[NF > 1 ? blockIdx.y : 0];
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T *smem = reinterpret_cast<T *>(smem_raw);
     constexpr bool WHOLE = MODE == 1 && PW == 8;
@@ -421,19 +434,30 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
         // -> 329-331 / 312 Gpts/s; on periodic ones no gain on y, z 323.5 ->
         // 313 with them)
         if constexpr (!ADJ) {
-#pragma unroll
-            for (int t = 4; t < M + 4; t++) w[t] = ld_s<BND && ROWS == kWholeLines>(fb + (long long)(pw0 - 4 + t) * stp, active ? hoff : loff);
             // halo rows (wrapped per partition, or clamped at the ends of a
             // bounded pencil, where the boundary rows replace the stencil)
-            const T *fq = fd.f + base0 + (long long)(loff / sizeof(T));
+            auto load_halo = [&] {
+                const T *fq = fd.f + base0 + (long long)(loff / sizeof(T));
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int jl = wrap_index(pM - 4 + k, n, !BND);
-                // a staggered operator's input may hold one point more than its rows
-                const int jr = wrap_index(pM + M + k, MODE == 2 ? a.n_in : n, !BND);
-                w[k] = fq[(long long)jl * stp];
-                w[M + 4 + k] = fq[(long long)jr * stp];
+                for (int k = 0; k < 4; k++) {
+                    const int jl = wrap_index(pM - 4 + k, n, !BND);
+                    // a staggered operator's input may hold one point more than its rows
+                    const int jr = wrap_index(pM + M + k, MODE == 2 ? a.n_in : n, !BND);
+                    w[k] = fq[(long long)jl * stp];
+                    w[M + 4 + k] = fq[(long long)jr * stp];
+                }
+            };
+            // (before the main rows on periodic FP32 pencils: 512^3 y / z 223.4
+            // / 228.7 -> 218.9 / 221.6 us, 222.0 / 222.7 as the compiler ordered
+            // them before the kernel served several fields)
+            constexpr bool HALO_FIRST = sizeof(T) == 4 && !BND && EPI == kStore;
+            if constexpr (HALO_FIRST) {
+                load_halo();
+                mem_region_fence();
             }
+#pragma unroll
+            for (int t = 4; t < M + 4; t++) w[t] = ld_s<BND && ROWS == kWholeLines>(fb + (long long)(pw0 - 4 + t) * stp, active ? hoff : loff);
+            if constexpr (!HALO_FIRST) load_halo();
         } else {
 #pragma unroll
             for (int t = 0; t < M; t++) w[t] = ld_s<BND && ROWS == kWholeLines>(fb + (long long)(pw0 + t) * stp, active ? hoff : loff);
@@ -620,9 +644,13 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
         }
     }
     // REP > 1: the operator applied REP times, the intermediate never leaving
-    // the registers (halos through LDS as in the adjoint)
+    // the registers (halos through LDS as in the adjoint).  (REP = 1: left at
+    // the end, no loop.  As a loop of one pass some kernels took four registers
+    // more, FP32 M = 64 system form accumulating 131 instead of 127; the stage
+    // takes two less as one.)
+    constexpr bool ONCE = REP == 1 && EPI != kStage;
 #pragma unroll 1
-    for (int rep = 0; rep < REP; rep++) {
+    for (int rep = 0; ONCE || rep < REP; rep++) {
     if constexpr (!ADJ) apply_stencil<T, M, MODE == 2 ? kBRowsSys : kBRowsFwd, MODE == 2 ? 1 : 0>(w, tab, bnd, edge_left, edge_right, fd.nbl, fd.nbr);
     // the padding slots of an uneven partition have a zero right-hand side
     if constexpr (UNE) {
@@ -750,6 +778,7 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
             if (exch) __syncthreads();
         if constexpr (ADJ) apply_stencil<T, M, kBRowsDev>(w, tab, bnd, edge_left, edge_right, fd.nbl, fd.nbr);
     }
+    if (ONCE) break;
     }
 
     // ---------------------------------------------------------------- store
@@ -873,12 +902,21 @@ __global__ __launch_bounds__(512) void spike_apply(ApplyArgs<T> a)
         // accumulate: a chunk's old values are loaded together, the next
         // chunk's before the current one is stored (a memory round trip per
         // chunk, overlapped with the previous chunk's stores; nontemporal
-        // loads, as on strided rows: 512^3 FP64 596 -> 545 us)
+        // loads, as on strided rows: 512^3 FP64 596 -> 545 us).  Rows that do
+        // not exist load the first one's: with conditional loads, partitions
+        // of one chunk (FP64 M = 16, FP32 M = 32) needed 230 registers, with
+        // these 96 to 117 (whole-pencil waves of more chunks the other way
+        // round: FP64 M = 48 182 and 166).
         vec_t cur[EPI ? XT / VL : 1], nxt[EPI ? XT / VL : 1];
         auto load_old = [&](int c, vec_t *o) {
 #pragma unroll
             for (int s = 0; s < XT / VL; s++)
-                if (row_ok(s)) o[s] = STREAM ? ldg_nt(ob + pw0 + c * XT, row_off(s)) : ldg(ob + pw0 + c * XT, row_off(s));
+            {
+                const bool ok = row_ok(s);
+                if (WHOLE && M > XT && !ok) continue;
+                const unsigned ro = ok ? row_off(s) : 0u;
+                o[s] = STREAM ? ldg_nt(ob + pw0 + c * XT, ro) : ldg(ob + pw0 + c * XT, ro);
+            }
         };
         if constexpr (EPI) load_old(0, cur);
 #pragma unroll
@@ -964,20 +1002,24 @@ RowLayout row_layout(const ApplyArgs<T> &a)
 // Workgroups per XCD run where neighbouring workgroups share lines.
 constexpr int kSharedRun = 64;
 
-template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, int EPI, bool UNE, int REP>
+template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, int EPI, bool UNE, int REP, int NF>
 hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
 {
     constexpr int NPEN = 64 / PW;
     constexpr bool WHOLE = MODE == 1 && PW == 8;
-    ApplyArgs<T> a = a_in;
+    if (a_in.nfields < 1 || a_in.nfields > NF) return hipErrorInvalidValue;
+    SolveArgs<T> a = a_in;
+    FieldSet<T, NF> fields;
+    std::copy_n(a_in.fld, NF, fields.fld);
     const int waves = WHOLE ? gw : (a.P + PW - 1) / PW;
     int coef_len = 0;
-    for (int k = 0; k < a.nfields; k++) coef_len = std::max(coef_len, a.fld[k].coef_len);
+    for (int k = 0; k < a.nfields; k++) coef_len = std::max(coef_len, fields.fld[k].coef_len);
     const size_t lds = spike_lds_bytes(sizeof(T), M, a.P, PW, ADJ || REP > 1, MODE, coef_len, BND, gw);
     const long long nblk = (a.npencils + (long long)NPEN * gw - 1) / ((long long)NPEN * gw);
     a.remap = 0;
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)nblk, (unsigned)a.nfields), dim3(64 * waves), lds, s, a);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nblk, (unsigned)a.nfields), dim3(64 * waves), lds, s,
+                           a, fields);
         return hipGetLastError();
     };
     if constexpr (MODE == 1) {
@@ -994,46 +1036,49 @@ hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
         // uneven x partitions may start anywhere in a line: cached stores, as
         // for strided rows (129 x 512 x 512 FP64 x 155 -> 229 Gpts/s)
         if constexpr (UNE) {
-            const auto bits = field_bits(a) | (uintptr_t)(a.n * sizeof(T)) |
+            const auto bits = field_bits(a_in) | (uintptr_t)(a.n * sizeof(T)) |
                               (uintptr_t)(a.uunit * sizeof(T));
-            if (bits % 128) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared, REP>);
+            if (bits % 128) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared, REP, NF>);
         }
-        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines, REP>);
+        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines, REP, NF>);
     } else {
-        const RowLayout rows = row_layout(a);
-        if (rows == kWholeLines) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines, REP>);
+        const RowLayout rows = row_layout(a_in);
+        if (rows == kWholeLines) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kWholeLines, REP, NF>);
         int c = kSharedRun;
         while (c > 1 && nblk < 16LL * c) c /= 2;
         if (c >= 2) a.remap = c;
-        if (rows == kShared) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared, REP>);
+        if (rows == kShared) return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, kShared, REP, NF>);
         // without an epilogue periodic kernels load alike for whole and half lines
-        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, (BND || EPI ? kHalfLines : kWholeLines), REP>);
+        return launch(spike_apply<T, M, PW, ADJ, MODE, BND, EPI, UNE, (BND || EPI ? kHalfLines : kWholeLines), REP, NF>);
     }
 }
 
-template <typename T, int M, int PW, bool ADJ, int MODE, bool UNE = false, int REP = 1>
+template <typename T, int M, int PW, bool ADJ, int MODE, bool UNE = false, int REP = 1,
+          int NF = sizeof(T) == 8 && !ADJ && MODE != 2 && (UNE || REP > 1) ? kMaxFields : 1>
 hipError_t launch_spike_t(const ApplyArgs<T> &a, int gw, hipStream_t s)
 {
     constexpr bool WHOLE = MODE == 1 && PW == 8;
-    if (!WHOLE) gw = 1;
+    // whole-pencil waves: no wave of a workgroup without pencils (its loads
+    // would start behind the field)
+    while (gw > 1 && (!WHOLE || (a.npencils + 7) / 8 % gw)) gw--;
     // the accumulate epilogue exists for the forward operator only
     if (ADJ && a.axpby) return hipErrorInvalidValue;
     const bool epi = !ADJ && a.axpby;
     if constexpr (MODE == 2) {
         // staggered operators: forward, bounded, strided rows only
         if (ADJ || a.periodic || a.n_in < a.n || a.n_in > a.n + 1) return hipErrorInvalidValue;
-        return epi ? launch_kernel<T, M, PW, false, 2, true, kAxpby, UNE, REP>(a, gw, s)
-                   : launch_kernel<T, M, PW, false, 2, true, kStore, UNE, REP>(a, gw, s);
+        return epi ? launch_kernel<T, M, PW, false, 2, true, kAxpby, UNE, REP, NF>(a, gw, s)
+                   : launch_kernel<T, M, PW, false, 2, true, kStore, UNE, REP, NF>(a, gw, s);
     } else if constexpr (ADJ) {
         // (a periodic adjoint runs the forward kernel on the transposed tables)
         if (a.periodic) return hipErrorInvalidValue;
-        return launch_kernel<T, M, PW, true, MODE, true, kStore, UNE, REP>(a, gw, s);
+        return launch_kernel<T, M, PW, true, MODE, true, kStore, UNE, REP, NF>(a, gw, s);
     } else {
         if (a.periodic)
-            return epi ? launch_kernel<T, M, PW, false, MODE, false, kAxpby, UNE, REP>(a, gw, s)
-                       : launch_kernel<T, M, PW, false, MODE, false, kStore, UNE, REP>(a, gw, s);
-        return epi ? launch_kernel<T, M, PW, false, MODE, true, kAxpby, UNE, REP>(a, gw, s)
-                   : launch_kernel<T, M, PW, false, MODE, true, kStore, UNE, REP>(a, gw, s);
+            return epi ? launch_kernel<T, M, PW, false, MODE, false, kAxpby, UNE, REP, NF>(a, gw, s)
+                       : launch_kernel<T, M, PW, false, MODE, false, kStore, UNE, REP, NF>(a, gw, s);
+        return epi ? launch_kernel<T, M, PW, false, MODE, true, kAxpby, UNE, REP, NF>(a, gw, s)
+                   : launch_kernel<T, M, PW, false, MODE, true, kStore, UNE, REP, NF>(a, gw, s);
     }
 }
 

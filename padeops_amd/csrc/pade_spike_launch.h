@@ -57,8 +57,8 @@ hipError_t launch_spike(const ApplyArgs<T> &a, int M, int PW, int GW, bool adj, 
     // line of FP64 per partition row)
     if (PW == 4 && mode == 0) {
         switch (M) {
-        case 32: return launch_spike_mp<T, 32, 4>(a, adj, mode, s);
-        case 64: return launch_spike_mp<T, 64, 4>(a, adj, mode, s);
+        case 32: return adj ? launch_spike_t<T, 32, 4, true, 0>(a, 1, s) : launch_spike_t<T, 32, 4, false, 0>(a, 1, s);
+        case 64: return adj ? launch_spike_t<T, 64, 4, true, 0>(a, 1, s) : launch_spike_t<T, 64, 4, false, 0>(a, 1, s);
         default: return hipErrorInvalidValue;
         }
     }

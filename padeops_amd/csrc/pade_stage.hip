@@ -9,8 +9,8 @@ namespace pade {
 template <int M, bool UNE>
 static hipError_t stage_m(const ApplyArgs<double> &a, hipStream_t s)
 {
-    return a.periodic ? launch_kernel<double, M, 2, false, 0, false, kStage, UNE, 1>(a, 1, s)
-                      : launch_kernel<double, M, 2, false, 0, true, kStage, UNE, 1>(a, 1, s);
+    return a.periodic ? launch_kernel<double, M, 2, false, 0, false, kStage, UNE, 1, kMaxFields>(a, 1, s)
+                      : launch_kernel<double, M, 2, false, 0, true, kStage, UNE, 1, kMaxFields>(a, 1, s);
 }
 
 hipError_t launch_stage(const ApplyArgs<double> &a, int M, bool uneven, hipStream_t s)
