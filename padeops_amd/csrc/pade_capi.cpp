@@ -714,11 +714,12 @@ int apply_one(pade_op_t op, const Plan &pl, int axis, const T *f, T *df, int na,
     return 0;
 }
 
-// Does one launch apply this operator twice?
+// Does one launch apply this operator twice?  (Whole-pencil x waves, which a
+// bounded pencil runs by request only, have no adjoint form.)
 template <typename T>
-bool twice_ok(const LaunchPlan<T> &L)
+bool twice_ok(const LaunchPlan<T> &L, bool adj)
 {
-    return std::is_same<T, double>::value && !L.generic && L.mode != 2 && (L.pw == 2 || L.pw == 8);
+    return std::is_same<T, double>::value && !L.generic && L.mode != 2 && (L.pw == 2 || (L.pw == 8 && !adj));
 }
 
 // Argument checks shared by every apply: 0 or the error code.
@@ -790,7 +791,7 @@ int apply_impl(pade_op_t op, int oper, int axis, const T *f, T *df, int na, int 
         LaunchPlan<T> L;
         if (int rc = plan_launch<T>(*p1, op->periodic, axis, f, df, na, nb, L)) return rc;
         if constexpr (std::is_same<T, double>::value) {
-            if (twice_ok(L)) {
+            if (twice_ok(L, adj)) {
                 // (the allocation-free entry point keeps its size limit, see apply_one)
                 if (ws.on && epi.on) {
                     const size_t fields = p1->even() ? 1 : 2;
@@ -1295,7 +1296,7 @@ int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *fld
             if (!pl) return 21;
             LaunchPlan<double> Lk;
             if (int rc = plan_launch<double>(*pl, op->periodic, axis, flds[k].f, flds[k].out, na, nb, Lk)) return rc;
-            one = !Lk.generic && (times == 2 ? twice_ok(Lk) : nf == 1 || Lk.v->uneven || Lk.pw == 2 || Lk.pw == 8);
+            one = !Lk.generic && (times == 2 ? twice_ok(Lk, false) : nf == 1 || Lk.v->uneven || Lk.pw == 2 || Lk.pw == 8);
             if (k == 0) L = Lk;
             else one = one && Lk.v->M == L.v->M && Lk.v->P == L.v->P && Lk.pw == L.pw && Lk.v->uneven == L.v->uneven;
             L.a.fld[k] = Lk.a.fld[0];

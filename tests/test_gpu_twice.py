@@ -8,6 +8,10 @@ passes; its grids here cover the one-launch path on even and uneven sizes and
 the one-field-at-a-time path of an axis without a partitioned kernel, viscous
 (properties added to) and inviscid (properties written), at the tolerance and
 step of the suite's other step tests."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -117,3 +121,28 @@ def test_batched_rhs_matches_oracle(shape, periodic, bc, inviscid):
     for k in range(5):
         assert rel(got[..., k], ref[..., k]) < 1e-12, k
     g.destroy()
+
+
+def test_whole_pencil_waves_by_request():
+    """PADE_SPIKE_PW=8 on bounded x pencils (read once per process): the cd06
+    second derivative and its adjoint, which has no twice-applied form."""
+    code = """
+import numpy as np, torch, padeops_amd as po
+from padeops_amd import _lib
+from oracle import pade_dense as pd
+n = 256
+assert _lib.plan_variant(1, 2, n, 0.05, False, 1, 67, 5, adjoint=True)["PW"] == 8
+op = po.cd06(); op.init(n, 0.05, False, 0, 0)
+f = po.as_fortran(torch.tensor(np.random.default_rng(3).standard_normal((n, 67, 5)), device="cuda:0"))
+D = pd.dense_operator("cd06", "d1", n, 0.05, False, 0, 0)
+for adj in (False, True):
+    out = po.fortran_empty(f.shape, device="cuda:0")
+    print("whole-pencil cd06 d2, adjoint", adj, flush=True)
+    op._apply(_lib.PADE_D2, 1, f, out, 67, 5, adjoint=adj)
+    ref = pd.apply_axis((D @ D).T if adj else D @ D, f.cpu().numpy(), 0)
+    assert np.abs(out.cpu().numpy() - ref).max() < 1e-12 * np.abs(ref).max(), adj
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, env={**os.environ, "PADE_SPIKE_PW": "8", "PYTHONPATH": root},
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
