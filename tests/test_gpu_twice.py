@@ -53,6 +53,34 @@ def test_bounded_cd06_second_derivative(n, axis):
     assert rel(out.cpu().numpy(), pd.apply_axis(D2.T, fh, axis - 1)) < 1e-12
 
 
+@pytest.mark.parametrize("n,axis,pencils", [(512, 1, (66, 63)), (512, 2, (129, 128)), (512, 3, (129, 128)),
+                                            (1024, 1, (33, 8)), (1024, 3, (33, 8)), (400, 1, (67, 5)), (400, 2, (67, 5)),
+                                            (700, 1, (67, 5)), (700, 3, (67, 5)), (1001, 1, (67, 5)), (1001, 2, (67, 5))])
+def test_bounded_cd06_second_derivative_64(n, axis, pencils):
+    """64 rows or slots per partition, even and uneven: 512 points with the
+    pencils from which these are chosen, the other lengths always."""
+    v = _lib.plan_variant(_lib.PADE_CD06, _lib.PADE_D2, n, 0.05, False, axis, *pencils)
+    assert v["M"] == 64 and v["PW"] == 2 and v["uneven"] == (n % 64 != 0), v
+    op = po.cd06()
+    assert op.init(n, 0.05, False, 0, 0) == 0
+    shape = list(pencils)
+    shape.insert(axis - 1, n)
+    f = po.as_fortran(torch.tensor(np.random.default_rng(n).standard_normal(shape), device=DEV))
+    fh = f.cpu().numpy()
+    D = pd.dense_operator("cd06", "d1", n, 0.05, False, 0, 0)
+    D2 = D @ D
+    ref = pd.apply_axis(D2, fh, axis - 1)
+    out = po.fortran_empty(f.shape, device=DEV)
+    print(f"cd06 d2 bounded, 64 per partition, n {n} axis {axis}", flush=True)
+    op._apply(_lib.PADE_D2, axis, f, out, *pencils)
+    assert rel(out.cpu().numpy(), ref) < 1e-12
+    acc = f.clone()
+    op._apply(_lib.PADE_D2, axis, f, acc, *pencils, alpha=0.5, beta=-2.0)
+    assert rel(acc.cpu().numpy(), 0.5 * ref - 2.0 * fh) < 1e-12
+    op._apply(_lib.PADE_D2, axis, f, out, *pencils, adjoint=True)
+    assert rel(out.cpu().numpy(), pd.apply_axis(D2.T, fh, axis - 1)) < 1e-12
+
+
 def _state(shape, seed):
     rng = np.random.default_rng(seed)
     h = tuple(2 * np.pi / n for n in shape)
@@ -120,6 +148,72 @@ def test_batched_rhs_matches_oracle(shape, periodic, bc, inviscid):
     got = rhs.cpu().numpy()
     for k in range(5):
         assert rel(got[..., k], ref[..., k]) < 1e-12, k
+    g.destroy()
+
+
+@pytest.mark.parametrize("shape,periodic,bc,tol", [
+    ((512, 64, 64), (True, True, True), ((0, 0),) * 3, 4e-12),          # x: whole pencils of 64 rows
+    ((1024, 16, 16), (True, True, True), ((0, 0),) * 3, 7e-12),
+    ((700, 16, 24), (True, True, True), ((0, 0),) * 3, 8e-12),          # 64 slots
+    ((16, 700, 24), (True, False, True), ((0, 0), (1, -1), (0, 0)), 2e-12),
+    ((400, 16, 700), (False, True, False), ((0, 0),) * 3, 1.5e-9)])
+def test_batched_rhs_64(shape, periodic, bc, tol):
+    """64 rows and slots per partition in the batched passes and the operators
+    applied twice.  The artificial properties' fourth derivatives amplify
+    rounding on long axes, most with walls: the bounds are ten times what the
+    oracle's right-hand sides differ by with operators from a 64-bit solve and
+    with the same refined in extended precision (512 points: between those of
+    384 and 700)."""
+    s0, h = _state(shape, sum(shape))
+    h = tuple(1.0 / (n - 1) if not p else hh for n, p, hh in zip(shape, periodic, h))
+    kw = dict(gam=1.4, Rgas=1.0, inviscid=True, mu_ref=0.01, T_ref=1.0, visc_n=0.75, Pr=0.7, periodic=periodic, bc=bc)
+    og = cg.Grid(shape, h, **kw)
+    s = og.from_p(dict(s0))
+    ref = og.rhs(og.conserved(s), s)
+    g = gcg.cgrid(*shape, *h, **kw)
+    for c in ("rho", "u", "v", "w", "p"):
+        getattr(g, c).copy_(torch.tensor(s0[c], device=DEV))
+    g.post_bc()
+    g.get_conserved()
+    rhs = po.fortran_empty((*shape, 5), device=DEV)
+    print(f"batched rhs, 64 per partition {shape} periodic {periodic}", flush=True)
+    g.getRHS(rhs)
+    got = rhs.cpu().numpy()
+    for k in range(5):
+        assert rel(got[..., k], ref[..., k]) < tol, k
+    g.destroy()
+
+
+@pytest.mark.parametrize("shape,periodic,tol", [
+    ((16, 16, 1024), (True, True, True), 2e-12), ((16, 16, 1024), (True, True, False), 1.2e-11),
+    ((16, 24, 700), (True, True, True), 2e-12), ((16, 24, 700), (True, True, False), 2e-12)])
+def test_stage_64_matches_oracle(shape, periodic, tol):
+    """The Runge-Kutta stage in the last flux derivative with 64 rows and slots
+    per partition of z.  On grids a tenth of these the oracle's step and the
+    library's are each 5e-13 to 7e-13 from extended precision (the cf90
+    filter's rounding); the largest of ten times the values is a tenth more,
+    and the two add up to less than 2e-12.  At the walls of 1024 points the
+    fourth derivatives' rounding is larger (see test_batched_rhs_64, whose rule
+    gives that bound: 1.2e-12 between the two oracles)."""
+    v = _lib.plan_variant(_lib.PADE_CD10, _lib.PADE_D1, shape[2], 0.1, periodic[2], 3, *shape[:2])
+    assert v["M"] == 64 and v["PW"] == 2, v
+    s0, h = _state(shape, sum(shape))
+    h = tuple(1.0 / (n - 1) if not p else hh for n, p, hh in zip(shape, periodic, h))
+    kw = dict(gam=1.4, Rgas=1.0, inviscid=True, periodic=periodic, bc=((0, 0),) * 3)
+    s1 = cg.Grid(shape, h, mu_ref=0.01, T_ref=1.0, visc_n=0.75, Pr=0.7, **kw).advance(s0, 1e-5)
+    g = gcg.cgrid(*shape, *h, mu_ref=0.01, T_ref=1.0, visc_n=0.75, Pr=0.7, **kw)
+    for c in ("rho", "u", "v", "w", "p"):
+        getattr(g, c).copy_(torch.tensor(s0[c], device=DEV))
+    g.post_bc()
+    g.get_conserved()
+    print(f"stage of 64 per partition {shape} periodic {periodic}", flush=True)
+    g.advance_RK45(1e-5)
+    torch.cuda.synchronize()
+    vscale = max(np.abs(s1[c]).max() for c in ("u", "v", "w"))
+    for c in ("rho", "u", "v", "w", "p", "T", "e"):
+        scale = vscale if c in ("u", "v", "w") else np.abs(s1[c]).max()
+        err = np.abs(getattr(g, c).cpu().numpy() - s1[c]).max() / scale
+        assert err < tol, (c, err)
     g.destroy()
 
 

@@ -128,3 +128,62 @@ def test_noalloc_limit_of_divided_lengths(kind, which, n, side, periodic):
                                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     assert rc == 0
     assert torch.equal(ref, out)
+
+
+# FP32 bounds: the same calls in FP64 are within 14 (cd06, cd10), 40 (the first
+# derivative twice) and 900 (cf90) rounding errors of the largest output; as
+# many of 6e-8, doubled.
+FP32_CASES = [("cd10", "d1", True, (0, 0), 2e-6), ("cd06", "d1", False, (0, 0), 2e-6), ("cd10", "d1", False, (1, -1), 2e-6),
+              ("cd06", "d2", False, (0, 0), 5e-6), ("cf90", "filter", True, (0, 0), 1.1e-4),
+              ("cf90", "filter", False, (0, 0), 1.1e-4)]
+
+
+@pytest.mark.parametrize("kind,which,periodic,bc,tol", FP32_CASES)
+@pytest.mark.parametrize("n,pencils", [(25, (67, 5)), (39, (67, 5)), (129, (67, 5)), (300, (67, 5)), (383, (150, 30)),
+                                       (701, (67, 5)), (1025, (67, 5))])
+@pytest.mark.parametrize("axis", [1, 2, 3])
+def test_uneven_fp32(kind, which, periodic, bc, tol, n, pencils, axis):
+    """Forward, accumulating and adjoint; cf90's bounded adjoint keeps the
+    one-lane path, cd06's second derivative runs twice, in place."""
+    op, f, fh = setup(kind, n, periodic, axis, n + axis, torch.float32, pencils)
+    v = _lib.plan_variant(op._kind, OPER[which], n, 0.05, periodic, axis, *pencils, *bc, dtype=_lib.PADE_F32)
+    assert v["uneven"], v
+    D = pd.dense_operator(kind, "d1" if which == "d2" else which, n, 1.0 if which == "filter" else 0.05, periodic, *bc)
+    if which == "d2":
+        D = D @ D
+    ref = pd.apply_axis(D, fh, axis - 1)
+    out = po.fortran_empty(f.shape, dtype=torch.float32, device=DEV)
+    print(f"uneven FP32 {kind} {which} periodic {periodic} bc {bc} n {n} axis {axis}", flush=True)
+    op._apply(OPER[which], axis, f, out, *pencils, *bc)
+    assert rel(out.cpu().double().numpy(), ref) < tol
+    acc = f.clone()
+    op._apply(OPER[which], axis, f, acc, *pencils, *bc, alpha=-0.75, beta=1.5)
+    assert rel(acc.cpu().double().numpy(), -0.75 * ref + 1.5 * fh) < tol
+    op._apply(OPER[which], axis, f, out, *pencils, *bc, adjoint=True)
+    assert rel(out.cpu().double().numpy(), pd.apply_axis(D.T, fh, axis - 1)) < tol
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 2e-6)])
+@pytest.mark.parametrize("n", [128, 129, 132])
+@pytest.mark.parametrize("axis", [1, 2, 3])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_element_aligned_arrays(dtype, tol, n, axis, periodic):
+    """Fields that start one element behind a 16-byte boundary."""
+    op, f, fh = setup("cd10", n, periodic, axis, n, dtype)
+    D = pd.dense_operator("cd10", "d1", n, 0.05, periodic, 0, 0)
+    flat = torch.zeros(f.numel() + 1, dtype=dtype, device=DEV)[1:]
+    out = torch.zeros(f.numel() + 1, dtype=dtype, device=DEV)[1:]
+    flat.copy_(f.permute(2, 1, 0).reshape(-1))
+    assert flat.data_ptr() % 16 and out.data_ptr() % 16
+
+    def array(t):
+        return t.cpu().double().numpy().reshape(tuple(f.shape), order="F")
+    ref = pd.apply_axis(D, fh, axis - 1)
+    print(f"element-aligned {dtype} n {n} axis {axis} periodic {periodic}", flush=True)
+    op._apply(_lib.PADE_D1, axis, flat, out, 67, 5)
+    assert rel(array(out), ref) < tol
+    out.copy_(flat)
+    op._apply(_lib.PADE_D1, axis, flat, out, 67, 5, alpha=2.0, beta=-0.5)
+    assert rel(array(out), 2.0 * ref - 0.5 * fh) < tol
+    op._apply(_lib.PADE_D1, axis, flat, out, 67, 5, adjoint=True)
+    assert rel(array(out), pd.apply_axis(D.T, fh, axis - 1)) < tol
