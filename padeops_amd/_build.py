@@ -24,7 +24,8 @@ FSRC = os.path.join(HERE, "fortran")
 HIP_SOURCES = ["pade_plan.cpp", "pade_kernels.hip", "pade_spike_f64.hip", "pade_spike_f32.hip",
                "pade_uneven_f64.hip", "pade_uneven_f32.hip", "pade_uneven_mid_f64.hip", "pade_uneven_mid_f32.hip",
                "pade_uneven_long_f64.hip", "pade_uneven_long_f32.hip",
-               "pade_twice_a.hip", "pade_twice_b.hip", "pade_twice_c.hip", "pade_twice_d.hip", "pade_stage.hip", "pade_fields.hip",
+               "pade_twice_a.hip", "pade_twice_b.hip", "pade_twice_c.hip", "pade_twice_d.hip", "pade_stage.hip",
+               "pade_fields.hip", "pade_fields_uneven_a.hip", "pade_fields_uneven_b.hip",
                "pade_dense.hip", "pade_capi.cpp", "pade_cgrid.hip",
                "pade_cgrid_step.cpp", "pade_composite.cpp"]
 FORTRAN_SOURCES = ["padeops_c.F90", "cd06stuff.F90", "cd10stuff.F90", "cf90stuff.F90", "gaussianstuff.F90",

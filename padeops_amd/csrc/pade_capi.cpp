@@ -1296,7 +1296,8 @@ int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *fld
             if (!pl) return 21;
             LaunchPlan<double> Lk;
             if (int rc = plan_launch<double>(*pl, op->periodic, axis, flds[k].f, flds[k].out, na, nb, Lk)) return rc;
-            one = !Lk.generic && (times == 2 ? twice_ok(Lk, false) : nf == 1 || Lk.v->uneven || Lk.pw == 2 || Lk.pw == 8);
+            one = !Lk.generic && (times == 2 ? twice_ok(Lk, false)
+                                             : nf == 1 || ((Lk.v->uneven || Lk.pw == 2 || Lk.pw == 8) && !(acc && Lk.mode == 1)));
             if (k == 0) L = Lk;
             else one = one && Lk.v->M == L.v->M && Lk.v->P == L.v->P && Lk.pw == L.pw && Lk.v->uneven == L.v->uneven;
             L.a.fld[k] = Lk.a.fld[0];
@@ -1321,8 +1322,8 @@ int apply_fields(pade_op_t op, int oper, int axis, int nf, const BatchField *fld
                 return e == hipSuccess ? 0 : hip_fail(e, "spike_apply launch");
             }
             if (times == 2) e = launch_twice(L.a, L.v->M, L.pw, gw, L.v->uneven, false, L.mode, s);
+            else if (nf > 1) e = launch_fields(L.a, L.v->M, L.pw, gw, L.v->uneven, L.mode, s);
             else if (L.v->uneven) e = launch_uneven<double>(L.a, L.v->M, false, L.mode, s);
-            else if (nf > 1) e = launch_fields(L.a, L.v->M, L.pw, gw, L.mode, s);
             else e = launch_spike<double>(L.a, L.v->M, L.pw, gw, false, L.mode, s);
             if (e != hipSuccess) return hip_fail(e, "spike_apply launch");
             return run_stage(op, nf, flds, na, nb, stage, s);

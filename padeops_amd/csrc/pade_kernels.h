@@ -93,9 +93,10 @@ struct ApplyArgs : SolveArgs<T> {
 template <typename T>
 hipError_t launch_spike(const ApplyArgs<T> &a, int M, int PW, int GW, bool adj, int mode, hipStream_t s);
 
-// launch_spike of several fields: forward, modes 0 and 1, two partitions per
-// wave or whole-pencil x waves (FP64).
-hipError_t launch_fields(const ApplyArgs<double> &a, int M, int PW, int GW, int mode, hipStream_t s);
+// launch_spike and launch_uneven of several fields: forward, mode 0, or mode 1
+// without an epilogue, two partitions per wave (uneven: four of more than
+// sixteen) or whole-pencil x waves (FP64).
+hipError_t launch_fields(const ApplyArgs<double> &a, int M, int PW, int GW, bool uneven, int mode, hipStream_t s);
 
 // The same solve over uneven partitions (a pencil length that is no multiple
 // of M), two partitions per wave; modes as above.

@@ -267,17 +267,23 @@ __device__ __forceinline__ void apply_stencil(T (&w)[M + 8], const T *__restrict
 // three waves per SIMD instead of four), and the dependent read of its entries
 // stands before the first load of every workgroup (FP64 cd06 64^3 x / z 5.7 /
 // 5.6 us indexed, 5.5 / 5.3 not; cd10 512^3 z 421.9 and 417.4, FP32 x 187.5 and
-// 186.0).
+// 186.0; uneven, 97 points, 192 x 144 pencils, z 12.3 and 11.5).
 template <typename T, int NF>
 struct FieldSet {
+    SolveArgs<T> shared;   // the other argument once more, see spike_apply
     FieldArgs<T> fld[NF];
 };
 
 template <typename T, int M, int PW, bool ADJ, int MODE, bool BND, int EPI, bool UNE = false, int ROWS = kWholeLines,
           int REP = 1, int NF = 1>
-__global__ __launch_bounds__(512) void spike_apply(SolveArgs<T> a, FieldSet<T, NF> fields)
+__global__ __launch_bounds__(512) void spike_apply(SolveArgs<T> args, FieldSet<T, NF> fields)
 {
     constexpr int NPEN = 64 / PW;
+    // Strided kernels of several fields run out of scalar registers and read
+    // the shared arguments from memory instead (129 points, 512 x 512 pencils,
+    // periodic z 117.6 -> 113.5 us; the stage, M = 32, 133 -> 122 registers, 51
+    // -> 0 spilled scalars)
+    const SolveArgs<T> &a = NF > 1 && (MODE == 0 || PW == 8) ? fields.shared : args;
     const FieldArgs<T> &fd = fields.fld[NF > 1 ? blockIdx.y : 0];
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T *smem = reinterpret_cast<T *>(smem_raw);
@@ -435,8 +441,28 @@ __global__ __launch_bounds__(512) void spike_apply(SolveArgs<T> a, FieldSet<T, N
         // 313 with them)
         if constexpr (!ADJ) {
             // halo rows (wrapped per partition, or clamped at the ends of a
-            // bounded pencil, where the boundary rows replace the stencil)
-            auto load_halo = [&] {
+            // bounded pencil, where the boundary rows replace the stencil):
+            // before the main rows on periodic FP32 pencils (512^3 y / z 223.4
+            // / 228.7 -> 218.9 / 221.6 us, 222.0 / 222.7 as the compiler ordered
+            // them before the kernel served several fields).  (Written out
+            // twice: as one lambda they held the main loads of every kernel
+            // back by 180 instructions, the twice-applied strided one 174 ->
+            // 179 us.)
+            constexpr bool HALO_FIRST = sizeof(T) == 4 && !BND && EPI == kStore;
+            if constexpr (HALO_FIRST) {
+                const T *fq = fd.f + base0 + (long long)(loff / sizeof(T));
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int jl = wrap_index(pM - 4 + k, n, !BND);
+                    const int jr = wrap_index(pM + M + k, MODE == 2 ? a.n_in : n, !BND);
+                    w[k] = fq[(long long)jl * stp];
+                    w[M + 4 + k] = fq[(long long)jr * stp];
+                }
+                mem_region_fence();
+            }
+#pragma unroll
+            for (int t = 4; t < M + 4; t++) w[t] = ld_s<BND && ROWS == kWholeLines>(fb + (long long)(pw0 - 4 + t) * stp, active ? hoff : loff);
+            if constexpr (!HALO_FIRST) {
                 const T *fq = fd.f + base0 + (long long)(loff / sizeof(T));
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
@@ -446,18 +472,7 @@ __global__ __launch_bounds__(512) void spike_apply(SolveArgs<T> a, FieldSet<T, N
                     w[k] = fq[(long long)jl * stp];
                     w[M + 4 + k] = fq[(long long)jr * stp];
                 }
-            };
-            // (before the main rows on periodic FP32 pencils: 512^3 y / z 223.4
-            // / 228.7 -> 218.9 / 221.6 us, 222.0 / 222.7 as the compiler ordered
-            // them before the kernel served several fields)
-            constexpr bool HALO_FIRST = sizeof(T) == 4 && !BND && EPI == kStore;
-            if constexpr (HALO_FIRST) {
-                load_halo();
-                mem_region_fence();
             }
-#pragma unroll
-            for (int t = 4; t < M + 4; t++) w[t] = ld_s<BND && ROWS == kWholeLines>(fb + (long long)(pw0 - 4 + t) * stp, active ? hoff : loff);
-            if constexpr (!HALO_FIRST) load_halo();
         } else {
 #pragma unroll
             for (int t = 0; t < M; t++) w[t] = ld_s<BND && ROWS == kWholeLines>(fb + (long long)(pw0 + t) * stp, active ? hoff : loff);
@@ -1009,7 +1024,7 @@ hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
     constexpr bool WHOLE = MODE == 1 && PW == 8;
     if (a_in.nfields < 1 || a_in.nfields > NF) return hipErrorInvalidValue;
     SolveArgs<T> a = a_in;
-    FieldSet<T, NF> fields;
+    FieldSet<T, NF> fields{};
     std::copy_n(a_in.fld, NF, fields.fld);
     const int waves = WHOLE ? gw : (a.P + PW - 1) / PW;
     int coef_len = 0;
@@ -1018,6 +1033,7 @@ hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
     const long long nblk = (a.npencils + (long long)NPEN * gw - 1) / ((long long)NPEN * gw);
     a.remap = 0;
     auto launch = [&](auto kernel) {
+        fields.shared = a;
         hipLaunchKernelGGL(kernel, dim3((unsigned)nblk, (unsigned)a.nfields), dim3(64 * waves), lds, s,
                            a, fields);
         return hipGetLastError();
@@ -1054,7 +1070,7 @@ hipError_t launch_kernel(const ApplyArgs<T> &a_in, int gw, hipStream_t s)
 }
 
 template <typename T, int M, int PW, bool ADJ, int MODE, bool UNE = false, int REP = 1,
-          int NF = sizeof(T) == 8 && !ADJ && MODE != 2 && (UNE || REP > 1) ? kMaxFields : 1>
+          int NF = (REP > 1 && !(ADJ && MODE == 1) ? kMaxFields : 1)>
 hipError_t launch_spike_t(const ApplyArgs<T> &a, int gw, hipStream_t s)
 {
     constexpr bool WHOLE = MODE == 1 && PW == 8;
@@ -1073,6 +1089,11 @@ hipError_t launch_spike_t(const ApplyArgs<T> &a, int gw, hipStream_t s)
         // (a periodic adjoint runs the forward kernel on the transposed tables)
         if (a.periodic) return hipErrorInvalidValue;
         return launch_kernel<T, M, PW, true, MODE, true, kStore, UNE, REP, NF>(a, gw, s);
+    } else if constexpr (NF > 1 && REP == 1 && MODE == 1) {
+        // several fields along x: without an epilogue
+        if (epi) return hipErrorInvalidValue;
+        return a.periodic ? launch_kernel<T, M, PW, false, MODE, false, kStore, UNE, REP, NF>(a, gw, s)
+                          : launch_kernel<T, M, PW, false, MODE, true, kStore, UNE, REP, NF>(a, gw, s);
     } else {
         if (a.periodic)
             return epi ? launch_kernel<T, M, PW, false, MODE, false, kAxpby, UNE, REP, NF>(a, gw, s)
