@@ -119,13 +119,16 @@ int pade_op_apply_axpby(pade_op_t op, int oper, int axis, double alpha, const do
  * callers that cannot allocate device memory during an apply (code under HIP
  * graph capture, tight serving or time-stepping loops, harnesses that forbid
  * hipMalloc).  Same arguments, result and error codes as
- * pade_op_apply_axpby.  The intermediates some applies need (the
- * one-lane-per-pencil path's accumulate temporary, reserved for every n not
- * a multiple of 16 or above 1024; the bounded cd06 second derivative with an
- * epilogue) come from one static device array of
- * PADE_NOALLOC_SCRATCH_BYTES per device instead of the stream-ordered
- * allocator; an apply that would need more returns 400 before launching
- * anything.  Every call on a device shares that device's array, so calls
+ * pade_op_apply_axpby.  The intermediates some applies need come from one
+ * static device array of PADE_NOALLOC_SCRATCH_BYTES per device instead of the
+ * stream-ordered allocator.  An apply is refused with 400, before anything
+ * is launched, when the array cannot hold what is reserved for it: one field
+ * for an accumulating apply of n points that no even partition serves (even
+ * ones are multiples of 16 up to 256, of 32 up to 512, of 64 up to 1024),
+ * and for the bounded cd06 second derivative with an epilogue one field more
+ * than its first derivative.  The limit depends on the call alone, not on
+ * the kernel that runs: uneven partitions and the second derivative in one
+ * launch keep it although they leave the array untouched.  Every call on a device shares that device's array, so calls
  * that overlap on one device (two streams, two threads) race; the array is
  * never read before it is written within a call. */
 #define PADE_NOALLOC_SCRATCH_BYTES (64ull << 20)
@@ -221,9 +224,10 @@ int pade_op_dense_info(pade_op_t op, int oper, int prec, int axis, int f_dtype, 
  * staggered system form, launches the solves of one apply (2: the bounded
  * cd06 second derivative, the first derivative twice, which the FP64
  * partitioned kernels run as one kernel launch), and
- * uneven = 1 when M does not divide the rows and the partitions hold at most
- * M of them.  The
- * strided-row kernels address the field with 32-bit per-lane byte offsets (a
+ * uneven = 1 when the kernel of padded slots runs: the partitions hold at
+ * most M rows each.  M then mostly does not divide the rows; 40 and 48 slots
+ * (257 to 384 rows), and 64 above 1024 rows, serve the lengths that they
+ * divide as well.  The strided-row kernels address the field with 32-bit per-lane byte offsets (a
  * lane's pencil relative to its workgroup's first pencil plus (PW - 1) * M
  * points along the pencil); variants whose offsets would reach 2^32, or
  * whose launch would exceed 2^32 - 1 threads, are not chosen.  No reference
@@ -263,9 +267,10 @@ int pade_permute3(const void *src, void *dst, int elem_size, int n1, int n2, int
 int pade_plan_export(int kind, int oper, int n, double dx, int periodic, int bc1, int bcn,
                      int adjoint, int M, double *tab, long long tab_len, int *meta);
 
-/* The same for a pencil length that M (16, 24, 32 or 64) does not divide, or
- * that M = 40 or 48 serves: the table of its uneven partitions (a staggered
- * operator with an edge array: its system form).  meta[64]: as
+/* The same for uneven partitions of M slots: 16 or 24 for a length between
+ * one and two of them, 32 or 64 for one that M does not divide (64: or of more
+ * than 1024 rows, up to 1344), 40 or 48 for any.  The table is that of the
+ * padded slots (a staggered operator with an edge array: its system form).  meta[64]: as
  * pade_plan_export in [0, 32), [32] = W, the partitions of a reduced-system
  * row, [33 + p] = first row of partition p, [54 + p - 16] = class of p > 15.
  * Every partition occupies M slots: its rows, then padding slots with y_t =

@@ -141,8 +141,8 @@ def plan_variant(kind, oper, n, dx, periodic, axis, na, nb, bc1=0, bcn=0, dtype=
     """Kernel an apply would run (host-only, pade_plan_variant): a dict with
     the partition length M, partitions per wave PW, partitions P, ``generic``
     (one lane per pencil), ``mode`` (0 strided rows, 1 x pencils, 2 staggered
-    system form), ``launches`` per apply and ``uneven`` (M does not divide the rows).  bc1 / bcn: the codes that build
-    the operator (init-time for cd06 / cd06stagg, else apply-time)."""
+    system form), ``launches`` per apply and ``uneven`` (partitions of at most M rows in padded slots; M may divide
+    the rows where it is 40, 48, or 64 above 1024 rows).  bc1 / bcn: the codes that build the operator (init-time for cd06 / cd06stagg, else apply-time)."""
     info = (ctypes.c_int * 8)()
     check(load().pade_plan_variant(int(kind), int(oper), int(n), float(dx), int(bool(periodic)), int(bc1), int(bcn),
                                    int(bool(adjoint)), int(axis), int(na), int(nb), int(dtype), info))

@@ -236,7 +236,9 @@ constexpr int kFilterRhsBc = 100 + pade::FILTER;
 // FP64 / FP32: n = 129 as one partition 6.0e-15 / 2.8e-6, in 32 slots 1.0e-14
 // / 5.9e-6; n = 320 in 64 rows 8.6e-15 / 4.4e-6, in 40 slots 1.04e-14 /
 // 4.8e-6; but n = 176 in 16 rows 1.8e-14 / 6.8e-6, in 32 slots 1.0e-14 /
-// 5.3e-6).
+// 5.3e-6).  It costs time (FP64, us, x / y / z, one lane per pencil and 32
+// slots: n = 97, 128^2 pencils, 319 / 214 / 195 and 16 / 14 / 14; n = 129,
+// 256^2 pencils, 677 / 352 / 335 and 53 / 46 / 46).
 void add_spike_variants(const pade::OpMatrices &m, bool adj, bool inverse, std::vector<double> &tab,
                         std::vector<pade::PartFactors> &known, Plan &pl)
 {
@@ -273,8 +275,8 @@ void add_spike_variants(const pade::OpMatrices &m, bool adj, bool inverse, std::
     }
 }
 
-// One plan: the operator's matrices and the factor tables of every partition
-// size that divides its rows (appended to `tab`), plus the
+// One plan: the operator's matrices and the factor tables of the partition
+// sizes that serve its rows, even and uneven (appended to `tab`), plus the
 // one-lane-per-pencil form.  bc1 / bcn are the codes that build the
 // operator (init-time for cd06 and cd06stagg).
 int build_plan(int kind, int oper, int n, double dx, bool periodic, int bc1, int bcn, bool adj,
@@ -381,14 +383,6 @@ int env_int(const char *name)
     return v ? std::atoi(v) : 0;
 }
 
-// Choose (partition size M, partitions per wave PW) for this launch.
-// Two partitions per wave (two workgroups per CU) throughout; x pencils
-// (LDS-transposed, mode 1) and bounded y/z pencils prefer M = 64, periodic
-// y/z pencils M = 32 -- the fastest variants measured at 512^3 (bounded z:
-// 279 vs 214 Gpts/s; the M = 32 bounded kernel runs at three waves per SIMD,
-// one 8-wave workgroup per CU).  Small problems take
-// the smallest M to raise the wave count.  PADE_SPIKE_M / PADE_SPIKE_PW
-// override the choice (tuning).
 // Largest thread count of one launch (grid size x workgroup size must stay
 // below 2^32).
 constexpr long long kMaxLaunchThreads = 0xffffffffLL;
@@ -410,11 +404,19 @@ bool offsets_fit(const pade::ApplyArgs<T> &a, int mode, int M, int PW)
     return lmax + part < (1LL << 32);
 }
 
-// Fewest pencils that uneven partitions serve.  Below it (one workgroup's
-// worth or two of the whole chip) the one-lane-per-pencil kernel runs, as
-// pade_plan_variant reports for 100 x pencils of 100 points.
+// Fewest pencils that uneven partitions serve.  Below it these lengths run one
+// lane per pencil, as pade_plan_variant reports for 100 x pencils of 100 points.
+// Not a crossover: from 1 to 127 pencils (periodic cd10, FP64, x and z) one
+// lane per pencil takes 44-54 us at n = 25, 106-136 at 65, 210-266 at 129,
+// 418-530 at 257 and 1146-1397 at 700, uneven partitions 4-5, 7-8, 7-9,
+// 10-11 and 17-19.
 constexpr long long kUnevenPencils = 128;
 
+// Choose (partition size M, partitions per wave PW) for this launch: two
+// partitions per wave but for whole x pencils and more than sixteen
+// partitions, M by type, axis, length and boundary as measured below, the
+// smallest M for small problems.  PADE_SPIKE_M / PADE_SPIKE_PW override the
+// choice (tuning).
 template <typename T>
 const Variant *pick_variant(const Plan &pl, const pade::ApplyArgs<T> &a, int mode, int *pw_out)
 {

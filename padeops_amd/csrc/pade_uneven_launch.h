@@ -26,8 +26,9 @@ hipError_t launch_uneven_mid(const ApplyArgs<T> &a, int M, bool adj, int mode, h
 // more than sixteen partitions of 64 slots, four per wave (two would need nine
 // or more waves of 256 registers in a workgroup, and a CU holds eight): 16
 // neighbouring pencils per strided row, one whole line in FP64.  Bound by
-// memory: 1025 points, 256 x 128 pencils, FP64 cd10 x / y / z 240 / 176 / 179
-// us (2.2 / 3.0 / 3.0 TB/s), 3780 / 2494 / 2450 with one lane per pencil.  In
+// each wave's own chain, its reduced system of up to 21 partitions included:
+// 1025 points, 256 x 128 pencils, FP64 cd10 x / y / z 240 / 176 / 179 us (2.2 /
+// 3.0 / 3.0 TB/s), 3780 / 2494 / 2450 with one lane per pencil.  In
 // translation units of their own
 template <typename T>
 hipError_t launch_uneven_long(const ApplyArgs<T> &a, bool adj, int mode, hipStream_t s);
